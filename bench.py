@@ -43,12 +43,12 @@ SETTLE = {"hulls64k": 200, "lattice4k": 40, "batched4k": 120}
 STAGES = ["setup", "sort", "pairs", "narrowphase", "constraints", "colouring", "solve",
           "integrate"]
 
-# k_tile_solve, per row and sweep: normal sweeps on precomputed rows read
-# 368 B and write the 16 B of impulses; friction sweeps read the full 312 B
-# row and write 16 B; scene tiles run every sweep in one launch and write
-# both impulse vectors once (328 B).  Per tile body and launch: velocities
-# read and written (4 float4 = 64 B).
-ROW_NORMAL, ROW_FRICTION, ROW_SCENE, TILE_BODY = 384, 328, 328, 64
+# k_tile_solve, per row and sweep: normal sweeps on packed rows read 384 B and
+# write the 16 B of impulses; friction sweeps read 320 B and write 8 B.  Scene
+# tiles (k_scene_solve) form each row once from its constraint and bodies
+# (316 B), run every sweep in one launch and write 24 B of impulses.  Per tile
+# body and launch: velocities read and written (4 float4 = 64 B).
+ROW_NORMAL, ROW_FRICTION, ROW_SCENE, TILE_BODY = 400, 328, 340, 64
 
 
 def solve_bytes(contacts, tile_bodies, sweeps, scene_tiles):

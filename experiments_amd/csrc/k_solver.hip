@@ -22,6 +22,8 @@
 #include <float.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dmath.h"
 #include "rb_internal.h"
 
@@ -30,7 +32,6 @@ using namespace rb;
 namespace {
 
 constexpr int TB = 256;        // threads per tile workgroup (colouring, spatial solve tiles)
-constexpr int TB_SCENE = 512;  // threads per scene tile in the solve
 constexpr int HASH_SLOTS = 2 * RB_TILE_MAX_BODIES;
 
 __device__ __forceinline__ uint32_t color_prio(uint32_t k) {
@@ -47,18 +48,16 @@ __device__ __forceinline__ float rel_vel(float4 l0, float4 l1, float4 a0, float4
                                          float4 wA, float4 vB, float4 wB) {
     return ((dot3(l0, vA) + dot3(a0, wA)) + dot3(l1, vB)) + dot3(a1, wB);
 }
+// (btPlaneSpace1, both cases by selects: one square root and one division for
+// the whole wave, and nothing for the compiler to put into scratch)
 __device__ __forceinline__ void plane_space(float4 n, float4 &p, float4 &q) {
-    if (fabsf(n.z) > 0.70710678f) {
-        float a = n.y * n.y + n.z * n.z;
-        float k = 1.f / sqrtf(a);
-        p = mk4(0.f, -n.z * k, n.y * k, 0.f);
-        q = mk4(a * k, -n.x * p.z, n.x * p.y, 0.f);
-    } else {
-        float a = n.x * n.x + n.y * n.y;
-        float k = 1.f / sqrtf(a);
-        p = mk4(-n.y * k, n.x * k, 0.f, 0.f);
-        q = mk4(-n.z * p.y, n.z * p.x, a * k, 0.f);
-    }
+    const bool z = fabsf(n.z) > 0.70710678f;
+    const float yy = n.y * n.y;
+    const float a = z ? yy + n.z * n.z : n.x * n.x + yy;
+    const float k = 1.f / sqrtf(a), ak = a * k;
+    const float pz = n.y * k, py = z ? -n.z * k : n.x * k;
+    p = mk4(z ? 0.f : -n.y * k, py, z ? pz : 0.f, 0.f);
+    q = mk4(z ? ak : -n.z * py, z ? -n.x * pz : n.z * p.x, z ? n.x * py : ak, 0.f);
 }
 
 // Tile coordinates of a point (clamped, so neighbours stay neighbours).
@@ -422,208 +421,332 @@ __global__ __launch_bounds__(TB) void k_tile_color(
 }
 
 // ---- solve ----
-constexpr int SOLVE_SLOTS = 1024;  // LDS velocity cache of one tile (32 KB)
-struct SolveLDS {
-    float4 v[SOLVE_SLOTS];
-    float4 w[SOLVE_SLOTS];
-};
-constexpr int SLOT_STATIC = -1;    // static body: zero velocity, no writes
-constexpr int SLOT_GLOBAL = -2;    // dynamic body beyond the LDS cache: global memory
+// Four lanes (a quad) run one row: lane 0 holds body A's linear velocity,
+// lane 1 its angular velocity, lanes 2 and 3 body B's.  Each lane multiplies
+// its own quarter of the row's Jacobian, the four dot products are summed in
+// lane order across the quad (DPP), every lane forms the same impulse, and
+// each lane updates its own velocity: the same operations in the same order
+// as one thread working through the row, so the results are identical.  What
+// bounds a sweep is the serial chain of a colour (up to four points, each
+// reading the velocities the last one wrote) in the one or two waves that
+// hold the colour's rows: split over a quad a point issues about 25
+// instructions where one thread per row issued 61, and the row's data is
+// spread over four lanes' registers (110 of them where a thread per row took
+// 212, so twice the workgroups of a phase run at once).  Launches of 65,537
+// hulls in contact: normal 9.6 -> 7.1 us, friction 9.9 -> 6.7 us; 4,096 cubes
+// on a triangle mesh: 16.3 -> 6.4 and 17.2 -> 6.2 us.
+constexpr int SOLVE_SLOTS = 1012;  // LDS velocity cache of one tile (five such tiles in a CU's LDS)
+constexpr int SLOT_STATIC = SOLVE_SLOTS;      // static body: the zero slot, no writes
+constexpr int SLOT_GLOBAL = SOLVE_SLOTS + 1;  // dynamic body beyond the LDS cache: global memory
+enum { ROW_NORMAL = 0, ROW_FRICTION = 1, ROW_WARM = 2 };
 
-// A row body's velocities by its slot.  The LDS read is unconditional (slot
-// clamped to 0) and the rare global and static cases overwrite it, so the
-// compiler keeps an LDS read (ds_read) instead of merging the two sources
-// into one generic-address load through a select of pointers (a flat load,
-// whose latency is that of the vector memory path, plus a zero vector
-// materialised in scratch).
-__device__ __forceinline__ void fetch_vel(int h, int b, const SolveLDS &L,
-                                          const float4 *__restrict__ linvel,
-                                          const float4 *__restrict__ angvel, float4 &v,
-                                          float4 &w) {
-    const int s = h >= 0 ? h : 0;
-    v = L.v[s];
-    w = L.w[s];
-    if (h < 0) {
-        // (both slots read the body's global velocity and select by value)
-        const float4 gv = linvel[b], gw = angvel[b];
-        const bool g = h == SLOT_GLOBAL;
-        v = g ? gv : mk4(0.f, 0.f, 0.f, 0.f);
-        w = g ? gw : mk4(0.f, 0.f, 0.f, 0.f);
-    }
+struct TileSolveLDS {
+    // slot s: linear at 2s + 2, angular at 2s + 3; the first two are zero
+    float4 vel[2 * (SOLVE_SLOTS + 1)];
+    unsigned int gred[2];  // add_sweep_residual's workgroup maxima
+};
+
+#define QUAD_PERM(p) " quad_perm:" p " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+// ((x0 + x1) + x2) + x3 over the lanes of a quad.  Lanes 0 and 1 first swap
+// and add (their sum is the same either way round).  A DPP read must trail the
+// write of its source by two instructions; written out, the copies of lanes 2
+// and 3 fill one of the two gaps, where the compiler's order needs four waits.
+__device__ __forceinline__ float quad_sum(float x) {
+    float r, y, z;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %3, %3" QUAD_PERM("[1,0,3,2]")
+        "v_mov_b32_dpp %1, %3" QUAD_PERM("[2,2,2,2]")
+        "v_mov_b32_dpp %2, %3" QUAD_PERM("[3,3,3,3]")
+        "v_add_f32_dpp %1, %0, %1" QUAD_PERM("[0,0,0,0]")
+        "v_add_f32_e32 %0, %1, %2"
+        : "=&v"(r), "=&v"(y), "=&v"(z)
+        : "v"(x));
+    return r;
+}
+// The quad's four values in every lane, formed before the row's serial chain
+// starts (folded into the chain's instructions as DPP operands, each would
+// cost the chain a wait instead).
+__device__ __forceinline__ void quad_spread(float x, float out[4]) {
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %4" QUAD_PERM("[0,0,0,0]")
+        "v_mov_b32_dpp %1, %4" QUAD_PERM("[1,1,1,1]")
+        "v_mov_b32_dpp %2, %4" QUAD_PERM("[2,2,2,2]")
+        "v_mov_b32_dpp %3, %4 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf bound_ctrl:1"
+        : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3])
+        : "v"(x));
 }
 
-// Constraint fields one row needs (Constraint4 minus the body indices).
-struct RowData {
-    float4 lin0, jac, bb, lam, fr, cen;
-    float4 p[4];
-};
-// The row's two bodies: inverse mass, world inverse inertia, position and the
-// LDS cache slot of the velocity (-1: static, or kept in global memory).
-struct RowBodies {
-    int a, b, ha, hb;
-    float imA, imB;
-    float4 IA[3], IB[3];
-    float4 pA, pB;
-};
-
-// A row of the packed solve arrays (position `i` in solve order).
-__device__ __forceinline__ void load_packed(int i, const PackedRows &pk, RowData &d, RowBodies &rb) {
-    d.lin0 = pk.lin0[i];
-    d.jac = pk.jac[i];
-    d.bb = pk.b[i];
-    d.lam = pk.lam[i];
-    d.fr = pk.fric[i];
-    d.cen = pk.cen[i];
-    for (int q = 0; q < 4; q++) d.p[q] = pk.p[4 * (size_t)i + q];
-    const int4 m = pk.meta[i];
-    rb.a = m.x;
-    rb.b = m.y;
-    rb.ha = m.z;
-    rb.hb = m.w;
-    const float2 im = pk.im[i];
-    rb.imA = im.x;
-    rb.imB = im.y;
-    for (int q = 0; q < 3; q++) {
-        rb.IA[q] = pk.IA[3 * (size_t)i + q];
-        rb.IB[q] = pk.IB[3 * (size_t)i + q];
-    }
-    rb.pA = pk.pA[i];
-    rb.pB = pk.pB[i];
+// A lane's part of a row: its LDS velocity slot in the low half, the row's
+// colour in the high half.
+__device__ __forceinline__ float4 fetch_vel(int slot, int body, int l, const float4 *vel,
+                                            const float4 *linvel, const float4 *angvel) {
+    const int s = slot < SLOT_STATIC ? slot + 1 : 0;
+    float4 v = vel[2 * s + (l & 1)];
+    if (slot == SLOT_GLOBAL) v = (l & 1 ? angvel : linvel)[body];
+    return v;
+}
+__device__ __forceinline__ void put_vel(int slot, int body, int l, float4 v, float4 *vel,
+                                        float4 *linvel, float4 *angvel) {
+    if (slot < SLOT_STATIC) vel[2 * (slot + 1) + (l & 1)] = v;
+    else if (slot == SLOT_GLOBAL) (l & 1 ? angvel : linvel)[body] = v;
 }
 
+// (a choice between two float4 variables is written by value: as a choice of
+// addresses it puts both into scratch)
+__device__ __forceinline__ float4 sel4(bool c, float4 a, float4 b) {
+    return mk4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
+}
+
+// What a solve reads besides the packed rows: the constraints and bodies the
+// scene tiles form their rows from, and the velocities.
+struct SolveView {
+    ConstraintSoA cs;
+    const int *order;
+    const float4 *pos;
+    const float *inv_mass;
+    const float4 *invI;
+    float4 *linvel, *angvel;
+};
+
+// A lane's quarter of a normal row: per point its Jacobian and the velocity
+// change per impulse (w of the linear lanes' is the friction coefficient over
+// the mass, the same for every point).  Lane q of the quad holds point q's
+// 1/J M J^T, bias and impulse; the quad reads them by DPP.
+struct NormalRow {
+    int code;  // slot | colour << 16, -1: no row
+    float J[4][3], M[4][3], mw, jac, b, lam;
+};
+// (the operations the constraint maths forms these terms with; every lane goes
+// through the angular ones and the linear lanes drop them, which costs a wave
+// nothing)
+__device__ __forceinline__ void form_normal(bool side, bool ang, float4 lin0, float im,
+                                            const float4 I[3], float4 p, const float4 wp[4],
+                                            float4 J[4], float4 M[4]) {
+    const float4 n = neg4(lin0), lin = sel4(side, neg4(lin0), lin0), lm = scl4(lin, im);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 a = cross3(sub4(wp[q], p), n), j = sel4(side, a, neg4(a));
+        J[q] = sel4(ang, j, lin);
+        M[q] = sel4(ang, mt_mul1(I, j), lm);
+    }
+}
+// ... and of a friction row: the tangents t0, t1 at the manifold centre
+__device__ __forceinline__ void form_friction(bool side, bool ang, float4 lin0, float im,
+                                              const float4 I[3], float4 p, float4 cen,
+                                              float4 J[2], float4 M[2]) {
+    float4 t[2];
+    plane_space(neg4(lin0), t[0], t[1]);
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const float4 lin = sel4(side, t[q], neg4(t[q]));
+        const float4 a = cross3(sub4(cen, p), t[q]), j = sel4(side, a, neg4(a));
+        J[q] = sel4(ang, j, lin);
+        M[q] = sel4(ang, mt_mul1(I, j), scl4(lin, im));
+    }
+}
+// whether a friction row damps the spin about its normal (the manifold centre
+// on the line of the bodies, or a static body)
+__device__ __forceinline__ bool row_damps(float4 pA, float4 pB, float4 cen, float imA, float imB) {
+    const float4 ab = normalize3(sub4(pB, pA)), ac = normalize3(sub4(cen, pA));
+    return dot3(ab, ac) > 0.95f || (imA == 0.f || imB == 0.f);
+}
+
+__device__ __forceinline__ float lane_of(const float4 *a, int i, int l) {
+    return reinterpret_cast<const float *>(a + i)[l];
+}
+__device__ __forceinline__ int row_code(const PackedRows &pk, int i, int l) {
+    return pk.meta[2 * (size_t)i + (l >> 1)].y;
+}
+__device__ __forceinline__ int row_body(const PackedRows &pk, int i, int l) {
+    return pk.meta[2 * (size_t)i + (l >> 1)].x;
+}
+// Spatial tiles: row i from the packed arrays.
+__device__ __forceinline__ void load_normal(int i, int l, const PackedRows &pk, NormalRow &r) {
+    r.code = row_code(pk, i, l);
+    const float4 *J = pk.nj + 10 * (size_t)i + (l >> 1), *M = pk.nm + 10 * (size_t)i + (l >> 1);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int e = l & 1 ? 2 * (q + 1) : 0;
+        const float4 j = J[e], m = M[e];
+        r.J[q][0] = j.x; r.J[q][1] = j.y; r.J[q][2] = j.z;
+        r.M[q][0] = m.x; r.M[q][1] = m.y; r.M[q][2] = m.z;
+        if (q == 0) r.mw = m.w;
+    }
+    r.jac = lane_of(pk.jac, i, l);
+    r.b = lane_of(pk.b, i, l);
+    r.lam = lane_of(pk.lam, i, l);
+}
+// Scene tiles: the row at solve position i from its constraint.
+__device__ __forceinline__ void load_normal(int i, int l, const PackedRows &pk,
+                                            const SolveView &sv, NormalRow &r) {
+    const int2 m = pk.meta[2 * (size_t)i + (l >> 1)];
+    const int k = sv.order[i], side = l >> 1;
+    const bool ang = l & 1;
+    r.code = m.y;
+    float4 J[4], M[4], I[3], wp[4];
+    const float4 lin0 = sv.cs.linear[k], p = sv.pos[m.x];
+    const float im = sv.inv_mass[m.x];
+#pragma unroll
+    for (int q = 0; q < 3; q++) I[q] = sv.invI[3 * (size_t)m.x + q];
+#pragma unroll
+    for (int q = 0; q < 4; q++) wp[q] = sv.cs.pos[4 * (size_t)k + q];
+    form_normal(side, ang, lin0, im, I, p, wp, J, M);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        r.J[q][0] = J[q].x; r.J[q][1] = J[q].y; r.J[q][2] = J[q].z;
+        r.M[q][0] = M[q].x; r.M[q][1] = M[q].y; r.M[q][2] = M[q].z;
+    }
+    r.mw = M[0].w;
+    r.jac = lane_of(sv.cs.jac_inv, k, l);
+    r.b = lane_of(sv.cs.b, k, l);
+    r.lam = lane_of(sv.cs.lambda, k, l);
+}
 // solveContact (solveContact.cl:272-312): sequential impulses on the normal
 // rows, lambda >= 0.
 // RES: compute the sweep residual terms (the largest scaled impulse change
-// and the largest impulse); launches whose sweep reports no residual skip
-// them, which leaves every velocity and impulse unchanged.
-template <bool RES = true>
-__device__ __forceinline__ void row_normal(RowData &d, float4 &vA, float4 &wA, float4 &vB,
-                                           float4 &wB, const RowBodies &rb, float &rmax,
-                                           float &lmax) {
-    const float4 lin0 = d.lin0;
-    float jv[4] = {d.jac.x, d.jac.y, d.jac.z, d.jac.w};
-    float bv[4] = {d.bb.x, d.bb.y, d.bb.z, d.bb.w};
-    float lv[4] = {d.lam.x, d.lam.y, d.lam.z, d.lam.w};
+// and the largest impulse); sweeps whose residual nobody reads skip them,
+// which leaves every velocity and impulse unchanged.
+// (a point beyond the manifold's has jac, b and lambda zero: its impulse
+// change is zero and its residual term 0 / 0, which fmaxf drops, so no branch
+// is needed to skip it)
+template <bool RES>
+__device__ __forceinline__ void run_normal(NormalRow &d, int i, int l, const PackedRows &pk,
+                                           float4 *vel, float4 *linvel, float4 *angvel,
+                                           float &rmax, float &lmax) {
+    const int slot = d.code & 0xffff;
+    const int body = slot == SLOT_GLOBAL ? row_body(pk, i, l) : 0;
+    float4 v = fetch_vel(slot, body, l, vel, linvel, angvel);
+    float jv[4], bv[4], lv[4];
+    quad_spread(d.jac, jv);
+    quad_spread(d.b, bv);
+    quad_spread(d.lam, lv);
+#pragma unroll
     for (int ic = 0; ic < 4; ic++) {
-        if (jv[ic] == 0.f) continue;
-        float4 wp = d.p[ic];
-        float4 r0 = sub4(wp, rb.pA), r1 = sub4(wp, rb.pB);
-        float4 n = neg4(lin0);
-        float4 lin = neg4(n);
-        float4 a0 = neg4(cross3(r0, n));
-        float4 a1 = cross3(r1, n);
-        float rl = rel_vel(lin0, neg4(lin0), a0, a1, vA, wA, vB, wB) + bv[ic];
+        float rl = quad_sum((d.J[ic][0] * v.x + d.J[ic][1] * v.y) + d.J[ic][2] * v.z) + bv[ic];
         rl *= jv[ic];
-        float prev = lv[ic];
-        float upd = prev + rl;
-        upd = fmaxf(upd, 0.f);
-        upd = fminf(upd, FLT_MAX);
-        rl = upd - prev;
-        lv[ic] = upd;
-        float4 li0 = scl4(scl4(lin, rb.imA), rl);
-        float4 li1 = scl4(scl4(neg4(lin), rb.imB), rl);
-        float4 ai0 = scl4(mt_mul1(rb.IA, a0), rl);
-        float4 ai1 = scl4(mt_mul1(rb.IB, a1), rl);
-        vA = add4(vA, li0); wA = add4(wA, ai0);
-        vB = add4(vB, li1); wB = add4(wB, ai1);
+        // (min(max(x, 0), FLT_MAX), NaN to 0, in one instruction)
+        const float upd = __builtin_amdgcn_fmed3f(lv[ic] + rl, 0.f, FLT_MAX);
+        rl = upd - lv[ic];
+        if (l == ic) d.lam = upd;
+        v = mk4(v.x + d.M[ic][0] * rl, v.y + d.M[ic][1] * rl, v.z + d.M[ic][2] * rl,
+                v.w + d.mw * rl);
         if (RES) {
-            float sc = fabsf(rl) / fabsf(jv[ic]);
-            rmax = fmaxf(rmax, sc);
+            rmax = fmaxf(rmax, fabsf(rl) / fabsf(jv[ic]));
             lmax = fmaxf(lmax, fabsf(upd));
         }
     }
-    d.lam = mk4(lv[0], lv[1], lv[2], lv[3]);
+    put_vel(slot, body, l, v, vel, linvel, angvel);
 }
 
-// solveFriction (solveFriction.cl:297-430): two tangents at the manifold
-// centre, |lambda| <= mu * sum lambda_n, then the angular damping about n.
-template <bool RES = true>
-__device__ __forceinline__ void row_friction(RowData &d, float4 &vA, float4 &wA, float4 &vB,
-                                             float4 &wB, const RowBodies &rb, float friction,
-                                             float &rmax, float &lmax) {
-    const float4 lam = d.lam;
+// A lane's quarter of a friction row: both tangents' Jacobians and velocity
+// changes per impulse, the normal (w: the friction coefficient, negated) and
+// the cone's limit.  Lanes 0 and 1 of the quad hold the tangents' 1/J M J^T,
+// lanes 2 and 3 their impulses.
+struct FrictionRow {
+    int code;
+    float J[2][3], M[2][3];
+    float4 n;
+    float fr, mx;
+};
+constexpr int ROW_DAMPS = 1 << 15;  // in a friction row's code: the angular damping applies
+static_assert(SLOT_GLOBAL < ROW_DAMPS, "slot, flag and colour share a word");
+__device__ __forceinline__ void set_friction(FrictionRow &r, const float4 J[2], const float4 M[2],
+                                             float4 lin0, float fr, float4 lam, float friction,
+                                             bool damp) {
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        r.J[q][0] = J[q].x; r.J[q][1] = J[q].y; r.J[q][2] = J[q].z;
+        r.M[q][0] = M[q].x; r.M[q][1] = M[q].y; r.M[q][2] = M[q].z;
+    }
+    r.n = neg4(lin0);
+    r.fr = fr;
     float sum = 0;
     sum += lam.x; sum += lam.y; sum += lam.z; sum += lam.w;
-    float mx = friction * sum, mn = -mx;
-    const float4 fr = d.fr;
-    if (fr.x == 0 && fr.x == 0) return;
-    const float4 cen = d.cen;
-    float4 n = neg4(d.lin0);
-    float4 t[2];
-    plane_space(n, t[0], t[1]);
-    float4 r0 = sub4(cen, rb.pA), r1 = sub4(cen, rb.pB);
-    float fj[2] = {fr.x, fr.y};
-    float fl[2] = {fr.z, fr.w};
-    for (int i = 0; i < 2; i++) {
-        float4 lin = neg4(t[i]);
-        float4 a0 = neg4(cross3(r0, t[i]));
-        float4 a1 = cross3(r1, t[i]);
-        float rl = rel_vel(lin, neg4(lin), a0, a1, vA, wA, vB, wB);
-        rl *= fj[i];
-        float prev = fl[i];
-        float upd = prev + rl;
-        upd = fmaxf(upd, mn);
-        upd = fminf(upd, mx);
-        rl = upd - prev;
-        fl[i] = upd;
-        float4 li0 = scl4(scl4(lin, rb.imA), rl);
-        float4 li1 = scl4(scl4(neg4(lin), rb.imB), rl);
-        float4 ai0 = scl4(mt_mul1(rb.IA, a0), rl);
-        float4 ai1 = scl4(mt_mul1(rb.IB, a1), rl);
-        vA = add4(vA, li0); wA = add4(wA, ai0);
-        vB = add4(vB, li1); wB = add4(wB, ai1);
+    r.mx = friction * sum;
+    if (damp) r.code |= ROW_DAMPS;
+}
+__device__ __forceinline__ void load_friction(int i, int l, const PackedRows &pk, float friction,
+                                              FrictionRow &r) {
+    r.code = row_code(pk, i, l);
+    const float4 *j = pk.fj + 8 * (size_t)i + l, *m = pk.fm + 8 * (size_t)i + l;
+    const float4 J[2] = {j[0], j[4]}, M[2] = {m[0], m[4]};
+    set_friction(r, J, M, pk.lin0[i], lane_of(pk.fric, i, l), pk.lam[i], friction, J[0].w != 0.f);
+}
+__device__ __forceinline__ void load_friction(int i, int l, const PackedRows &pk,
+                                              const SolveView &sv, float friction,
+                                              FrictionRow &r) {
+    const int2 mA = pk.meta[2 * (size_t)i], mB = pk.meta[2 * (size_t)i + 1];
+    const int k = sv.order[i], side = l >> 1;
+    const bool ang = l & 1;
+    const int body = side ? mB.x : mA.x;
+    r.code = side ? mB.y : mA.y;
+    const float4 lin0 = sv.cs.linear[k], cen = sv.cs.center[k];
+    const float4 pA = sv.pos[mA.x], pB = sv.pos[mB.x];
+    const float imA = sv.inv_mass[mA.x], imB = sv.inv_mass[mB.x];
+    float4 I[3], J[2], M[2];
+#pragma unroll
+    for (int q = 0; q < 3; q++) I[q] = sv.invI[3 * (size_t)body + q];
+    form_friction(side, ang, lin0, side ? imB : imA, I, sel4(side, pB, pA), cen, J, M);
+    set_friction(r, J, M, lin0, lane_of(sv.cs.fric, k, l), sv.cs.lambda[k], friction,
+                 row_damps(pA, pB, cen, imA, imB));
+}
+// solveFriction (solveFriction.cl:297-430): two tangents at the manifold
+// centre, |lambda| <= mu * sum lambda_n, then the angular damping about n.
+template <bool RES>
+__device__ __forceinline__ void run_friction(FrictionRow &d, int i, int l, const PackedRows &pk,
+                                             float4 *vel, float4 *linvel, float4 *angvel,
+                                             float &rmax, float &lmax) {
+    float f[4];
+    quad_spread(d.fr, f);
+    if (f[0] == 0.f) return;
+    const int slot = d.code & (ROW_DAMPS - 1);
+    const int body = slot == SLOT_GLOBAL ? row_body(pk, i, l) : 0;
+    float4 v = fetch_vel(slot, body, l, vel, linvel, angvel);
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        float rl = quad_sum((d.J[t][0] * v.x + d.J[t][1] * v.y) + d.J[t][2] * v.z);
+        rl *= f[t];
+        float upd = f[2 + t] + rl;
+        upd = fmaxf(upd, -d.mx);
+        upd = fminf(upd, d.mx);
+        rl = upd - f[2 + t];
+        if (l == 2 + t) d.fr = upd;
+        v.x += d.M[t][0] * rl; v.y += d.M[t][1] * rl; v.z += d.M[t][2] * rl;
         if (RES) {
-            float sc = fabsf(rl) / fabsf(fj[i]);
-            rmax = fmaxf(rmax, sc);
+            rmax = fmaxf(rmax, fabsf(rl) / fabsf(f[t]));
             lmax = fmaxf(lmax, fabsf(upd));
         }
     }
-    d.fr = mk4(fr.x, fr.y, fl[0], fl[1]);
-    float4 ab = normalize3(sub4(rb.pB, rb.pA));
-    float4 ac = normalize3(sub4(cen, rb.pA));
-    if (dot3(ab, ac) > 0.95f || (rb.imA == 0.f || rb.imB == 0.f)) {
-        float na = dot3(n, wA), nb = dot3(n, wB);
-        wA = sub4(wA, scl4(n, na * 0.1f));
-        wB = sub4(wB, scl4(n, nb * 0.1f));
-    }
+    if ((l & 1) && (d.code & ROW_DAMPS)) v = sub4(v, scl4(d.n, dot3(d.n, v) * 0.1f));
+    put_vel(slot, body, l, v, vel, linvel, angvel);
 }
 
 // Apply the impulses a row already holds (warm start) to its bodies.
-__device__ __forceinline__ void row_warm(const RowData &d, float4 &vA, float4 &wA, float4 &vB,
-                                         float4 &wB, const RowBodies &rb) {
-    const float4 lin0 = d.lin0;
-    float jv[4] = {d.jac.x, d.jac.y, d.jac.z, d.jac.w};
-    float lv[4] = {d.lam.x, d.lam.y, d.lam.z, d.lam.w};
+__device__ __forceinline__ void run_warm(const NormalRow &d, const FrictionRow &f, int i, int l,
+                                         const PackedRows &pk, float4 *vel, float4 *linvel,
+                                         float4 *angvel) {
+    const int slot = d.code & 0xffff;
+    const int body = slot == SLOT_GLOBAL ? row_body(pk, i, l) : 0;
+    float4 v = fetch_vel(slot, body, l, vel, linvel, angvel);
+    float jv[4], lv[4], fv[4];
+    quad_spread(d.jac, jv);
+    quad_spread(d.lam, lv);
+    quad_spread(f.fr, fv);
+#pragma unroll
     for (int ic = 0; ic < 4; ic++) {
         if (jv[ic] == 0.f || lv[ic] == 0.f) continue;
-        float4 wp = d.p[ic];
-        float4 r0 = sub4(wp, rb.pA), r1 = sub4(wp, rb.pB);
-        float4 n = neg4(lin0);
-        float4 lin = neg4(n);
-        float4 a0 = neg4(cross3(r0, n)), a1 = cross3(r1, n);
-        float rl = lv[ic];
-        vA = add4(vA, scl4(scl4(lin, rb.imA), rl));
-        wA = add4(wA, scl4(mt_mul1(rb.IA, a0), rl));
-        vB = add4(vB, scl4(scl4(neg4(lin), rb.imB), rl));
-        wB = add4(wB, scl4(mt_mul1(rb.IB, a1), rl));
+        v = mk4(v.x + d.M[ic][0] * lv[ic], v.y + d.M[ic][1] * lv[ic], v.z + d.M[ic][2] * lv[ic],
+                v.w + d.mw * lv[ic]);
     }
-    const float4 fr = d.fr;
-    if (fr.x == 0.f) return;
-    float4 n = neg4(lin0);
-    float4 t[2];
-    plane_space(n, t[0], t[1]);
-    float4 r0 = sub4(d.cen, rb.pA), r1 = sub4(d.cen, rb.pB);
-    float fl[2] = {fr.z, fr.w};
-    for (int i = 0; i < 2; i++) {
-        float rl = fl[i];
-        if (rl == 0.f) continue;
-        float4 lin = neg4(t[i]);
-        float4 a0 = neg4(cross3(r0, t[i])), a1 = cross3(r1, t[i]);
-        vA = add4(vA, scl4(scl4(lin, rb.imA), rl));
-        wA = add4(wA, scl4(mt_mul1(rb.IA, a0), rl));
-        vB = add4(vB, scl4(scl4(neg4(lin), rb.imB), rl));
-        wB = add4(wB, scl4(mt_mul1(rb.IB, a1), rl));
+    if (fv[0] != 0.f) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const float fl = fv[2 + q];
+            if (fl == 0.f) continue;
+            v.x += f.M[q][0] * fl; v.y += f.M[q][1] * fl; v.z += f.M[q][2] * fl;
+        }
     }
+    put_vel(slot, body, l, v, vel, linvel, angvel);
 }
 
 // After the solve: the impulses go back from the packed solve arrays to the
@@ -648,7 +771,7 @@ __global__ void k_save_prev(const int *counters, ConstraintSoA cs, const int *so
         f = pk_fric[pos];
         cs.lambda[k] = l;
         cs.fric[k] = f;
-    } else {  // not solved (tile capacity exceeded): the initial impulses stay
+    } else {  // solved in place, or not at all (tile capacity exceeded): the initial impulses
         l = cs.lambda[k];
         f = cs.fric[k];
     }
@@ -663,11 +786,16 @@ __global__ void k_save_prev(const int *counters, ConstraintSoA cs, const int *so
     }
 }
 
-// Per step, after the colouring: each tile's rows in solve order as packed
-// arrays (constraint fields, both bodies' inverse mass, world inverse inertia
-// and position, and their slots in a dense list of the tile's dynamic
-// bodies), so that a solve launch reads them contiguously, with no hashing
-// and no gathers through body indices.
+// Per step, after the colouring: each tile's dynamic bodies as a dense list
+// and each row's slots in it, so that a solve does no hashing.  Spatial tiles
+// also get their rows in solve order as packed arrays with everything of a
+// row that no sweep changes already formed (the Jacobians, the velocity
+// changes per impulse): 20 launches read them, contiguously.  (A scene's rows
+// are read by one launch, which forms them itself from the constraints: packed
+// for it as well, they took this kernel from 130 to 265 us at 4,096 scenes.)
+// Four lanes pack a row, each the quarter that the same lane of the solver's
+// quad reads.
+constexpr int SOLVED_IN_PLACE = -2;  // solve_pos: the solve stores to the constraint itself
 struct PackLDS {
     int key[HASH_SLOTS];
     int dense[HASH_SLOTS];
@@ -675,11 +803,12 @@ struct PackLDS {
 };
 __global__ __launch_bounds__(TB) void k_tile_pack(
     const int *__restrict__ tile_first, const int *__restrict__ tile_cnt,
-    const int *__restrict__ order, ConstraintSoA cs, const float4 *__restrict__ pos,
-    const float *__restrict__ inv_mass, const float4 *__restrict__ invI, PackedRows pk,
-    int *__restrict__ solve_pos, int *__restrict__ tile_bodies, int *__restrict__ tile_nb,
+    const int *__restrict__ order, const int *__restrict__ row_color, ConstraintSoA cs,
+    const float4 *__restrict__ pos, const float *__restrict__ inv_mass,
+    const float4 *__restrict__ invI, PackedRows pk, int *__restrict__ solve_pos,
+    int *__restrict__ tile_bodies, int *__restrict__ tile_nb,
     const int *__restrict__ tile_ncolors, int4 *__restrict__ tile_hdr, int *counters,
-    int precompute) {
+    int spatial) {
     __shared__ PackLDS L;
     const int t = blockIdx.x, tid = threadIdx.x;
     const int first = tile_first[t];
@@ -715,148 +844,60 @@ __global__ __launch_bounds__(TB) void k_tile_pack(
         tile_hdr[t] = make_int4(first, R, tile_ncolors[t], nb < SOLVE_SLOTS ? nb : SOLVE_SLOTS);
         atomicAdd(counters + RB_CNT_SOLVE_BODIES, nb);
     }
-    for (int r = tid; r < R; r += TB) {
+    const int l = tid & 3, side = l >> 1;
+    const bool ang = l & 1;
+    for (int r = tid >> 2; r < R; r += TB / 4) {
         const int i = first + r;
         const int k = order[i];
         const int2 bd = cs.bodies[k];
-        const float imA = inv_mass[bd.x], imB = inv_mass[bd.y];
-        int sa = SLOT_STATIC, sb = SLOT_STATIC;
-        if (imA != 0.f) {
-            int h = hash_find<HASH_SLOTS>(L.key, bd.x);
-            sa = h >= 0 && L.dense[h] < SOLVE_SLOTS ? L.dense[h] : SLOT_GLOBAL;
-        }
-        if (imB != 0.f) {
-            int h = hash_find<HASH_SLOTS>(L.key, bd.y);
-            sb = h >= 0 && L.dense[h] < SOLVE_SLOTS ? L.dense[h] : SLOT_GLOBAL;
-        }
-        pk.lin0[i] = cs.linear[k];
-        pk.jac[i] = cs.jac_inv[k];
-        pk.b[i] = cs.b[k];
-        pk.lam[i] = cs.lambda[k];
-        pk.fric[i] = cs.fric[k];
-        pk.cen[i] = cs.center[k];
-        for (int q = 0; q < 4; q++) pk.p[4 * (size_t)i + q] = cs.pos[4 * (size_t)k + q];
-        pk.meta[i] = make_int4(bd.x, bd.y, sa, sb);
-        pk.im[i] = make_float2(imA, imB);
-        for (int q = 0; q < 3; q++) {
-            pk.IA[3 * (size_t)i + q] = invI[3 * (size_t)bd.x + q];
-            pk.IB[3 * (size_t)i + q] = invI[3 * (size_t)bd.y + q];
-        }
-        const float4 pA = pos[bd.x], pB = pos[bd.y];
-        pk.pA[i] = pA;
-        pk.pB[i] = pB;
-        solve_pos[k] = i;
-        // velocity-independent terms of the normal row (as row_normal forms
-        // them), read by the spatial tiles' normal sweeps only
-        if (precompute) {
-            const float4 lin0 = cs.linear[k];
-            const float4 n = neg4(lin0), lin = neg4(n);
-            float4 IA[3], IB[3];
-            for (int q = 0; q < 3; q++) {
-                IA[q] = invI[3 * (size_t)bd.x + q];
-                IB[q] = invI[3 * (size_t)bd.y + q];
+        const int body = side ? bd.y : bd.x;
+        const float imA = inv_mass[bd.x], imB = inv_mass[bd.y], im = side ? imB : imA;
+        if (!ang) {
+            int slot = SLOT_STATIC;
+            if (im != 0.f) {
+                const int h = hash_find<HASH_SLOTS>(L.key, body);
+                slot = h >= 0 && L.dense[h] < SOLVE_SLOTS ? L.dense[h] : SLOT_GLOBAL;
             }
-            for (int q = 0; q < 4; q++) {
-                const float4 wp = cs.pos[4 * (size_t)k + q];
-                const float4 r0 = sub4(wp, pA), r1 = sub4(wp, pB);
-                const float4 a0 = neg4(cross3(r0, n)), a1 = cross3(r1, n);
-                pk.na0[4 * (size_t)i + q] = a0;
-                pk.na1[4 * (size_t)i + q] = a1;
-                pk.nia0[4 * (size_t)i + q] = mt_mul1(IA, a0);
-                pk.nia1[4 * (size_t)i + q] = mt_mul1(IB, a1);
+            pk.meta[2 * (size_t)i + side] = make_int2(body, slot | row_color[k] << 16);
+        }
+        if (!spatial) {
+            if (l == 0) solve_pos[k] = SOLVED_IN_PLACE;
+            continue;
+        }
+        const float4 lin0 = cs.linear[k], fr = cs.fric[k];
+        const float4 pA = pos[bd.x], pB = pos[bd.y], p = sel4(side, pB, pA);
+        float4 I[3], wp[4];
+        for (int q = 0; q < 3; q++) I[q] = invI[3 * (size_t)body + q];
+        for (int q = 0; q < 4; q++) wp[q] = cs.pos[4 * (size_t)k + q];
+        if (l == 0) {
+            pk.lin0[i] = lin0;
+            pk.lam[i] = cs.lambda[k];
+            solve_pos[k] = i;
+        } else if (l == 1) {
+            pk.jac[i] = cs.jac_inv[k];
+        } else if (l == 2) {
+            pk.b[i] = cs.b[k];
+        } else {
+            pk.fric[i] = fr;
+        }
+        float4 J[4], M[4];
+        form_normal(side, ang, lin0, im, I, p, wp, J, M);
+        float4 *nj = pk.nj + 10 * (size_t)i + side, *nm = pk.nm + 10 * (size_t)i + side;
+        for (int q = 0; q < 4; q++)
+            if (ang || q == 0) {
+                nj[ang ? 2 * (q + 1) : 0] = J[q];
+                nm[ang ? 2 * (q + 1) : 0] = M[q];
             }
-            pk.nl[2 * (size_t)i] = scl4(lin, imA);
-            pk.nl[2 * (size_t)i + 1] = scl4(neg4(lin), imB);
+        const float4 cen = cs.center[k];
+        form_friction(side, ang, lin0, im, I, p, cen, J, M);
+        const bool damp = row_damps(pA, pB, cen, imA, imB);
+        float4 *fj = pk.fj + 8 * (size_t)i + l, *fm = pk.fm + 8 * (size_t)i + l;
+        for (int q = 0; q < 2; q++) {
+            J[q].w = damp ? 1.f : 0.f;  // (no sweep reads w)
+            fj[4 * q] = J[q];
+            fm[4 * q] = M[q];
         }
     }
-}
-
-// One row of a sweep (mode 0 normal, 1 friction, 2 warm start), velocities
-// from the LDS cache or, for bodies that did not fit it, global memory.
-template <bool RES = true>
-__device__ __forceinline__ void run_row(int mode, RowData &d, const RowBodies &rb, SolveLDS &L,
-                                        float4 *linvel, float4 *angvel, float friction,
-                                        float &rmax, float &lmax) {
-    float4 vA, wA, vB, wB;
-    fetch_vel(rb.ha, rb.a, L, linvel, angvel, vA, wA);
-    fetch_vel(rb.hb, rb.b, L, linvel, angvel, vB, wB);
-    if (mode == 0) row_normal<RES>(d, vA, wA, vB, wB, rb, rmax, lmax);
-    else if (mode == 1) row_friction<RES>(d, vA, wA, vB, wB, rb, friction, rmax, lmax);
-    else row_warm(d, vA, wA, vB, wB, rb);
-    if (rb.ha >= 0) { L.v[rb.ha] = vA; L.w[rb.ha] = wA; }
-    else if (rb.ha == SLOT_GLOBAL) { linvel[rb.a] = vA; angvel[rb.a] = wA; }
-    if (rb.hb >= 0) { L.v[rb.hb] = vB; L.w[rb.hb] = wB; }
-    else if (rb.hb == SLOT_GLOBAL) { linvel[rb.b] = vB; angvel[rb.b] = wB; }
-}
-
-// A normal row with its velocity-independent terms precomputed by
-// k_tile_pack (the same operations as row_normal performs, so the results
-// are identical): what a launch of normal sweeps needs.
-struct NormalRow {
-    float4 lin0, jac, bb, lam;
-    float4 a0[4], a1[4], ia0[4], ia1[4];
-    float4 l0, l1;  // lin0 * imA, -lin0 * imB
-    int a, b, ha, hb;
-};
-__device__ __forceinline__ void load_normal(int i, const PackedRows &pk, NormalRow &r) {
-    r.lin0 = pk.lin0[i];
-    r.jac = pk.jac[i];
-    r.bb = pk.b[i];
-    r.lam = pk.lam[i];
-    for (int q = 0; q < 4; q++) {
-        r.a0[q] = pk.na0[4 * (size_t)i + q];
-        r.a1[q] = pk.na1[4 * (size_t)i + q];
-        r.ia0[q] = pk.nia0[4 * (size_t)i + q];
-        r.ia1[q] = pk.nia1[4 * (size_t)i + q];
-    }
-    r.l0 = pk.nl[2 * (size_t)i];
-    r.l1 = pk.nl[2 * (size_t)i + 1];
-    const int4 m = pk.meta[i];
-    r.a = m.x;
-    r.b = m.y;
-    r.ha = m.z;
-    r.hb = m.w;
-}
-// row_normal on a NormalRow
-template <bool RES = true>
-__device__ __forceinline__ void row_normal_pre(NormalRow &d, float4 &vA, float4 &wA, float4 &vB,
-                                               float4 &wB, float &rmax, float &lmax) {
-    const float4 lin0 = d.lin0;
-    float jv[4] = {d.jac.x, d.jac.y, d.jac.z, d.jac.w};
-    float bv[4] = {d.bb.x, d.bb.y, d.bb.z, d.bb.w};
-    float lv[4] = {d.lam.x, d.lam.y, d.lam.z, d.lam.w};
-#pragma unroll
-    for (int ic = 0; ic < 4; ic++) {
-        if (jv[ic] == 0.f) continue;
-        float rl = rel_vel(lin0, neg4(lin0), d.a0[ic], d.a1[ic], vA, wA, vB, wB) + bv[ic];
-        rl *= jv[ic];
-        float prev = lv[ic];
-        float upd = prev + rl;
-        upd = fmaxf(upd, 0.f);
-        upd = fminf(upd, FLT_MAX);
-        rl = upd - prev;
-        lv[ic] = upd;
-        vA = add4(vA, scl4(d.l0, rl)); wA = add4(wA, scl4(d.ia0[ic], rl));
-        vB = add4(vB, scl4(d.l1, rl)); wB = add4(wB, scl4(d.ia1[ic], rl));
-        if (RES) {
-            float sc = fabsf(rl) / fabsf(jv[ic]);
-            rmax = fmaxf(rmax, sc);
-            lmax = fmaxf(lmax, fabsf(upd));
-        }
-    }
-    d.lam = mk4(lv[0], lv[1], lv[2], lv[3]);
-}
-template <bool RES = true>
-__device__ __forceinline__ void run_row_normal(NormalRow &d, SolveLDS &L, float4 *linvel,
-                                               float4 *angvel, float &rmax, float &lmax) {
-    float4 vA, wA, vB, wB;
-    fetch_vel(d.ha, d.a, L, linvel, angvel, vA, wA);
-    fetch_vel(d.hb, d.b, L, linvel, angvel, vB, wB);
-    row_normal_pre<RES>(d, vA, wA, vB, wB, rmax, lmax);
-    if (d.ha >= 0) { L.v[d.ha] = vA; L.w[d.ha] = wA; }
-    else if (d.ha == SLOT_GLOBAL) { linvel[d.a] = vA; angvel[d.a] = wA; }
-    if (d.hb >= 0) { L.v[d.hb] = vB; L.w[d.hb] = wB; }
-    else if (d.hb == SLOT_GLOBAL) { linvel[d.b] = vB; angvel[d.b] = wB; }
 }
 
 // The sweep residual terms (largest scaled impulse change, largest impulse)
@@ -898,254 +939,357 @@ __device__ __forceinline__ void add_sweep_residual(float *residual, int sweep, f
     __syncthreads();
 }
 
-// Shared state of one tile's solve: the LDS velocity cache and the
-// tile-wide residual reduction of the current sweep.
-struct TileSolveLDS {
-    SolveLDS c;
-    unsigned int red[2];
-    unsigned int gred[2];  // add_sweep_residual's workgroup maxima
+// A tile's sweeps take their rows through a row source: load(i, row) and
+// store(i, row) of normal and friction rows by solve position, from the packed
+// arrays (spatial tiles: a row is read by 20 launches) or straight from the
+// constraints (scene tiles: one launch reads it once and keeps it).
+struct PackedSource {
+    const PackedRows &pk;
+    float friction;
+    __device__ void load(int i, int l, NormalRow &r) const { load_normal(i, l, pk, r); }
+    __device__ void load(int i, int l, FrictionRow &r) const { load_friction(i, l, pk, friction, r); }
+    __device__ void store(int i, int l, const NormalRow &r) const {
+        reinterpret_cast<float *>(pk.lam + i)[l] = r.lam;
+    }
+    __device__ void store(int i, int l, const FrictionRow &r) const {
+        if (l & 2) reinterpret_cast<float *>(pk.fric + i)[l] = r.fr;
+    }
 };
-
-// The sweeps of one tile: the optional warm-start pass, then normal sweeps,
-// then friction sweeps, over the tile's packed rows (positions first..first+R
-// in solve order).  REG: the tile has at most TBK rows and row r lives in the
-// registers of thread r for the whole launch (rd, rb and its colour rc,
-// loaded by the caller; stored once at the end);
-// otherwise rows are read from the packed arrays on every pass.  Within a
-// colour rows share no dynamic body, so the thread that runs a row does not
-// change the result.  local_tol: a scene tile ends each phase as soon as its
-// own residual is below sp.tol.
-template <int TBK, bool REG, bool RES>
-__device__ __forceinline__ void tile_sweeps(const StepParams &sp, int sweep0, int nsweeps_n,
-                                            int nsweeps_f, int warm, bool local_tol, int first,
-                                            int R, int nc, const int *coff, const PackedRows &pk,
-                                            float4 *linvel, float4 *angvel, float *residual,
-                                            TileSolveLDS &L, int used[2], float rfin[2],
-                                            RowData &rd, RowBodies &rb, int rc) {
-    const int tid = threadIdx.x;
-    bool swept = false;
-    for (int phase = warm ? -1 : 0; phase < 2; phase++) {
-        const int nsw = phase < 0 ? 1 : (phase == 0 ? nsweeps_n : nsweeps_f);
-        const int mode = phase < 0 ? 2 : phase;
-        for (int it = 0; it < nsw; it++) {
-            float rmax = 0.f, lmax = 0.f;
-            if (local_tol) {
-                if (tid == 0) { L.red[0] = 0u; L.red[1] = 0u; }
-                __syncthreads();
-            }
-            for (int c = 0; c < nc; c++) {
-                if (REG) {
-                    if (rc == c)
-                        run_row<RES>(mode, rd, rb, L.c, linvel, angvel, sp.friction, rmax, lmax);
-                } else {
-                    int c0 = coff[c], c1 = coff[c + 1];
-                    if (c1 > R) c1 = R;
-                    for (int r = c0 + tid; r < c1; r += TBK) {
-                        RowData d;
-                        RowBodies b;
-                        load_packed(first + r, pk, d, b);
-                        run_row<RES>(mode, d, b, L.c, linvel, angvel, sp.friction, rmax, lmax);
-                        if (mode == 0) pk.lam[first + r] = d.lam;
-                        else if (mode == 1) pk.fric[first + r] = d.fr;
-                    }
-                }
-                __syncthreads();
-            }
-            if (phase < 0) continue;
-            swept = true;
-            const int sweep = sweep0 + (phase == 0 ? it : nsweeps_n + it);
-            if (RES && sweep_residual_needed(sp, sweep)) add_sweep_residual(residual, sweep, rmax, lmax, L.gred);
-            if (local_tol) {
-                // rmax, lmax >= 0: their float bits order like the values
-                if (rmax > 0.f) atomicMax(&L.red[0], __float_as_uint(rmax));
-                if (lmax > 0.f) atomicMax(&L.red[1], __float_as_uint(lmax));
-                __syncthreads();
-                float rm = __uint_as_float(L.red[0]), lm = __uint_as_float(L.red[1]);
-                float r = rm / (lm > 1.f ? lm : 1.f);
-                used[phase] = it + 1;
-                rfin[phase] = r;
-                __syncthreads();  // every thread has read red before the next reset
-                if (r < sp.tol) break;
-            }
-        }
+struct ConstraintSource {
+    const PackedRows &pk;
+    const SolveView &sv;
+    float friction;
+    __device__ void load(int i, int l, NormalRow &r) const { load_normal(i, l, pk, sv, r); }
+    __device__ void load(int i, int l, FrictionRow &r) const {
+        load_friction(i, l, pk, sv, friction, r);
     }
-    if (REG && tid < R && swept) {
-        pk.lam[first + tid] = rd.lam;
-        pk.fric[first + tid] = rd.fr;
+    __device__ void store(int i, int l, const NormalRow &r) const {
+        reinterpret_cast<float *>(sv.cs.lambda + sv.order[i])[l] = r.lam;
     }
+    __device__ void store(int i, int l, const FrictionRow &r) const {
+        if (l & 2) reinterpret_cast<float *>(sv.cs.fric + sv.order[i])[l] = r.fr;
+    }
+};
+template <bool RES>
+__device__ __forceinline__ void run_row(NormalRow &d, int i, int l, const PackedRows &pk,
+                                        float4 *vel, float4 *linvel, float4 *angvel, float &rmax,
+                                        float &lmax) {
+    run_normal<RES>(d, i, l, pk, vel, linvel, angvel, rmax, lmax);
+}
+template <bool RES>
+__device__ __forceinline__ void run_row(FrictionRow &d, int i, int l, const PackedRows &pk,
+                                        float4 *vel, float4 *linvel, float4 *angvel, float &rmax,
+                                        float &lmax) {
+    run_friction<RES>(d, i, l, pk, vel, linvel, angvel, rmax, lmax);
 }
 
-// One normal sweep of a tile on precomputed rows (spatial tiles: a launch
-// per sweep and parity phase).  REG: row tid is nr, colour rc.
-template <int TBK, bool REG, bool RES>
-__device__ __forceinline__ void tile_normal_sweep(const StepParams &sp, int sweep, int first,
-                                                  int R, int nc, const int *coff,
-                                                  const PackedRows &pk,
-                                                  float4 *linvel, float4 *angvel,
-                                                  float *residual, TileSolveLDS &L,
-                                                  NormalRow &nr, int rc) {
-    const int tid = threadIdx.x;
-    float rmax = 0.f, lmax = 0.f;
-    for (int c = 0; c < nc; c++) {
-        if (REG) {
-            if (rc == c) run_row_normal<RES>(nr, L.c, linvel, angvel, rmax, lmax);
-        } else {
-            int c0 = coff[c], c1 = coff[c + 1];
-            if (c1 > R) c1 = R;
-            for (int r = c0 + tid; r < c1; r += TBK) {
-                NormalRow d;
-                load_normal(first + r, pk, d);
-                run_row_normal<RES>(d, L.c, linvel, angvel, rmax, lmax);
-                pk.lam[first + r] = d.lam;
-            }
-        }
-        __syncthreads();
+// The quad of a thread among the QN quads that share a tile, and its lane.
+struct Quad {
+    int QN, q, l;
+};
+// The rows of a tile of at most K * QN rows in the registers of QN quads: row
+// r in quad r % QN, set r / QN.  Within a colour rows share no dynamic body,
+// so which quad runs a row does not change the result.
+template <int K, class Row, class Src>
+__device__ __forceinline__ void load_rows(Row (&row)[K], Quad u, const Src &src, int first, int R) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        row[k].code = -1;
+        if (k * u.QN + u.q < R) src.load(first + k * u.QN + u.q, u.l, row[k]);
     }
-    if (RES && sweep_residual_needed(sp, sweep)) add_sweep_residual(residual, sweep, rmax, lmax, L.gred);
-    if (REG && tid < R) pk.lam[first + tid] = nr.lam;
+}
+template <int K, class Row, class Src>
+__device__ __forceinline__ void store_rows(const Row (&row)[K], Quad u, const Src &src, int first,
+                                           int R) {
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if (k * u.QN + u.q < R) src.store(first + k * u.QN + u.q, u.l, row[k]);
+}
+// One sweep, colour by colour; sync() orders the velocities between colours
+// among the tile's threads (after_last: what every thread does between the
+// last colour and its sync).
+template <int K, bool RES, class Row, class S, class F>
+__device__ __forceinline__ void sweep_rows(Row (&row)[K], Quad u, int first, int nc,
+                                           const PackedRows &pk, float4 *vel, float4 *linvel,
+                                           float4 *angvel, float &rmax, float &lmax, S sync,
+                                           F after_last) {
+    for (int c = 0; c < nc; c++) {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (row[k].code >> 16 == c)
+                run_row<RES>(row[k], first + k * u.QN + u.q, u.l, pk, vel, linvel, angvel, rmax,
+                             lmax);
+        if (c == nc - 1) after_last();
+        sync();
+    }
+}
+// The same for a tile of more rows: they are read on every pass.
+template <bool RES, class Row, class Src, class S, class F>
+__device__ __forceinline__ void sweep_memory(Quad u, const Src &src, int first, int R, int nc,
+                                             const int *coff, const PackedRows &pk, float4 *vel,
+                                             float4 *linvel, float4 *angvel, float &rmax,
+                                             float &lmax, S sync, F after_last) {
+    for (int c = 0; c < nc; c++) {
+        const int c1 = min(coff[c + 1], R);
+        for (int r = coff[c] + u.q; r < c1; r += u.QN) {
+            Row d;
+            src.load(first + r, u.l, d);
+            run_row<RES>(d, first + r, u.l, pk, vel, linvel, angvel, rmax, lmax);
+            src.store(first + r, u.l, d);
+        }
+        if (c == nc - 1) after_last();
+        sync();
+    }
+}
+template <class Src, class S>
+__device__ __forceinline__ void sweep_warm(Quad u, const Src &src, int first, int R, int nc,
+                                           const int *coff, const PackedRows &pk, float4 *vel,
+                                           float4 *linvel, float4 *angvel, S sync) {
+    for (int c = 0; c < nc; c++) {
+        const int c1 = min(coff[c + 1], R);
+        for (int r = coff[c] + u.q; r < c1; r += u.QN) {
+            NormalRow d;
+            FrictionRow f;
+            src.load(first + r, u.l, d);
+            src.load(first + r, u.l, f);
+            run_warm(d, f, first + r, u.l, pk, vel, linvel, angvel);
+        }
+        sync();
+    }
 }
 
 // The tile's dynamic bodies' velocities into LDS slots (slot s: body
-// bodies[s]).  Thread tid keeps the body of slot tid (every slot when nb <=
-// TBK) in a register for the store back, which then waits on no index load.
-template <int TBK>
-__device__ __forceinline__ int gather_velocities(const int *__restrict__ bodies, int nb,
-                                                 const float4 *__restrict__ linvel,
-                                                 const float4 *__restrict__ angvel, SolveLDS &L) {
-    const int tid = threadIdx.x;
-    const int b0 = tid < nb ? bodies[tid] : 0;
-    if (tid < nb) {
-        L.v[tid] = linvel[b0];
-        L.w[tid] = angvel[b0];
-    }
-    for (int s = tid + TBK; s < nb; s += TBK) {
-        const int b = bodies[s];
-        L.v[s] = linvel[b];
-        L.w[s] = angvel[b];
-    }
+// bodies[s]), thread pairs of a slot taking its linear and its angular half
+// (nt threads, tid counted among them).  Thread tid keeps the body of slot
+// tid / 2 in a register for the store back, which then waits on no index load.
+__device__ __forceinline__ int gather_velocities(int tid, int nt, const int *__restrict__ bodies,
+                                                 int nb, const float4 *__restrict__ linvel,
+                                                 const float4 *__restrict__ angvel, float4 *vel) {
+    const float4 *src = tid & 1 ? angvel : linvel;
+    const int b0 = tid < 2 * nb ? bodies[tid >> 1] : 0;
+    if (tid < 2 * nb) vel[2 + tid] = src[b0];
+    for (int s = tid + nt; s < 2 * nb; s += nt) vel[2 + s] = src[bodies[s >> 1]];
+    if (tid < 2) vel[tid] = mk4(0.f, 0.f, 0.f, 0.f);
     return b0;
 }
-template <int TBK>
-__device__ __forceinline__ void store_velocities(const int *__restrict__ bodies, int nb, int b0,
-                                                 float4 *__restrict__ linvel,
-                                                 float4 *__restrict__ angvel, const SolveLDS &L) {
-    const int tid = threadIdx.x;
-    if (tid < nb) {
-        linvel[b0] = L.v[tid];
-        angvel[b0] = L.w[tid];
-    }
-    for (int s = tid + TBK; s < nb; s += TBK) {
-        const int b = bodies[s];
-        linvel[b] = L.v[s];
-        angvel[b] = L.w[s];
-    }
+__device__ __forceinline__ void store_velocities(int tid, int nt, const int *__restrict__ bodies,
+                                                 int nb, int b0, float4 *__restrict__ linvel,
+                                                 float4 *__restrict__ angvel, const float4 *vel) {
+    float4 *dst = tid & 1 ? angvel : linvel;
+    if (tid < 2 * nb) dst[b0] = vel[2 + tid];
+    for (int s = tid + nt; s < 2 * nb; s += nt) dst[bodies[s >> 1]] = vel[2 + s];
 }
 
-// One workgroup per tile (spatial: the tiles of one parity phase; scene: one
-// scene); the tile's dynamic body velocities live in LDS for the launch.
-// The solve of one tile (rows first..first+R of the packed arrays): its
-// dynamic bodies' velocities gathered into LDS, the sweeps, the velocities
-// stored back.  NORMAL: one normal sweep on the precomputed rows.
-// RES: the launch's sweeps compute their residual terms (a launch of one
-// sweep whose residual is not reported runs without them)
-template <int TBK, bool NORMAL, bool RES>
-__device__ __forceinline__ void solve_tile(
-    const StepParams &sp, int t, int sweep0, int nsweeps_n, int nsweeps_f, int warm,
-    const int4 *__restrict__ tile_hdr, const int *__restrict__ tile_color_off,
-    const int *__restrict__ tile_bodies, const PackedRows &pk, float4 *__restrict__ linvel,
-    float4 *__restrict__ angvel, float *__restrict__ residual, int *counters,
-    int4 *__restrict__ tile_stats, TileSolveLDS &L) {
-    const bool local_tol = sp.tile_mode == 1 && sp.tol > 0.f;
-    const int tid = threadIdx.x;
+// Spatial tiles: one sweep (MODE: normal, friction, or the warm start's
+// impulses) over the tiles of one parity phase, a workgroup per tile, the
+// tile's dynamic body velocities in LDS.
+template <int TBK, int MODE, bool RES>
+__global__ __launch_bounds__(TBK) void k_tile_solve(
+    StepParams sp, int phase, int sweep, const int4 *__restrict__ tile_hdr,
+    const int *__restrict__ tile_color_off, const int *__restrict__ tile_bodies, PackedRows pk,
+    float4 *linvel, float4 *angvel, float *__restrict__ residual, const int *counters) {
+    constexpr int K = 2;
+    __shared__ TileSolveLDS L;
+    // tiles of this phase: (tx & 1, tz & 1) == (phase & 1, phase >> 1)
+    const int px = phase & 1, pz = phase >> 1;
+    const int nx = (sp.tiles_x - px + 1) / 2;
+    const int tx = px + 2 * (int)(blockIdx.x % nx), tz = pz + 2 * (int)(blockIdx.x / nx);
+    if (tx >= sp.tiles_x || tz >= sp.tiles_z) return;
+    const int t = tz * sp.tiles_x + tx, tid = threadIdx.x;
     // (first, rows, colours, cached bodies) of the tile, written by k_tile_pack
     const int4 hdr = tile_hdr[t];
     if (sp.tol > 0.f && counters[RB_CNT_DONE] != 0) return;  // converged in an earlier sweep
     const int first = hdr.x, R = hdr.y, nc = hdr.z, nb = hdr.w;
+    if (R <= 0) return;
+    const int *coff = tile_color_off + t * (RB_MAX_LOCAL_COLORS + 1);
+    const int *bodies = tile_bodies + 2 * (size_t)first;
+    if (tid < 2) L.gred[tid] = 0u;
+    float rmax = 0.f, lmax = 0.f;
+    auto sync = []() { __syncthreads(); };
+    auto nothing = []() {};
+    const Quad u{TBK / 4, tid >> 2, tid & 3};
+    const PackedSource src{pk, sp.friction};
+    int b0;
+    if constexpr (MODE == ROW_WARM) {
+        b0 = gather_velocities(tid, TBK, bodies, nb, linvel, angvel, L.vel);
+        __syncthreads();
+        sweep_warm(u, src, first, R, nc, coff, pk, L.vel, linvel, angvel, sync);
+    } else {
+        using Row = std::conditional_t<MODE == ROW_NORMAL, NormalRow, FrictionRow>;
+        if (R <= K * TBK / 4) {
+            // (the rows' loads go out before the velocity gather's)
+            Row row[K];
+            load_rows(row, u, src, first, R);
+            b0 = gather_velocities(tid, TBK, bodies, nb, linvel, angvel, L.vel);
+            __syncthreads();
+            sweep_rows<K, RES>(row, u, first, nc, pk, L.vel, linvel, angvel, rmax, lmax, sync,
+                               nothing);
+            store_rows(row, u, src, first, R);
+        } else {
+            b0 = gather_velocities(tid, TBK, bodies, nb, linvel, angvel, L.vel);
+            __syncthreads();
+            sweep_memory<RES, Row>(u, src, first, R, nc, coff, pk, L.vel, linvel, angvel, rmax,
+                                   lmax, sync, nothing);
+        }
+    }
+    if (RES) add_sweep_residual(residual, sweep, rmax, lmax, L.gred);
+    store_velocities(tid, TBK, bodies, nb, b0, linvel, angvel, L.vel);
+}
+
+// Scene tiles: every sweep of a scene in one workgroup, the warm-start pass
+// first; with a tolerance a scene ends each phase as soon as its own residual
+// is below it.  A workgroup (a whole CU: 1,024 threads of up to 128 registers)
+// solves 2^lg scenes, each with 1024 >> lg threads whose quads hold two rows
+// each in registers, lg by the scene's rows (scene_class).  The scenes of a
+// workgroup share its barriers: a scene's own barriers order its colours
+// whatever the others are at, and waves that have finished their scene end
+// and are no longer waited for.  Scenes are sorted by rows, so those that
+// share a workgroup take about as long.  What bounds a scene is its colours
+// times its sweeps in sequence; what bounds the launch at thousands of scenes
+// is how many of those chains the chip runs at once, which the registers
+// limit (124 words a row).  4,096 scenes of 8 to 512 bodies, 10 + 10 sweeps:
+// 958 -> 498 us against 256 threads per scene, a thread per row and the rows
+// of scenes above 256 read on every pass; 256 scenes to a tolerance: 2.4x.  A
+// launch per class in sequence took 612 us, and on 256 scenes, where each is
+// as long as its longest scene, twice this one's time.
+constexpr int SCENE_TB = 1024, SCENE_CLASSES = 5;
+constexpr int SCENE_SLOTS = SCENE_TB + (1 << (SCENE_CLASSES - 1));
+// Threads of a scene: at most two rows a quad while that leaves a whole wave,
+// and no fewer than leave every CU a workgroup (max_class).
+__device__ __forceinline__ int scene_class(int R, int max_class) {
+    int lg = 0;
+    while (lg < max_class && 2 * (SCENE_TB >> (lg + 1)) / 4 >= R) lg++;
+    return lg;
+}
+__global__ __launch_bounds__(SCENE_TB) void k_scene_solve(
+    StepParams sp, int warm, const int4 *__restrict__ tile_hdr,
+    const int *__restrict__ tile_color_off, const int *__restrict__ tile_bodies, PackedRows pk,
+    SolveView sv, float *__restrict__ residual, int4 *__restrict__ tile_stats,
+    const uint2 *__restrict__ tile_order, const int *__restrict__ counters) {
+    __shared__ float4 s_vel[2 * SCENE_SLOTS];
+    __shared__ unsigned int s_red[2][2][SCENE_TB / 64];  // per sweep parity: the waves' maxima
+    // this workgroup's scenes: the classes in turn, largest scenes first, so
+    // that the workgroups dispatched last are the short ones
+    int b = blockIdx.x, base = 0, lg = 0, n = 0;
+    for (; lg < SCENE_CLASSES; lg++) {
+        n = counters[RB_CNT_SCENES + lg];
+        const int wgs = (n + (1 << lg) - 1) >> lg;
+        if (b < wgs) break;
+        b -= wgs;
+        base += n;
+    }
+    if (lg == SCENE_CLASSES) return;
+    const int nt = SCENE_TB >> lg;
+    const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / nt), tid = threadIdx.x - g * nt;
+    if ((b << lg) + g >= n) return;
+    const int t = (int)tile_order[base + (b << lg) + g].y;
+    const int4 hdr = tile_hdr[t];
+    const int first = hdr.x, R = hdr.y, nc = hdr.z, nb = hdr.w;
+    const bool tol = sp.tol > 0.f;
     if (R <= 0) {
-        if (local_tol && tid == 0) tile_stats[t] = make_int4(-1, -1, 0, 0);
+        if (tol && tid == 0) tile_stats[t] = make_int4(-1, -1, 0, 0);
         return;
     }
     const int *coff = tile_color_off + t * (RB_MAX_LOCAL_COLORS + 1);
     const int *bodies = tile_bodies + 2 * (size_t)first;
-    // (the barrier after the velocity gather orders this before any use)
-    if (tid == 0) {
-        L.gred[0] = 0u;
-        L.gred[1] = 0u;
-    }
-    if constexpr (NORMAL) {
-        // one normal sweep (nsweeps_n == 1) on the precomputed rows
-        NormalRow nr;
-        int rc = -1;
-        if (R <= TBK && tid < R) {
-            load_normal(first + tid, pk, nr);
-            for (int c = 0; c < nc; c++)
-                if (coff[c] <= tid && tid < coff[c + 1]) rc = c;
-        }
-        const int b0 = gather_velocities<TBK>(bodies, nb, linvel, angvel, L.c);
-        __syncthreads();
-        if (R <= TBK)
-            tile_normal_sweep<TBK, true, RES>(sp, sweep0, first, R, nc, coff, pk, linvel, angvel,
-                                              residual, L, nr, rc);
-        else
-            tile_normal_sweep<TBK, false, RES>(sp, sweep0, first, R, nc, coff, pk, linvel,
-                                               angvel, residual, L, nr, rc);
-        __syncthreads();
-        store_velocities<TBK>(bodies, nb, b0, linvel, angvel, L.c);
-        return;
-    }
-    // a tile of at most TBK rows keeps row tid in thread tid's registers;
-    // its loads go out together with the velocity gather below
-    RowData rd;
-    RowBodies rb;
-    int rc = -1;
-    if (R <= TBK && tid < R) {
-        load_packed(first + tid, pk, rd, rb);
-        for (int c = 0; c < nc; c++)
-            if (coff[c] <= tid && tid < coff[c + 1]) rc = c;
-    }
-    const int b0 = gather_velocities<TBK>(bodies, nb, linvel, angvel, L.c);
-    __syncthreads();
+    // (a scene of a shared workgroup has at most nt / 2 rows, hence nt bodies)
+    float4 *vel = s_vel + 2 * g * (nt + 1);
+    float4 *linvel = sv.linvel, *angvel = sv.angvel;
+    const ConstraintSource src{pk, sv, sp.friction};
+    const Quad u{nt / 4, tid >> 2, tid & 3};
+    const int wave0 = g * (nt / 64), waves = nt / 64;
+    // (one wave: its LDS operations are in order)
+    auto sync = [&]() {
+        if (waves == 1) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        else __syncthreads();
+    };
+    const int b0 = gather_velocities(tid, nt, bodies, nb, linvel, angvel, vel);
+    sync();
+    if (warm) sweep_warm(u, src, first, R, nc, coff, pk, vel, linvel, angvel, sync);
+
     int used[2] = {0, 0};
     float rfin[2] = {0.f, 0.f};
-    if (R <= TBK)
-        tile_sweeps<TBK, true, RES>(sp, sweep0, nsweeps_n, nsweeps_f, warm, local_tol, first, R,
-                                    nc, coff, pk, linvel, angvel, residual, L, used, rfin, rd, rb,
-                                    rc);
-    else
-        tile_sweeps<TBK, false, RES>(sp, sweep0, nsweeps_n, nsweeps_f, warm, local_tol, first, R,
-                                     nc, coff, pk, linvel, angvel, residual, L, used, rfin, rd,
-                                     rb, rc);
-    if (local_tol && tid == 0)
+    int parity = 0;
+    // the sweeps of one phase; sweep(res, rmax, lmax, after_last) runs one.
+    // The residual is needed after every sweep with a tolerance, else of the
+    // last one.
+    auto run_phase = [&](int phase, int nsw, int sweep0, auto sweep) {
+        for (int it = 0; it < nsw; it++) {
+            float rmax = 0.f, lmax = 0.f;
+            if (!tol && it < nsw - 1) {
+                sweep(std::false_type{}, rmax, lmax, []() {});
+                continue;
+            }
+            // each wave's maxima reach the scene's threads over the last
+            // colour's sync; the buffer of the other parity is free again by
+            // the syncs of this sweep
+            unsigned int(*red)[SCENE_TB / 64] = s_red[parity];
+            parity ^= 1;
+            sweep(std::true_type{}, rmax, lmax, [&]() {
+                // (the terms are >= 0: their bits order like the values)
+                unsigned r = __float_as_uint(rmax), m = __float_as_uint(lmax);
+#pragma unroll
+                for (int o = 32; o >= 4; o >>= 1) {
+                    r = max(r, (unsigned)__shfl_xor((int)r, o));
+                    m = max(m, (unsigned)__shfl_xor((int)m, o));
+                }
+                if ((tid & 63) == 0) {
+                    red[0][wave0 + (tid >> 6)] = r;
+                    red[1][wave0 + (tid >> 6)] = m;
+                }
+            });
+            unsigned r = 0u, m = 0u;
+            for (int w = 0; w < waves; w++) {
+                r = max(r, red[0][wave0 + w]);
+                m = max(m, red[1][wave0 + w]);
+            }
+            if (tol) {
+                const float rm = __uint_as_float(r), lm = __uint_as_float(m);
+                const float res = rm / (lm > 1.f ? lm : 1.f);
+                used[phase] = it + 1;
+                rfin[phase] = res;
+                if (res < sp.tol) break;
+            } else if (tid == 0 && (r != 0u || m != 0u)) {
+                atomicMax((unsigned int *)&residual[2 * (sweep0 + it)], r);
+                atomicMax((unsigned int *)&residual[2 * (sweep0 + it) + 1], m);
+            }
+        }
+    };
+    auto solve_held = [&](auto row0, auto sets, int phase, int nsw, int sweep0) {
+        constexpr int K = decltype(sets)::value;
+        decltype(row0) row[K];
+        load_rows(row, u, src, first, R);
+        run_phase(phase, nsw, sweep0, [&](auto res, float &rmax, float &lmax, auto last) {
+            sweep_rows<K, decltype(res)::value>(row, u, first, nc, pk, vel, linvel, angvel, rmax,
+                                                lmax, sync, last);
+        });
+        store_rows(row, u, src, first, R);
+    };
+    auto solve_rows = [&](auto row0, int phase, int nsw, int sweep0) {
+        if (R <= 2 * u.QN) {
+            solve_held(row0, std::integral_constant<int, 2>{}, phase, nsw, sweep0);
+        } else if (R <= 3 * u.QN) {
+            // (a few of the third set's registers spill, which is still faster
+            // than reading the rows again)
+            solve_held(row0, std::integral_constant<int, 3>{}, phase, nsw, sweep0);
+        } else {
+            run_phase(phase, nsw, sweep0, [&](auto res, float &rmax, float &lmax, auto last) {
+                sweep_memory<decltype(res)::value, decltype(row0)>(
+                    u, src, first, R, nc, coff, pk, vel, linvel, angvel, rmax, lmax, sync, last);
+            });
+        }
+    };
+    if (sp.normal_iters > 0) {
+        solve_rows(NormalRow{}, 0, sp.normal_iters, 0);
+        // the friction rows read the stored normal impulses
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        sync();
+    }
+    if (sp.friction_iters > 0) solve_rows(FrictionRow{}, 1, sp.friction_iters, sp.normal_iters);
+    if (tol && tid == 0)
         tile_stats[t] = make_int4(used[0], used[1], (int)__float_as_uint(rfin[0]),
                                   (int)__float_as_uint(rfin[1]));
-    __syncthreads();
-    store_velocities<TBK>(bodies, nb, b0, linvel, angvel, L.c);
-}
-
-
-template <int TBK, bool NORMAL = false, bool RES = true>
-__global__ __launch_bounds__(TBK) void k_tile_solve(
-    StepParams sp, int phase, int sweep0, int nsweeps_n, int nsweeps_f, int warm,
-    const int4 *__restrict__ tile_hdr, const int *__restrict__ tile_color_off,
-    const int *__restrict__ tile_bodies, PackedRows pk,
-    float4 *__restrict__ linvel, float4 *__restrict__ angvel, float *__restrict__ residual,
-    int *counters, int4 *__restrict__ tile_stats, const uint2 *__restrict__ tile_order) {
-    __shared__ TileSolveLDS L;
-    int t;
-    if (sp.tile_mode == 1) {
-        // largest scenes first: the workgroups dispatched last are the short ones
-        t = (int)tile_order[blockIdx.x].y;
-    } else {
-        // tiles of this phase: (tx & 1, tz & 1) == (phase & 1, phase >> 1)
-        int px = phase & 1, pz = phase >> 1;
-        int nx = (sp.tiles_x - px + 1) / 2;
-        int bx = blockIdx.x % nx, bz = blockIdx.x / nx;
-        int tx = px + 2 * bx, tz = pz + 2 * bz;
-        if (tx >= sp.tiles_x || tz >= sp.tiles_z) return;
-        t = tz * sp.tiles_x + tx;
-    }
-    solve_tile<TBK, NORMAL, RES>(sp, t, sweep0, nsweeps_n, nsweeps_f, warm, tile_hdr, tile_color_off,
-                            tile_bodies, pk, linvel, angvel, residual, counters, tile_stats, L);
+    store_velocities(tid, nt, bodies, nb, b0, linvel, angvel, vel);
 }
 
 // Scene tiles with a tolerance: sweeps used and final residuals over the
@@ -1279,32 +1423,46 @@ hipError_t launch_tiles(const DeviceWorld &d, const StepParams &p, hipStream_t s
                        d.tile_cnt, d.cs.bodies, d.inv_mass, d.solve_order, d.row_color,
                        d.tile_color_off, d.tile_ncolors, d.counters);
     RB_LAUNCH(k_tile_pack, dim3(p.n_tiles), dim3(TB), 0, s, d.tile_first, d.tile_cnt,
-                       d.solve_order, d.cs, d.pos, d.inv_mass, d.inv_inertia_world, d.pk,
-                       d.solve_pos, d.tile_bodies, d.tile_nb, d.tile_ncolors, d.tile_hdr,
+                       d.solve_order, d.row_color, d.cs, d.pos, d.inv_mass, d.inv_inertia_world,
+                       d.pk, d.solve_pos, d.tile_bodies, d.tile_nb, d.tile_ncolors, d.tile_hdr,
                        d.counters, p.tile_mode == 0 ? 1 : 0);
     return rb_launch_status();
 }
 
 namespace {
-__global__ void k_tile_order_keys(int n_tiles, const int4 *__restrict__ tile_hdr,
-                                  uint2 *__restrict__ kv) {
+__global__ void k_tile_order_keys(int n_tiles, int max_class, const int4 *__restrict__ tile_hdr,
+                                  uint2 *__restrict__ kv, int *counters) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_tiles) return;
-    const int R = tile_hdr[t].y;
-    const uint32_t r = (uint32_t)(R < 0 ? 0 : (R > 0xffff ? 0xffff : R));
-    kv[t] = make_uint2(0xffffu - r, (uint32_t)t);
+    int lg = -1;
+    if (t < n_tiles) {
+        const int R = tile_hdr[t].y;
+        const uint32_t r = (uint32_t)(R < 0 ? 0 : (R > 0xffff ? 0xffff : R));
+        kv[t] = make_uint2(0xffffu - r, (uint32_t)t);
+        lg = scene_class(R, max_class);
+    }
+    for (int c = 0; c < SCENE_CLASSES; c++) {
+        const uint64_t m = __ballot(lg == c);
+        if (m && (threadIdx.x & 63) == 0)
+            atomicAdd(counters + RB_CNT_SCENES + c, (int)__popcll(m));
+    }
 }
 }  // namespace
 
 hipError_t launch_tile_order(const DeviceWorld &d, const StepParams &p, hipStream_t s,
                              const SortWork &sw) {
     if (p.tile_mode != 1) return hipSuccess;
+    // scenes share a workgroup only while every CU still gets one (a lone
+    // scene is fastest with a CU to itself); a tuned block of 512 threads
+    // gives every scene twice the threads
+    int max_class = 0;
+    while (max_class < SCENE_CLASSES - 1 && p.n_tiles >> (max_class + 1) >= rb_num_cus()) max_class++;
+    if (p.solve_block == 512 && max_class > 0) max_class--;
     RB_LAUNCH(k_tile_order_keys, dim3((p.n_tiles + 255) / 256), dim3(256), 0, s, p.n_tiles,
-              d.tile_hdr, d.tile_order);
+              max_class, d.tile_hdr, d.tile_order, d.counters);
     hipError_t e = rb_launch_status();
     if (e != hipSuccess) return e;
-    // (the order is a schedule only: every scene is solved by its own
-    // workgroup, so results do not depend on it)
+    // (the order is a schedule only: every scene is solved by itself, so
+    // results do not depend on it)
     return launch_radix_sort(d.tile_order, p.n_tiles, 16, 8, sw, s);
 }
 
@@ -1319,20 +1477,18 @@ hipError_t launch_solve(const DeviceWorld &d, const StepParams &p, hipStream_t s
         if (end) nl++;
     };
     // (the step's first kernel has cleared the converged flag and the residuals)
-    // scene tiles: one workgroup per scene, 256 or 512 threads
-#define RB_SOLVE_ARGS                                                                         \
-    d.tile_hdr, d.tile_color_off, d.tile_bodies, d.pk, d.linvel, d.angvel, d.residual,        \
-        d.counters, d.tile_stats, d.tile_order
+#define RB_SOLVE_ARGS \
+    d.tile_hdr, d.tile_color_off, d.tile_bodies, d.pk, d.linvel, d.angvel, d.residual
     if (p.tile_mode == 1) {
-        // independent scenes: every sweep of a scene in one workgroup, one
-        // launch; with a tolerance each scene stops on its own residual
+        // independent scenes: every sweep of a scene in one workgroup; with a
+        // tolerance each scene stops on its own residual
         mark(0);
-        if (p.solve_block == 256)
-            RB_LAUNCH(k_tile_solve<256>, dim3(p.n_tiles), dim3(256), 0, s, p, 0, 0,
-                               p.normal_iters, p.friction_iters, warm, RB_SOLVE_ARGS);
-        else
-            RB_LAUNCH(k_tile_solve<TB_SCENE>, dim3(p.n_tiles), dim3(TB_SCENE), 0, s, p,
-                               0, 0, p.normal_iters, p.friction_iters, warm, RB_SOLVE_ARGS);
+        const SolveView sv{d.cs, d.solve_order, d.pos, d.inv_mass, d.inv_inertia_world, d.linvel,
+                           d.angvel};
+        // (a workgroup per scene at most: those beyond the classes' end at once)
+        RB_LAUNCH(k_scene_solve, dim3(p.n_tiles), dim3(SCENE_TB), 0, s, p, warm, d.tile_hdr,
+                  d.tile_color_off, d.tile_bodies, d.pk, sv, d.residual, d.tile_stats,
+                  d.tile_order, d.counters);
         mark(1);
         if (p.tol > 0.f)
             RB_LAUNCH(k_tile_summary, dim3(1), dim3(256), 0, s, p.n_tiles, d.tile_stats,
@@ -1342,26 +1498,18 @@ hipError_t launch_solve(const DeviceWorld &d, const StepParams &p, hipStream_t s
                                p.friction_iters, d.counters);
     } else {
         for (int sw = warm ? -1 : 0; sw < S; sw++) {
-            int fr = sw >= p.normal_iters;
+            const bool fr = sw >= p.normal_iters, res = sw >= 0 && sweep_residual_needed(p, sw);
             for (int ph = 0; ph < 4; ph++) {
                 int nx = (p.tiles_x - (ph & 1) + 1) / 2, nz = (p.tiles_z - (ph >> 1) + 1) / 2;
                 if (nx <= 0 || nz <= 0) continue;
                 mark(0);
-                if (sw < 0)
-                    RB_LAUNCH(k_tile_solve<TB>, dim3(nx * nz), dim3(TB), 0, s, p, ph, 0, 0, 0,
-                                       1, RB_SOLVE_ARGS);
-                else if (!fr && sweep_residual_needed(p, sw))
-                    RB_LAUNCH((k_tile_solve<TB, true>), dim3(nx * nz), dim3(TB), 0, s, p,
-                                       ph, sw, 1, 0, 0, RB_SOLVE_ARGS);
-                else if (!fr)
-                    RB_LAUNCH((k_tile_solve<TB, true, false>), dim3(nx * nz), dim3(TB), 0, s, p,
-                              ph, sw, 1, 0, 0, RB_SOLVE_ARGS);
-                else if (sweep_residual_needed(p, sw))
-                    RB_LAUNCH(k_tile_solve<TB>, dim3(nx * nz), dim3(TB), 0, s, p, ph, sw,
-                                       0, 1, 0, RB_SOLVE_ARGS);
-                else
-                    RB_LAUNCH((k_tile_solve<TB, false, false>), dim3(nx * nz), dim3(TB), 0, s,
-                              p, ph, sw, 0, 1, 0, RB_SOLVE_ARGS);
+                auto kern = sw < 0 ? k_tile_solve<TB, ROW_WARM, false>
+                            : !fr  ? (res ? k_tile_solve<TB, ROW_NORMAL, true>
+                                          : k_tile_solve<TB, ROW_NORMAL, false>)
+                                   : (res ? k_tile_solve<TB, ROW_FRICTION, true>
+                                          : k_tile_solve<TB, ROW_FRICTION, false>);
+                RB_LAUNCH(kern, dim3(nx * nz), dim3(TB), 0, s, p, ph, sw, RB_SOLVE_ARGS,
+                          d.counters);
                 mark(1);
             }
             if (sw >= 0 && p.tol > 0.f) {

@@ -101,16 +101,16 @@ struct ConstraintSoA {
 
 // Device state of one world.
 // A tile's rows in solve order, packed for the solve launches (position i).
+// Side 0 is body A, side 1 body B; lane 2 * side + (0 linear, 1 angular) of
+// the four lanes that run a row.
 struct PackedRows {
-    float4 *lin0, *p /* 4 per row */, *cen, *jac, *b, *lam, *fric;
-    float4 *IA, *IB;  // 3 rows each: world inverse inertia of body A, B
-    float4 *pA, *pB;
-    int4 *meta;       // body A, body B, their LDS slots (-1 static, -2 global)
-    float2 *im;       // inverse masses
-    // the velocity-independent terms of the normal rows, 4 per row (one per
-    // point): angular Jacobians a0, a1 and their images under the inverse
-    // inertias; 2 per row: the linear impulse directions scaled by 1/m
-    float4 *na0, *na1, *nia0, *nia1, *nl;
+    float4 *lin0, *jac, *b, *lam, *fric;
+    int2 *meta;        // per side: the body, its LDS slot | the row's colour << 16
+    // normal rows, 10 per row at 2 * e + side: Jacobians nj and velocity
+    // changes per impulse nm, e = 0 linear, e = 1 + q angular of point q
+    float4 *nj, *nm;
+    // friction rows, 8 per row at 4 * tangent + lane: the same of the tangents
+    float4 *fj, *fm;
 };
 
 struct DeviceWorld {
@@ -207,7 +207,8 @@ enum {
     RB_CNT_FACE_WORK = 16,    // uint32 pairs the quick face test left for the face pass
     RB_CNT_CLIP_SPLIT = 17,   // first small-hull candidate in the clip order
     RB_CNT_FACE_SMALL = 18,   // uint32 small-hull pairs of the face pass (after FACE_WORK's)
-    RB_CNT_COUNT = 19
+    RB_CNT_SCENES = 19,       // scene tiles: scenes of each solver class (5)
+    RB_CNT_COUNT = 24
 };
 
 // Step parameters passed by value to kernels.
@@ -243,7 +244,7 @@ struct StepParams {
     float tol;
     int warm_start;
     // launch shapes (mi_rb_tuning)
-    int solve_block;     // threads per scene-tile solve workgroup: 256 or 512
+    int solve_block;     // 256, or 512: twice the threads per scene in a shared workgroup
     int narrow_waves;    // narrowphase waves per SIMD (grid = CUs * 4 * narrow_waves)
     int has_vertexless;  // some shape is a sphere, a plane or a compound
     int n_proxies;       // compound children bodies (after the n bodies)

@@ -375,23 +375,15 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.tile_ncolors, p.n_tiles));
     RB_CHECK(w.alloc(&d.tile_stats, p.n_tiles));
     RB_CHECK(w.alloc(&d.pk.lin0, maxC));
-    RB_CHECK(w.alloc(&d.pk.na0, 4 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.na1, 4 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.nia0, 4 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.nia1, 4 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.nl, 2 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.p, 4 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.cen, maxC));
     RB_CHECK(w.alloc(&d.pk.jac, maxC));
     RB_CHECK(w.alloc(&d.pk.b, maxC));
     RB_CHECK(w.alloc(&d.pk.lam, maxC));
     RB_CHECK(w.alloc(&d.pk.fric, maxC));
-    RB_CHECK(w.alloc(&d.pk.IA, 3 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.IB, 3 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.pA, maxC));
-    RB_CHECK(w.alloc(&d.pk.pB, maxC));
-    RB_CHECK(w.alloc(&d.pk.meta, maxC));
-    RB_CHECK(w.alloc(&d.pk.im, maxC));
+    RB_CHECK(w.alloc(&d.pk.meta, 2 * (size_t)maxC));
+    RB_CHECK(w.alloc(&d.pk.nj, 10 * (size_t)maxC));
+    RB_CHECK(w.alloc(&d.pk.nm, 10 * (size_t)maxC));
+    RB_CHECK(w.alloc(&d.pk.fj, 8 * (size_t)maxC));
+    RB_CHECK(w.alloc(&d.pk.fm, 8 * (size_t)maxC));
     RB_CHECK(w.alloc(&d.solve_pos, maxC));
     RB_CHECK(w.alloc(&d.tile_bodies, 2 * (size_t)maxC));
     RB_CHECK(w.alloc(&d.tile_nb, p.n_tiles));

@@ -415,7 +415,8 @@ mi_rb_status mi_rb_set_solve_timing(void *world, int enable);
  * its work-group sizes in the host code).  0 = default.  Changing them drops
  * the captured graph; results do not depend on them. */
 typedef struct mi_rb_tuning {
-    int solve_block;     /* threads per scene-tile solver workgroup: 256 or 512 */
+    int solve_block;     /* batched scenes: 256, or 512 for twice the threads per scene where
+                          * scenes share a solver workgroup */
     int narrow_waves;    /* narrowphase waves per SIMD: 1..8 */
     int sort_tile;       /* body-key sort, keys per tile: 1024 or 4096; 0 = by key count */
     int sort_digit_bits; /* body-key sort, bits per radix digit: 4, 6, 7 or 8; 0 = 8 */

@@ -372,11 +372,15 @@ hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float i
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,
                               uint32_t *scan_status, hipStream_t s, hipEvent_t *ev,
                               uint32_t *lane_hits);
+// the sweep-and-prune API.  rec, rec_n: where the count pass leaves the pairs
+// of each 32 sorted AABBs for the write pass, RB_SAP_REC pairs and one count
+#define RB_SAP_REC 512
 hipError_t launch_sap_pairs(const float4 *mn, const float4 *mx, const int *is_large, int n,
                             int axis, uint2 *kv, float4 *smn, float4 *smx, uint32_t *counts,
                             uint32_t *offsets, uint32_t *cursor, uint32_t *big, uint32_t *lg,
                             uint32_t *total, uint32_t *ys, int max_pairs, int2 *pairs,
                             int *num_pairs, int *overflow, const SortWork &sw,
-                            uint32_t *scan_status, hipStream_t s, hipEvent_t *ev);
+                            uint32_t *scan_status, hipStream_t s, hipEvent_t *ev, uint2 *rec,
+                            uint32_t *rec_n);
 
 int rb_num_cus();

@@ -1822,14 +1822,15 @@ struct Sap {
     uint2 *kv = nullptr;
     float4 *smn = nullptr, *smx = nullptr;
     uint32_t *ys = nullptr, *counts = nullptr, *offsets = nullptr, *cursor = nullptr,
-             *big = nullptr, *lg = nullptr, *total = nullptr;
+             *big = nullptr, *lg = nullptr, *total = nullptr, *rec_n = nullptr;
+    uint2 *rec = nullptr;
     int *overflow = nullptr;
     SortWork sw{};
     uint32_t *scan_status = nullptr;
     hipEvent_t ev[5] = {};
     void release() {
         void *ps[] = {kv, smn, smx, ys, counts, offsets, cursor, big, lg, total, overflow, sw.tmp,
-                      sw.hist, sw.status, sw.tile_ctr, scan_status};
+                      sw.hist, sw.status, sw.tile_ctr, scan_status, rec, rec_n};
         for (void *p : ps) if (p) hipFree(p);
         for (auto &e : ev) if (e) hipEventDestroy(e);
     }
@@ -1853,7 +1854,9 @@ extern "C" mi_rb_status mi_rb_sap_create(const mi_rb_sap_desc *desc, int max_aab
               dalloc(&g->sw.tmp, n) == hipSuccess && dalloc(&g->sw.hist, 8 * 256) == hipSuccess &&
               dalloc(&g->sw.status, sort_status_words(n, 8)) == hipSuccess &&
               dalloc(&g->sw.tile_ctr, 16) == hipSuccess &&
-              dalloc(&g->scan_status, rb_scan_status_words(n)) == hipSuccess;
+              dalloc(&g->scan_status, rb_scan_status_words(n)) == hipSuccess &&
+              dalloc(&g->rec, ((size_t)n + 31) / 32 * RB_SAP_REC) == hipSuccess &&
+              dalloc(&g->rec_n, ((size_t)n + 31) / 32) == hipSuccess;
     if (!ok) { g->release(); delete g; return MI_RB_DEVICE; }
     g->sw.max_n = n;
     g->sw.max_tiles = rb_sort_tiles(n);
@@ -1889,7 +1892,7 @@ extern "C" mi_rb_status mi_rb_sap_find_pairs(void *sap, const void *d_aabb_min,
                               g->smn, g->smx, g->counts, g->offsets, g->cursor, g->big, g->lg,
                               g->total, g->ys, g->desc.max_pairs, static_cast<int2 *>(d_pairs),
                               static_cast<int *>(d_num_pairs), g->overflow, g->sw,
-                              g->scan_status, s, g->ev));
+                              g->scan_status, s, g->ev, g->rec, g->rec_n));
     return MI_RB_OK;
 }
 

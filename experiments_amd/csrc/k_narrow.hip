@@ -1683,10 +1683,58 @@ __global__ __launch_bounds__(256) void k_clip_split(const uint32_t *__restrict__
 // Proxy body n + k is child proxy[k].y of body proxy[k].x: its world
 // transform is the body's times the child's (qtRotate(orn, childPos) + pos,
 // qtMul(orn, childOrn)).
-__global__ __launch_bounds__(256) void k_proxy_transforms(int P, int n, const int2 *__restrict__ proxy,
+// Blocks from proxy_blocks on: a wave per group of up to 64 consecutive
+// triangles of a mesh body (mesh_groups: first proxy, triangles, body), whose
+// world AABBs it leaves in tri_lo/tri_hi by proxy and their union in
+// grp_lo/grp_hi: sat.cl:985-1023 tests a triangle's mesh-frame AABB against
+// the other body's world AABB; here its vertices are taken to world space
+// first, which is the same test for a mesh body at the identity.
+struct MeshBounds {
+    const int4 *groups;
+    float4 *tri_lo, *tri_hi, *grp_lo, *grp_hi;
+    int n_groups;
+};
+__global__ __launch_bounds__(256) void k_proxy_transforms(int P, int n, int proxy_blocks,
+                                                          const int2 *__restrict__ proxy,
                                                           const ChildShape *__restrict__ children,
                                                           float4 *__restrict__ pos,
-                                                          float4 *__restrict__ quat) {
+                                                          float4 *__restrict__ quat,
+                                                          const HullInfo *__restrict__ hulls,
+                                                          const float4 *__restrict__ verts,
+                                                          MeshBounds mb) {
+    if ((int)blockIdx.x >= proxy_blocks) {
+        const int g = ((int)blockIdx.x - proxy_blocks) * 4 + (int)(threadIdx.x >> 6);
+        const int lane = threadIdx.x & 63;
+        if (g >= mb.n_groups) return;
+        const int4 gr = mb.groups[g];
+        float4 lo = mk4(1e30f, 1e30f, 1e30f, 0.f), hi = mk4(-1e30f, -1e30f, -1e30f, 0.f);
+        if (lane < gr.y) {
+            const int k = gr.x + lane;
+            const int v0 = hulls[children[proxy[k].y].shape].vertex_offset;
+            const float4 pm = pos[gr.z], qm = quat[gr.z];
+            for (int c = 0; c < 3; c++) {
+                const float4 v = add4(qt_rotate(qm, verts[v0 + c]), pm);
+                lo = mk4(fminf(lo.x, v.x), fminf(lo.y, v.y), fminf(lo.z, v.z), 0.f);
+                hi = mk4(fmaxf(hi.x, v.x), fmaxf(hi.y, v.y), fmaxf(hi.z, v.z), 0.f);
+            }
+            mb.tri_lo[k] = lo;
+            mb.tri_hi[k] = hi;
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            lo.x = fminf(lo.x, __shfl_xor(lo.x, o));
+            lo.y = fminf(lo.y, __shfl_xor(lo.y, o));
+            lo.z = fminf(lo.z, __shfl_xor(lo.z, o));
+            hi.x = fmaxf(hi.x, __shfl_xor(hi.x, o));
+            hi.y = fmaxf(hi.y, __shfl_xor(hi.y, o));
+            hi.z = fmaxf(hi.z, __shfl_xor(hi.z, o));
+        }
+        if (lane == 0) {
+            mb.grp_lo[g] = lo;
+            mb.grp_hi[g] = hi;
+        }
+        return;
+    }
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= P) return;
     const int2 pr = proxy[k];
@@ -1703,27 +1751,42 @@ __global__ __launch_bounds__(256) void k_proxy_transforms(int P, int n, const in
 __device__ __forceinline__ int compound_children(const HullInfo &h) {
     return shape_kind_of(h) == SHAPE_KIND_COMPOUND ? h.num_edges : 0;
 }
-// Triangle tri (a child hull of mesh body m at the identity) against body
-// b's world AABB: sat.cl:985-1023 tests the triangle's mesh-frame AABB
-// against b's world AABB; here its vertices are taken to world space first,
-// which is the same test for a mesh body at the identity.
-__device__ __forceinline__ bool mesh_tri_overlaps(const HullInfo &tri, const float4 *__restrict__ verts,
-                                                  float4 pm, float4 qm, float4 bmin, float4 bmax) {
-    float4 lo = mk4(1e30f, 1e30f, 1e30f, 0.f), hi = mk4(-1e30f, -1e30f, -1e30f, 0.f);
-    for (int k = 0; k < 3; k++) {
-        const float4 v = add4(qt_rotate(qm, verts[tri.vertex_offset + k]), pm);
-        lo = mk4(fminf(lo.x, v.x), fminf(lo.y, v.y), fminf(lo.z, v.z), 0.f);
-        hi = mk4(fmaxf(hi.x, v.x), fmaxf(hi.y, v.y), fmaxf(hi.z, v.z), 0.f);
-    }
+// What the triangle cull reads: the bodies' world AABBs from the broadphase,
+// the triangles' and their groups', and each mesh body's first proxy and group.
+struct MeshView {
+    const float4 *aabb_min, *aabb_max, *tri_lo, *tri_hi, *grp_lo, *grp_hi;
+    const int *proxy_first, *group_first;
+};
+__device__ __forceinline__ bool mesh_box_overlaps(float4 lo, float4 hi, float4 bmin, float4 bmax) {
     return !(lo.x > bmax.x || hi.x < bmin.x || lo.z > bmax.z || hi.z < bmin.z || lo.y > bmax.y ||
              hi.y < bmin.y);
 }
-// What the triangle cull reads: transforms, the bodies' world AABBs from
-// the broadphase, hull vertices and the child table.
-struct MeshView {
-    const float4 *pos, *quat, *aabb_min, *aabb_max, *verts;
-    const ChildShape *children;
-};
+// The triangles of mesh body m (T of them) whose world AABB overlaps body b's,
+// 64 at a time in triangle order: f(t, mask) with the wave's first triangle t
+// and the lanes that overlap, until it returns false.  A wave tests 64 groups
+// of triangles at once and only looks into those whose union overlaps (every
+// triangle of a 20,000-triangle mesh against each of 4,096 cubes, from its
+// vertices: 416 us to count and 326 to write, against 7.6 and 7.9).
+template <class F>
+__device__ __forceinline__ void mesh_overlaps(const MeshView &mv, int m, int b, int T, F f) {
+    const int lane = threadIdx.x & 63;
+    const float4 bmin = mv.aabb_min[b], bmax = mv.aabb_max[b];
+    const int g0 = mv.group_first[m], k0 = mv.proxy_first[m], G = (T + 63) >> 6;
+    for (int gb = 0; gb < G; gb += 64) {
+        const int g = gb + lane;
+        uint64_t open = __ballot(g < G && mesh_box_overlaps(mv.grp_lo[g0 + (g < G ? g : 0)],
+                                                            mv.grp_hi[g0 + (g < G ? g : 0)], bmin,
+                                                            bmax));
+        while (open) {
+            const int t0 = 64 * (gb + __ffsll((unsigned long long)open) - 1);
+            open &= open - 1;
+            const int t = t0 + lane;
+            const int k = k0 + (t < T ? t : 0);
+            const bool ov = t < T && mesh_box_overlaps(mv.tri_lo[k], mv.tri_hi[k], bmin, bmax);
+            if (!f(t0, __ballot(ov))) return;
+        }
+    }
+}
 // A mesh pairs with convex hull bodies only: 0 when A is the mesh, 1 when B
 // is, 2 for a mesh with anything else (no child pairs), -1 without a mesh.
 __device__ __forceinline__ int mesh_side(const HullInfo &ha, const HullInfo &hb) {
@@ -1764,15 +1827,10 @@ __global__ __launch_bounds__(256) void k_compound_count(int max_pairs, const int
             if (side < 2 && !both_static) {
                 const int m = side == 0 ? pr.x : pr.y, b = side == 0 ? pr.y : pr.x;
                 const HullInfo &hm = side == 0 ? ha : hb;
-                const float4 pm = mv.pos[m], qm = mv.quat[m], bmin = mv.aabb_min[b],
-                             bmax = mv.aabb_max[b];
-                for (int t0 = 0; t0 < hm.num_edges; t0 += 64) {
-                    const int t = t0 + lane;
-                    const bool ov = t < hm.num_edges &&
-                                    mesh_tri_overlaps(hulls[mv.children[hm.edge_offset + t].shape],
-                                                      mv.verts, pm, qm, bmin, bmax);
-                    c += (uint32_t)__popcll(__ballot(ov));
-                }
+                mesh_overlaps(mv, m, b, hm.num_edges, [&](int, uint64_t mask) {
+                    c += (uint32_t)__popcll(mask);
+                    return true;
+                });
             }
         } else {
             const int ca = compound_children(ha);
@@ -1806,19 +1864,15 @@ __global__ __launch_bounds__(256) void k_compound_write(int max_pairs, const int
         if (side >= 0) {  // overlapping triangles in triangle order (c > 0: side is 0 or 1)
             const int m = side == 0 ? pr.x : pr.y, b = side == 0 ? pr.y : pr.x;
             const HullInfo &hm = side == 0 ? ha : hb;
-            const float4 pm = mv.pos[m], qm = mv.quat[m], bmin = mv.aabb_min[b], bmax = mv.aabb_max[b];
             uint32_t k0 = 0;
-            for (int t0 = 0; t0 < hm.num_edges && k0 < c; t0 += 64) {
+            mesh_overlaps(mv, m, b, hm.num_edges, [&](int t0, uint64_t mask) {
                 const int t = t0 + lane;
-                const bool ov = t < hm.num_edges &&
-                                mesh_tri_overlaps(hulls[mv.children[hm.edge_offset + t].shape], mv.verts,
-                                                  pm, qm, bmin, bmax);
-                const unsigned long long mask = __ballot(ov);
                 const uint32_t k = k0 + (uint32_t)__popcll(mask & lanes_below(lane));
-                if (ov && k < c && base + k < max_pairs)
+                if (((mask >> lane) & 1ull) && k < c && base + k < max_pairs)
                     pairs[base + k] = side == 0 ? make_int2(n + fa + t, pr.y) : make_int2(pr.x, n + fb + t);
                 k0 += (uint32_t)__popcll(mask);
-            }
+                return k0 < c;
+            });
             continue;
         }
         const int cb = compound_children(hb);
@@ -1909,10 +1963,14 @@ hipError_t launch_narrowphase(const DeviceWorld &d, const StepParams &p, hipStre
 
 hipError_t launch_compound_pairs(const DeviceWorld &d, const StepParams &p, hipStream_t s,
                                  uint32_t *scan_status, size_t scan_stride) {
-    RB_LAUNCH(k_proxy_transforms, dim3((p.n_proxies + 255) / 256), dim3(256), 0, s,
-                       p.n_proxies, p.n_bodies, d.proxy, d.children, d.pos, d.quat);
+    const int proxy_blocks = (p.n_proxies + 255) / 256;
+    const MeshBounds mb{d.mesh_groups, d.tri_lo, d.tri_hi, d.grp_lo, d.grp_hi, p.n_mesh_groups};
+    RB_LAUNCH(k_proxy_transforms, dim3(proxy_blocks + (p.n_mesh_groups + 3) / 4), dim3(256), 0, s,
+              p.n_proxies, p.n_bodies, proxy_blocks, d.proxy, d.children, d.pos, d.quat, d.hulls,
+              d.verts, mb);
     const int grid = rb_num_cus() * 4;
-    const MeshView mv{d.pos, d.quat, d.aabb_min, d.aabb_max, d.verts, d.children};
+    const MeshView mv{d.aabb_min, d.aabb_max, d.tri_lo, d.tri_hi, d.grp_lo, d.grp_hi,
+                      d.proxy_first, d.mesh_group_first};
     RB_LAUNCH(k_compound_count, dim3(grid), dim3(256), 0, s, p.max_pairs,
                        d.counters + RB_CNT_PAIRS, d.pairs, d.shape, d.inv_mass, d.hulls, mv,
                        d.narrow_cand, d.counters + RB_CNT_OVERFLOW);

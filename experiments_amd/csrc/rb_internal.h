@@ -128,6 +128,10 @@ struct DeviceWorld {
     int2 *proxy;          // per proxy: (parent body, child index)
     int *proxy_first;     // per body: its first proxy (-1: not a compound)
     int *owner;           // per body and proxy: the body a contact names
+    // mesh bodies' triangles in groups of up to 64 consecutive proxies
+    int4 *mesh_groups;    // first proxy, triangles, body
+    int *mesh_group_first;// per body: its first group (-1: not a mesh)
+    float4 *tri_lo, *tri_hi, *grp_lo, *grp_hi;  // world AABBs by proxy and by group, each step
     float4 *inv_inertia_local;   // diagonal
     float4 *inv_inertia_world;   // 3 rows per body
     int *scene_start, *scene_count;
@@ -248,6 +252,7 @@ struct StepParams {
     int narrow_waves;    // narrowphase waves per SIMD (grid = CUs * 4 * narrow_waves)
     int has_vertexless;  // some shape is a sphere, a plane or a compound
     int n_proxies;       // compound children bodies (after the n bodies)
+    int n_mesh_groups;   // groups of mesh triangles among them
 };
 
 // ---- checked kernel launches ----

@@ -318,6 +318,18 @@ mi_rb_status derive_and_upload(World &w) {
     }
     const int P = (int)proxies.size();
     p.n_proxies = P;
+    // a mesh body's triangles in groups of 64, whose bounds a step culls first
+    std::vector<int> group_first(n, -1);
+    std::vector<int4> groups;
+    for (int i = 0; i < n; i++) {
+        const HullInfo &h = w.hulls[w.shape[i]];
+        if (!compound_is_mesh(h)) continue;
+        group_first[i] = (int)groups.size();
+        for (int t = 0; t < h.num_edges; t += 64)
+            groups.push_back(make_int4(proxy_first[i] + t, std::min(64, h.num_edges - t), i, 0));
+    }
+    p.n_mesh_groups = (int)groups.size();
+    const size_t tris = groups.empty() ? 1 : (size_t)P;
     for (int i = 0; i < n; i++) owner.push_back(i);
     for (const int2 &pr : proxies) owner.push_back(pr.x);
     RB_CHECK(w.alloc(&d.pos, (size_t)n + P));
@@ -330,6 +342,12 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.proxy_first, n));
     RB_CHECK(w.alloc(&d.proxy, std::max(P, 1)));
     RB_CHECK(w.alloc(&d.children, std::max((int)w.children.size(), 1)));
+    RB_CHECK(w.alloc(&d.mesh_groups, groups.size()));
+    RB_CHECK(w.alloc(&d.mesh_group_first, n));
+    RB_CHECK(w.alloc(&d.tri_lo, tris));
+    RB_CHECK(w.alloc(&d.tri_hi, tris));
+    RB_CHECK(w.alloc(&d.grp_lo, groups.size()));
+    RB_CHECK(w.alloc(&d.grp_hi, groups.size()));
     RB_CHECK(w.alloc(&d.scene, n));
     RB_CHECK(w.alloc(&d.is_large, n));
     RB_CHECK(w.alloc(&d.inv_inertia_local, n));
@@ -465,6 +483,9 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(up(d.shape, w.shape.data(), sizeof(int) * n));
     RB_CHECK(up(d.owner, owner.data(), sizeof(int) * owner.size()));
     RB_CHECK(up(d.proxy_first, proxy_first.data(), sizeof(int) * n));
+    RB_CHECK(up(d.mesh_group_first, group_first.data(), sizeof(int) * n));
+    if (!groups.empty())
+        RB_CHECK(up(d.mesh_groups, groups.data(), sizeof(int4) * groups.size()));
     if (P > 0) {
         std::vector<float> pim(P);
         std::vector<int> psh(P);

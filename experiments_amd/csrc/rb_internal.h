@@ -175,7 +175,8 @@ struct DeviceWorld {
     uint32_t *cand_off;          // its exclusive scan
     int4 *face_best;             // per pair: face minimum (depth bits, axis), edge-axis count
     uint2 *cand_kv;              // (cost key, pair) of the candidates, sorted
-    float *residual;             // per sweep: max scaled dlambda, max lambda (as uint bits)
+    uint2 *tile_res;             // per tile, of the normal then of the friction sweeps: the last
+                                 // residual terms, max scaled dlambda and max lambda (float bits)
     // warm start
     int2 *prev_keys;             // previous step's contacts keyed by their pair entry (x, y), sorted
     int2 *stage_keys;            // worlds with compound children: the cache before it is sorted

@@ -57,16 +57,13 @@ int ilog2(uint64_t v) {
     return b;
 }
 
-// Start of a step: the counters (the overflow bits are sticky), the
-// solver's per-sweep residual maxima, the scans' status words and the sorts'
-// digit and tile counters, and the solver tiles' row ranges.
-__global__ void k_zero_counters(int *c, float *residual, int n_residual, uint32_t *scan_status,
-                                int n_scan_words, int *tile_first, int *tile_cnt, int n_tiles) {
+// Start of a step: the counters (the overflow bits are sticky), the scans'
+// status words and the sorts' digit and tile counters, and the solver tiles'
+// row ranges.
+__global__ void k_zero_counters(int *c, uint32_t *scan_status, int n_scan_words, int *tile_first,
+                                int *tile_cnt, int n_tiles) {
     const int i = threadIdx.x;
-    if (blockIdx.x == 0) {
-        if (i < RB_CNT_COUNT && i != RB_CNT_OVERFLOW) c[i] = 0;
-        for (int k = i; k < n_residual; k += blockDim.x) residual[k] = 0.f;
-    }
+    if (blockIdx.x == 0 && i < RB_CNT_COUNT && i != RB_CNT_OVERFLOW) c[i] = 0;
     // the status words of the step's scans (one region per scan), then the
     // step's sort heads
     for (int k = blockIdx.x * blockDim.x + i; k < n_scan_words; k += gridDim.x * blockDim.x)
@@ -411,7 +408,7 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.cand_off, maxP));
     RB_CHECK(w.alloc(&d.face_best, maxP));
     RB_CHECK(w.alloc(&d.cand_kv, maxP));
-    RB_CHECK(w.alloc(&d.residual, 4 * RB_MAX_SWEEPS + 2));  // 2 floats per sweep of both phases
+    RB_CHECK(w.alloc(&d.tile_res, 2 * (size_t)p.n_tiles));
     RB_CHECK(w.alloc(&d.counters, RB_CNT_COUNT));
     RB_CHECK(w.alloc(&d.prev_keys, maxC));
     RB_CHECK(w.alloc(&d.prev_imp, maxC));
@@ -529,8 +526,7 @@ mi_rb_status enqueue_step(World &w, int last_stage) {
     (void)hipGetLastError();  // start from a clean error state: launches below are checked one by one
     w.events_full = ev && last_stage >= MI_RB_STAGE_INTEGRATE;
     if (ev) RB_CHECK(hipEventRecord(w.ev[0], s));
-    RB_LAUNCH(k_zero_counters, dim3(16), dim3(256), 0, s, d.counters, d.residual,
-                       2 * (p.normal_iters + p.friction_iters + 1), w.scan_status,
+    RB_LAUNCH(k_zero_counters, dim3(16), dim3(256), 0, s, d.counters, w.scan_status,
                        (int)(RB_SCAN_REGIONS * w.scan_stride + RB_STEP_SORTS * RB_SORT_HEAD_WORDS),
                        d.tile_first, d.tile_cnt,
                        p.n_tiles);

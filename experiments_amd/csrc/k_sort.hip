@@ -123,11 +123,14 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_onesweep(const uint2 *__restrict
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
+    // as many workgroups as there are tiles take one each; the others of a
+    // capacity-sized launch leave the counter alone (600k keys in a launch sized
+    // for 8M: 23.8 -> 16.1 us)
+    if ((int64_t)blockIdx.x * TILE >= n) return;
     if (tid == 0) s_tile = atomicAdd(tile_ctr, 1u);
     for (int i = tid; i < WAVES * RADIX; i += SORT_BLOCK) (&s_wave_hist[0][0])[i] = 0;
     __syncthreads();
     const int tile = (int)s_tile;
-    if (tile * TILE >= n) return;  // beyond the device-side count: nothing looks back here
     const int base = tile * TILE + wave * (ITEMS * 64);
     const uint32_t dmask = (1u << bits) - 1u;
 
@@ -253,6 +256,11 @@ constexpr uint64_t SFLAG_AGG = 1ull << 62;
 constexpr uint64_t SFLAG_INC = 2ull << 62;
 constexpr uint64_t SVAL_MASK = (1ull << 62) - 1ull;
 
+// VEC: in and out are 16-byte aligned: whole tiles move 16 bytes a lane, each
+// wave a contiguous piece per load.  3.4M flags (13.6 MB in, as much out in one
+// scan of five) in a launch sized for 8M: 43.8 -> 18.3 us against a lane reading
+// 16 consecutive words and every workgroup of the launch counting itself in.
+template <bool VEC>
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_t *out, int n,
                                                      uint32_t *total, uint64_t *status,
                                                      uint32_t *tile_ctr, const int *n_dev,
@@ -260,36 +268,51 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
                                                      uint32_t *idx_out,
                                                      const uint32_t *idx_base) {
     if (n_dev && *n_dev < n) n = *n_dev;
-    __shared__ uint32_t s_wave[SCAN_BLOCK / 64];
+    constexpr int ROUNDS = SCAN_ITEMS / 4, NWAVES = SCAN_BLOCK / 64;
+    __shared__ uint32_t s_wave[ROUNDS * NWAVES];
     __shared__ uint32_t s_tile;
     __shared__ uint64_t s_prefix;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (n <= 0) {
+        if (total && blockIdx.x == 0 && tid == 0) *total = 0;
+        return;
+    }
+    // as many workgroups as there are tiles take one each; the others of a
+    // capacity-sized launch leave the counter alone
+    if ((int64_t)blockIdx.x * SCAN_TILE >= n) return;
     if (tid == 0) s_tile = atomicAdd(tile_ctr, 1u);
     __syncthreads();
     const int tile = (int)s_tile;
-    if (n <= 0) {
-        if (total && tile == 0 && tid == 0) *total = 0;
-        return;
-    }
-    if (tile * SCAN_TILE >= n) return;
-    const int base = tile * SCAN_TILE + tid * SCAN_ITEMS;  // blocked arrangement
-    uint32_t v[SCAN_ITEMS];
-    uint32_t sum = 0;
+    // round r: elements tile * SCAN_TILE + r * 1024 + 4 * tid .. + 3
+    const int base = tile * SCAN_TILE + 4 * tid;
+    const bool whole = n - tile * SCAN_TILE >= SCAN_TILE;
+    uint32_t v[ROUNDS][4], sum[ROUNDS], incl[ROUNDS];
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        int i = base + k;
-        v[k] = i < n ? in[i] : 0u;
-        sum += v[k];
+    for (int r = 0; r < ROUNDS; r++) {
+        const int i = base + r * 4 * SCAN_BLOCK;
+        if (VEC && whole) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(in + i);
+            v[r][0] = q.x; v[r][1] = q.y; v[r][2] = q.z; v[r][3] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[r][k] = i + k < n ? in[i + k] : 0u;
+        }
     }
-    uint32_t incl = wave_incl_scan(sum);
-    if (lane == 63) s_wave[wave] = incl;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        sum[r] = ((v[r][0] + v[r][1]) + v[r][2]) + v[r][3];
+        incl[r] = wave_incl_scan(sum[r]);
+        if (lane == 63) s_wave[r * NWAVES + wave] = incl[r];
+    }
     __syncthreads();
-    uint32_t wave_off = 0, tile_sum = 0;
-    for (int w = 0; w < SCAN_BLOCK / 64; w++) {
-        uint32_t c = s_wave[w];
-        if (w < wave) wave_off += c;
-        tile_sum += c;
-    }
+    uint32_t off[ROUNDS], tile_sum = 0;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+#pragma unroll
+        for (int w = 0; w < NWAVES; w++) {
+            if (w == wave) off[r] = tile_sum;
+            tile_sum += s_wave[r * NWAVES + w];
+        }
     if (wave == 0) {
         uint64_t *st = status + tile;
         if (tile == 0) {
@@ -337,17 +360,31 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
         }
     }
     __syncthreads();
-    uint32_t run = (uint32_t)s_prefix + wave_off + (incl - sum);
+    const uint32_t prefix = (uint32_t)s_prefix;
     const uint32_t ibase = idx_out && idx_base ? *idx_base : 0u;
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        int i = base + k;
-        if (out && i < n) out[i] = run;
-        if (idx_out && v[k]) idx_out[ibase + run] = (uint32_t)i;  // flags: the set indices, in order
-        run += v[k];
+    for (int r = 0; r < ROUNDS; r++) {
+        const int i = base + r * 4 * SCAN_BLOCK;
+        uint32_t run = prefix + off[r] + (incl[r] - sum[r]);
+        uint32_t o[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            o[k] = run;
+            if (idx_out && v[r][k]) idx_out[ibase + run] = (uint32_t)(i + k);  // flags: the set indices, in order
+            run += v[r][k];
+        }
+        if (out) {
+            if (VEC && whole) {
+                *reinterpret_cast<uint4 *>(out + i) = make_uint4(o[0], o[1], o[2], o[3]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (i + k < n) out[i + k] = o[k];
+            }
+        }
     }
-    int last_tile = (n - 1) / SCAN_TILE;
-    if (total && tile == last_tile && tid == SCAN_BLOCK - 1) *total = run;
+    const int last_tile = (n - 1) / SCAN_TILE;
+    if (total && tile == last_tile && tid == 0) *total = prefix + tile_sum;
 }
 
 __global__ void k_scan_empty(uint32_t *total) { if (total) *total = 0; }
@@ -485,7 +522,9 @@ hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, int n, uint3
     // word after the tile counter (cleared with the status words)
     uint32_t *e = err ? reinterpret_cast<uint32_t *>(err) : status + 1;
     const uint32_t bit = err ? (uint32_t)MI_RB_OVERFLOW_LOOKBACK : 1u;
-    RB_LAUNCH(k_scan, dim3(tiles), dim3(SCAN_BLOCK), 0, s, in, out, n, total, st, ctr,
+    const bool vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+    auto kern = vec ? k_scan<true> : k_scan<false>;
+    RB_LAUNCH(kern, dim3(tiles), dim3(SCAN_BLOCK), 0, s, in, out, n, total, st, ctr,
                        n_dev, e, bit, idx_out, idx_base);
     return rb_launch_status();
 }

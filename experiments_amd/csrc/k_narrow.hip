@@ -681,8 +681,7 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face(
 // group's LDS), so the separation and the lexicographic (overlap, axis)
 // minimum are the same.
 __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
-    int max_pairs, const uint32_t *__restrict__ n_large_ptr,
-    const uint32_t *__restrict__ n_small_ptr, const uint32_t *__restrict__ work,
+    int max_pairs, const uint32_t *__restrict__ n_small_ptr, const uint32_t *__restrict__ work,
     const int2 *__restrict__ pairs, const float4 *__restrict__ pos,
     const float4 *__restrict__ quat, const float *__restrict__ inv_mass,
     const int *__restrict__ shape, const HullInfo *__restrict__ hulls,
@@ -692,12 +691,9 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
     __shared__ float4 sVA[SG_GROUPS][SG_VERTS], sVB[SG_GROUPS][SG_VERTS];
     const int lane = threadIdx.x;
     const int grp = lane / SG, gl = lane & (SG - 1), gbase = grp * SG;
-    const uint32_t n_large = *n_large_ptr;
-    const uint32_t n_small = *n_small_ptr;
-    int first = (int)min(n_large, (uint32_t)max_pairs);
-    int end = (int)min(n_large + n_small, (uint32_t)max_pairs);
+    const int end = (int)min(*n_small_ptr, (uint32_t)max_pairs);
     const int W = (int)gridDim.x * SG_GROUPS;
-    for (int i = first + (int)blockIdx.x * SG_GROUPS + grp; i < end; i += W) {
+    for (int i = (int)blockIdx.x * SG_GROUPS + grp; i < end; i += W) {
         const int p = (int)work[i];
         const int2 pr = pairs[p];
         const HullInfo hA = hulls[shape[pr.x]];
@@ -750,21 +746,21 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
 }
 
 // Candidates in descending order of edge-edge axis count (stable), pairs of
-// small hulls (the SG-lane clip pass) after the others.
-__global__ __launch_bounds__(256) void k_narrow_keys(int max_pairs, const int *__restrict__ num_pairs_ptr,
-                                                     const uint32_t *__restrict__ cand,
-                                                     const uint32_t *__restrict__ cand_off,
+// small hulls (the SG-lane clip pass) after the others: the sort keys of the
+// listed candidates.
+__global__ __launch_bounds__(256) void k_narrow_keys(int max_pairs, const uint32_t *__restrict__ n_cand,
+                                                     const uint32_t *__restrict__ cand_list,
                                                      const int4 *__restrict__ face_best,
                                                      uint2 *__restrict__ kv) {
-    int npairs = *num_pairs_ptr;
-    if (npairs > max_pairs) npairs = max_pairs;
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npairs || !cand[p]) return;
+    const uint32_t n = min(*n_cand, (uint32_t)max_pairs);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t p = cand_list[i];
     // large pairs first, each class by descending edge-axis count (at most
     // 128 x 128 < 0x8000)
     const int4 fb = face_best[p];
     const uint32_t ne = (uint32_t)(fb.z < 0x7fff ? fb.z : 0x7fff);
-    kv[cand_off[p]] = make_uint2((fb.w ? 0x8000u : 0u) | (0x7fffu - ne), (uint32_t)p);
+    kv[i] = make_uint2((fb.w ? 0x8000u : 0u) | (0x7fffu - ne), p);
 }
 
 // Pass 2, the candidates: edge x edge axes (never reject), then clipping of
@@ -1901,44 +1897,37 @@ hipError_t launch_narrowphase(const DeviceWorld &d, const StepParams &p, hipStre
                               const SortWork &sw, uint32_t *scan_status, size_t scan_stride) {
     const int grid = rb_num_cus() * 4 * (p.narrow_waves > 0 ? p.narrow_waves : 4);
     // pass 1's pairs: the flags of pass 0 compacted into cand_kv, which
-    // k_narrow_keys fills only after pass 1
-    uint32_t *work = (uint32_t *)d.cand_kv;
+    // k_narrow_keys fills only after pass 1, the wave kernel's in its first
+    // half, the small-hull kernel's in its second
+    uint32_t *work = (uint32_t *)d.cand_kv, *work_small = work + p.max_pairs;
     uint32_t *n_work = (uint32_t *)(d.counters + RB_CNT_FACE_WORK);
+    uint32_t *n_small = (uint32_t *)(d.counters + RB_CNT_FACE_SMALL);
     RB_LAUNCH(k_narrow_quick<QUICK_LANES>,
               dim3(((long long)p.max_pairs * QUICK_LANES + 255) / 256), dim3(256), 0, s,
               p.max_pairs, d.counters + RB_CNT_PAIRS, d.pairs, d.pos, d.quat, d.inv_mass, d.shape,
               d.hulls, d.verts, d.planes, d.has_contact, d.narrow_cand);
-    // the wave kernel's pairs, then the small-hull kernel's after them
-    uint32_t *n_small = (uint32_t *)(d.counters + RB_CNT_FACE_SMALL);
-    hipError_t e0 = launch_compact_flags(d.has_contact, work, p.max_pairs, n_work,
-                                         scan_status + RB_SCAN_WORK * scan_stride, s,
-                                         d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW,
-                                         nullptr, true);
-    if (e0 != hipSuccess) return e0;
-    e0 = launch_compact_flags(d.narrow_cand, work, p.max_pairs, n_small,
-                              scan_status + RB_SCAN_SMALL * scan_stride, s,
-                              d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW, n_work, true);
+    hipError_t e0 = launch_compact2(d.has_contact, d.narrow_cand, p.max_pairs, work, work_small,
+                                    n_work, n_small, scan_status + RB_SCAN_WORK * scan_stride, s,
+                                    d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW);
     if (e0 != hipSuccess) return e0;
     RB_LAUNCH(k_narrow_face, dim3(grid), dim3(NP_BLOCK), 0, s, p.max_pairs, n_work, work,
                        d.pairs, d.pos, d.quat, d.inv_mass, d.shape,
                        d.hulls, d.verts, d.planes, d.has_contact, d.narrow_cand, d.face_best,
                        d.counters + RB_CNT_OVERFLOW);
-    RB_LAUNCH(k_narrow_face_small, dim3(grid), dim3(NP_BLOCK), 0, s, p.max_pairs, n_work, n_small,
-              work, d.pairs, d.pos, d.quat, d.inv_mass, d.shape, d.hulls, d.verts, d.planes,
+    RB_LAUNCH(k_narrow_face_small, dim3(grid), dim3(NP_BLOCK), 0, s, p.max_pairs, n_small,
+              work_small, d.pairs, d.pos, d.quat, d.inv_mass, d.shape, d.hulls, d.verts, d.planes,
               d.has_contact, d.narrow_cand, d.face_best);
     if (p.has_vertexless)
         RB_LAUNCH(k_narrow_special, dim3(rb_num_cus() * 4), dim3(256), 0, s, p.max_pairs,
                            d.counters + RB_CNT_PAIRS, d.pairs, d.pos, d.quat, d.inv_mass, d.shape,
                            d.hulls, d.planes, p.friction, d.contact_slots, d.has_contact);
-    hipError_t e = launch_exclusive_scan(d.narrow_cand, d.cand_off, p.max_pairs,
-                                         (uint32_t *)(d.counters + RB_CNT_NARROW_CAND),
-                                         scan_status + RB_SCAN_CAND * scan_stride, s,
-                                         d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW,
-                                         nullptr, nullptr, true);
+    uint32_t *n_cand = (uint32_t *)(d.counters + RB_CNT_NARROW_CAND);
+    hipError_t e = launch_compact_flags(d.narrow_cand, d.cand_off, p.max_pairs, n_cand,
+                                        scan_status + RB_SCAN_CAND * scan_stride, s,
+                                        d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW, true);
     if (e != hipSuccess) return e;
-    RB_LAUNCH(k_narrow_keys, dim3((p.max_pairs + 255) / 256), dim3(256), 0, s,
-                       p.max_pairs, d.counters + RB_CNT_PAIRS, d.narrow_cand, d.cand_off,
-                       d.face_best, d.cand_kv);
+    RB_LAUNCH(k_narrow_keys, dim3((p.max_pairs + 255) / 256), dim3(256), 0, s, p.max_pairs, n_cand,
+              d.cand_off, d.face_best, d.cand_kv);
     e = launch_radix_sort(d.cand_kv, p.max_pairs, 16, 8, sw, s, d.counters + RB_CNT_NARROW_CAND);
     if (e != hipSuccess) return e;
     // large-hull candidates [0, split) a wave each, then the small-hull ones
@@ -1978,7 +1967,7 @@ hipError_t launch_compound_pairs(const DeviceWorld &d, const StepParams &p, hipS
                                          (uint32_t *)(d.counters + RB_CNT_NARROW_CAND),
                                          scan_status + RB_SCAN_COMPOUND * scan_stride, s,
                                          d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW,
-                                         nullptr, nullptr, true);
+                                         nullptr, true);
     if (e != hipSuccess) return e;
     RB_LAUNCH(k_compound_write, dim3(grid), dim3(256), 0, s, p.max_pairs,
                        d.counters + RB_CNT_PAIRS, d.pairs, d.shape, d.hulls, mv, d.proxy_first,

@@ -256,6 +256,42 @@ constexpr uint64_t SFLAG_AGG = 1ull << 62;
 constexpr uint64_t SFLAG_INC = 2ull << 62;
 constexpr uint64_t SVAL_MASK = (1ull << 62) - 1ull;
 
+// One wave publishes a tile's sum and returns the sum of the tiles before it.
+__device__ __forceinline__ uint64_t scan_look_back(uint64_t *status, int tile, uint64_t tile_sum,
+                                                   int lane, uint32_t *err, uint32_t err_bit) {
+    if (lane == 0)
+        __hip_atomic_store(status + tile, SFLAG_AGG | tile_sum, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    // lane k reads the word of tile t - k: 64 predecessors per round trip,
+    // summed back to the nearest inclusive one; from an unpublished word on,
+    // the words are read again
+    uint64_t prefix = 0;
+    uint32_t spins = 0;
+    int t = tile - 1;
+    while (true) {
+        const int tt = t - lane;
+        const uint64_t w = tt >= 0 ? __hip_atomic_load(status + tt, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT)
+                                   : SFLAG_INC;  // (never reached: tile 0 is inclusive)
+        const uint64_t unpub = __ballot((w & ~SVAL_MASK) == 0);
+        const uint64_t inc = __ballot((w & SFLAG_INC) != 0);
+        const uint64_t stop = unpub | inc;
+        const int j = stop ? __ffsll((long long)stop) - 1 : 64;
+        const bool j_inc = j < 64 && ((inc >> j) & 1ull);
+        uint64_t mine = (lane < j || (lane == j && j_inc)) ? (w & SVAL_MASK) : 0ull;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) mine += __shfl_xor(mine, o, 64);
+        prefix += mine;
+        if (j_inc) break;
+        t -= j;
+        if (j < 64 && ++spins > (1u << 26)) {
+            if (lane == 0) atomicOr(err, err_bit);
+            break;
+        }
+    }
+    return prefix;
+}
+
 // VEC: in and out are 16-byte aligned: whole tiles move 16 bytes a lane, each
 // wave a contiguous piece per load.  3.4M flags (13.6 MB in, as much out in one
 // scan of five) in a launch sized for 8M: 43.8 -> 18.3 us against a lane reading
@@ -265,8 +301,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
                                                      uint32_t *total, uint64_t *status,
                                                      uint32_t *tile_ctr, const int *n_dev,
                                                      uint32_t *err, uint32_t err_bit,
-                                                     uint32_t *idx_out,
-                                                     const uint32_t *idx_base) {
+                                                     uint32_t *idx_out) {
     if (n_dev && *n_dev < n) n = *n_dev;
     constexpr int ROUNDS = SCAN_ITEMS / 4, NWAVES = SCAN_BLOCK / 64;
     __shared__ uint32_t s_wave[ROUNDS * NWAVES];
@@ -322,36 +357,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
                 s_prefix = 0;
             }
         } else {
-            if (lane == 0)
-                __hip_atomic_store(st, SFLAG_AGG | tile_sum, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            // lane k reads the word of tile t - k: 64 predecessors per round
-            // trip, summed back to the nearest inclusive one; from an
-            // unpublished word on, the words are read again
-            uint64_t prefix = 0;
-            uint32_t spins = 0;
-            int t = tile - 1;
-            while (true) {
-                const int tt = t - lane;
-                const uint64_t w = tt >= 0 ? __hip_atomic_load(status + tt, __ATOMIC_RELAXED,
-                                                               __HIP_MEMORY_SCOPE_AGENT)
-                                           : SFLAG_INC;  // (never reached: tile 0 is inclusive)
-                const uint64_t unpub = __ballot((w & ~SVAL_MASK) == 0);
-                const uint64_t inc = __ballot((w & SFLAG_INC) != 0);
-                const uint64_t stop = unpub | inc;
-                const int j = stop ? __ffsll((long long)stop) - 1 : 64;
-                const bool j_inc = j < 64 && ((inc >> j) & 1ull);
-                uint64_t mine = (lane < j || (lane == j && j_inc)) ? (w & SVAL_MASK) : 0ull;
-#pragma unroll
-                for (int o = 32; o >= 1; o >>= 1) mine += __shfl_xor(mine, o, 64);
-                prefix += mine;
-                if (j_inc) break;
-                t -= j;
-                if (j < 64 && ++spins > (1u << 26)) {
-                    if (lane == 0) atomicOr(err, err_bit);
-                    break;
-                }
-            }
+            const uint64_t prefix = scan_look_back(status, tile, tile_sum, lane, err, err_bit);
             if (lane == 0) {
                 __hip_atomic_store(st, SFLAG_INC | (prefix + tile_sum), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
@@ -361,7 +367,6 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
     }
     __syncthreads();
     const uint32_t prefix = (uint32_t)s_prefix;
-    const uint32_t ibase = idx_out && idx_base ? *idx_base : 0u;
 #pragma unroll
     for (int r = 0; r < ROUNDS; r++) {
         const int i = base + r * 4 * SCAN_BLOCK;
@@ -370,7 +375,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             o[k] = run;
-            if (idx_out && v[r][k]) idx_out[ibase + run] = (uint32_t)(i + k);  // flags: the set indices, in order
+            if (idx_out && v[r][k]) idx_out[run] = (uint32_t)(i + k);  // flags: the set indices, in order
             run += v[r][k];
         }
         if (out) {
@@ -385,6 +390,92 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t *in, uint32_
     }
     const int last_tile = (n - 1) / SCAN_TILE;
     if (total && tile == last_tile && tid == 0) *total = prefix + tile_sum;
+}
+
+// Compaction of two flag arrays in one pass over both: the indices of a's set
+// flags, in order, to list_a and their number to *n_a; b's likewise.  The
+// look-back words carry both counts, 31 bits each.  (3.4M pairs: 23 us against
+// two scans of 18.)
+__global__ __launch_bounds__(SCAN_BLOCK) void k_compact2(const uint32_t *__restrict__ a,
+                                                         const uint32_t *__restrict__ b, int n,
+                                                         uint32_t *__restrict__ list_a,
+                                                         uint32_t *__restrict__ list_b,
+                                                         uint32_t *n_a, uint32_t *n_b,
+                                                         uint64_t *status, uint32_t *tile_ctr,
+                                                         const int *n_dev, uint32_t *err) {
+    if (n_dev && *n_dev < n) n = *n_dev;
+    constexpr int ROUNDS = SCAN_ITEMS / 4, NWAVES = SCAN_BLOCK / 64;
+    __shared__ uint32_t s_wave[ROUNDS * NWAVES];
+    __shared__ uint32_t s_tile;
+    __shared__ uint64_t s_prefix;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if ((int64_t)blockIdx.x * SCAN_TILE >= n) {
+        if (n <= 0 && blockIdx.x == 0 && tid == 0) *n_a = *n_b = 0u;
+        return;
+    }
+    if (tid == 0) s_tile = atomicAdd(tile_ctr, 1u);
+    __syncthreads();
+    const int tile = (int)s_tile;
+    const int base = tile * SCAN_TILE + 4 * tid;
+    const bool whole = n - tile * SCAN_TILE >= SCAN_TILE;
+    // one flag of each array per element, packed: a in the low half (a tile
+    // has at most 4,096 of either)
+    uint32_t v[ROUNDS][4], incl[ROUNDS], sum[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int i = base + r * 4 * SCAN_BLOCK;
+        if (whole) {
+            const uint4 p = *reinterpret_cast<const uint4 *>(a + i);
+            const uint4 q = *reinterpret_cast<const uint4 *>(b + i);
+            v[r][0] = p.x | q.x << 16; v[r][1] = p.y | q.y << 16;
+            v[r][2] = p.z | q.z << 16; v[r][3] = p.w | q.w << 16;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[r][k] = i + k < n ? a[i + k] | b[i + k] << 16 : 0u;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        sum[r] = ((v[r][0] + v[r][1]) + v[r][2]) + v[r][3];
+        incl[r] = wave_incl_scan(sum[r]);
+        if (lane == 63) s_wave[r * NWAVES + wave] = incl[r];
+    }
+    __syncthreads();
+    uint32_t off[ROUNDS], tile_sum = 0;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+#pragma unroll
+        for (int w = 0; w < NWAVES; w++) {
+            if (w == wave) off[r] = tile_sum;
+            tile_sum += s_wave[r * NWAVES + w];
+        }
+    const uint64_t both = (uint64_t)(tile_sum >> 16) << 31 | (tile_sum & 0xffffu);
+    if (wave == 0) {
+        const uint64_t prefix = tile == 0 ? 0ull : scan_look_back(status, tile, both, lane, err,
+                                                                   (uint32_t)MI_RB_OVERFLOW_LOOKBACK);
+        if (lane == 0) {
+            __hip_atomic_store(status + tile, SFLAG_INC | (prefix + both), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            s_prefix = prefix;
+        }
+    }
+    __syncthreads();
+    const uint32_t pa = (uint32_t)(s_prefix & 0x7fffffffull), pb = (uint32_t)(s_prefix >> 31);
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int i = base + r * 4 * SCAN_BLOCK;
+        uint32_t run = off[r] + (incl[r] - sum[r]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (v[r][k] & 0xffffu) list_a[pa + (run & 0xffffu)] = (uint32_t)(i + k);
+            if (v[r][k] >> 16) list_b[pb + (run >> 16)] = (uint32_t)(i + k);
+            run += v[r][k];
+        }
+    }
+    if (tile == (n - 1) / SCAN_TILE && tid == 0) {
+        *n_a = pa + (tile_sum & 0xffffu);
+        *n_b = pb + (tile_sum >> 16);
+    }
 }
 
 __global__ void k_scan_empty(uint32_t *total) { if (total) *total = 0; }
@@ -507,7 +598,7 @@ hipError_t launch_radix_sort(uint2 *kv, int n, int sort_bits, int digit_bits, co
 
 hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, int n, uint32_t *total,
                                  uint32_t *status, hipStream_t s, const int *n_dev, int *err,
-                                 uint32_t *idx_out, const uint32_t *idx_base, bool precleared) {
+                                 uint32_t *idx_out, bool precleared) {
     if (n <= 0) {
         RB_LAUNCH(k_scan_empty, dim3(1), dim3(1), 0, s, total);
         return rb_launch_status();
@@ -525,15 +616,24 @@ hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, int n, uint3
     const bool vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
     auto kern = vec ? k_scan<true> : k_scan<false>;
     RB_LAUNCH(kern, dim3(tiles), dim3(SCAN_BLOCK), 0, s, in, out, n, total, st, ctr,
-                       n_dev, e, bit, idx_out, idx_base);
+                       n_dev, e, bit, idx_out);
     return rb_launch_status();
 }
 
 hipError_t launch_compact_flags(const uint32_t *flags, uint32_t *idx_out, int n, uint32_t *total,
                                 uint32_t *status, hipStream_t s, const int *n_dev, int *err,
-                                const uint32_t *idx_base, bool precleared) {
+                                bool precleared) {
     return launch_exclusive_scan(flags, nullptr, n, total, status, s, n_dev, err, idx_out,
-                                 idx_base, precleared);
+                                 precleared);
+}
+
+hipError_t launch_compact2(const uint32_t *a, const uint32_t *b, int n, uint32_t *list_a,
+                           uint32_t *list_b, uint32_t *n_a, uint32_t *n_b, uint32_t *status,
+                           hipStream_t s, const int *n_dev, int *err) {
+    RB_LAUNCH(k_compact2, dim3((n + SCAN_TILE - 1) / SCAN_TILE), dim3(SCAN_BLOCK), 0, s, a, b, n,
+              list_a, list_b, n_a, n_b, reinterpret_cast<uint64_t *>(status + 2), status, n_dev,
+              reinterpret_cast<uint32_t *>(err));
+    return rb_launch_status();
 }
 
 hipError_t launch_bound_search(const uint2 *kv, int n, uint32_t *dst, int n_dst, int mode,

@@ -153,7 +153,8 @@ struct DeviceWorld {
     int2 *pairs;
     // narrowphase
     Contact4 *contact_slots;     // one per pair
-    uint32_t *has_contact, *contact_off;
+    uint32_t *has_contact;
+    uint32_t *contact_pair;      // the pairs with a contact, in order (capacity maxP)
     Contact4 *contacts;          // compacted, ordered by pair
     // solver
     ConstraintSoA cs;
@@ -172,7 +173,7 @@ struct DeviceWorld {
     uint2 *tile_order;           // scene tiles by descending rows: (key, tile)
     // narrowphase pass 1 -> pass 2
     uint32_t *narrow_cand;       // per pair: 1 if not separated by a face axis
-    uint32_t *cand_off;          // its exclusive scan
+    uint32_t *cand_off;          // the candidates' pairs, in order (and the compound scan's offsets)
     int4 *face_best;             // per pair: face minimum (depth bits, axis), edge-axis count
     uint2 *cand_kv;              // (cost key, pair) of the candidates, sorted
     uint2 *tile_res;             // per tile, of the normal then of the friction sweeps: the last
@@ -211,7 +212,7 @@ enum {
     RB_CNT_TILES_SOLVED = 15, // ... and the number of tiles that had rows
     RB_CNT_FACE_WORK = 16,    // uint32 pairs the quick face test left for the face pass
     RB_CNT_CLIP_SPLIT = 17,   // first small-hull candidate in the clip order
-    RB_CNT_FACE_SMALL = 18,   // uint32 small-hull pairs of the face pass (after FACE_WORK's)
+    RB_CNT_FACE_SMALL = 18,   // uint32 small-hull pairs of the face pass
     RB_CNT_SCENES = 19,       // scene tiles: scenes of each solver class (5)
     RB_CNT_COUNT = 24
 };
@@ -300,21 +301,25 @@ size_t sort_status_words(int max_n, int digit_bits);
 hipError_t launch_radix_sort(uint2 *kv, int n, int sort_bits, int digit_bits, const SortWork &w,
                              hipStream_t s, const int *n_dev = nullptr, int tile_keys = 0);
 // out (may be null): exclusive prefix sums of in; idx_out (may be null, in
-// holding 0/1 flags): the indices of the set flags in increasing order, from
-// idx_out[*idx_base] when idx_base (a device count) is given.  precleared:
-// the status words are already zero (a step clears the regions of its scans
-// in its first kernel), so no clearing launch precedes the scan.
+// holding 0/1 flags): the indices of the set flags in increasing order.
+// precleared: the status words are already zero (a step clears the regions of
+// its scans in its first kernel), so no clearing launch precedes the scan.
 hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, int n, uint32_t *total,
                                  uint32_t *status, hipStream_t s, const int *n_dev = nullptr,
                                  int *err = nullptr, uint32_t *idx_out = nullptr,
-                                 const uint32_t *idx_base = nullptr, bool precleared = false);
+                                 bool precleared = false);
 hipError_t launch_compact_flags(const uint32_t *flags, uint32_t *idx_out, int n, uint32_t *total,
                                 uint32_t *status, hipStream_t s, const int *n_dev, int *err,
-                                const uint32_t *idx_base = nullptr, bool precleared = false);
+                                bool precleared = false);
+// both flag arrays (16-byte aligned device allocations) compacted in one pass;
+// the status words are already zero
+hipError_t launch_compact2(const uint32_t *a, const uint32_t *b, int n, uint32_t *list_a,
+                           uint32_t *list_b, uint32_t *n_a, uint32_t *n_b, uint32_t *status,
+                           hipStream_t s, const int *n_dev, int *err);
 // the step's scans, each on its own region of the scan status words
 enum {
     RB_SCAN_PAIRS = 0, RB_SCAN_CONTACTS = 1, RB_SCAN_COMPOUND = 2,
-    RB_SCAN_WORK = 3, RB_SCAN_SMALL = 4, RB_SCAN_CAND = 5, RB_SCAN_REGIONS = 6
+    RB_SCAN_WORK = 3, RB_SCAN_CAND = 4, RB_SCAN_REGIONS = 5
 };
 hipError_t launch_bound_search(const uint2 *kv, int n, uint32_t *dst, int n_dst, int mode,
                                hipStream_t s);

@@ -370,7 +370,7 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.pairs, maxP));
     RB_CHECK(w.alloc(&d.contact_slots, maxP));
     RB_CHECK(w.alloc(&d.has_contact, maxP));
-    RB_CHECK(w.alloc(&d.contact_off, maxP));
+    RB_CHECK(w.alloc(&d.contact_pair, maxP));
     RB_CHECK(w.alloc(&d.contacts, maxC));
     RB_CHECK(w.alloc(&d.cs.linear, maxC));
     RB_CHECK(w.alloc(&d.cs.pos, 4 * (size_t)maxC));
@@ -544,7 +544,7 @@ mi_rb_status enqueue_step(World &w, int last_stage) {
     RB_CHECK(launch_exclusive_scan(d.pair_count, d.pair_off, p.n_bodies,
                                    (uint32_t *)(d.counters + RB_CNT_SORT_TILE),
                                    w.scan_status + RB_SCAN_PAIRS * w.scan_stride, s, nullptr,
-                                   d.counters + RB_CNT_OVERFLOW, nullptr, nullptr, true));
+                                   d.counters + RB_CNT_OVERFLOW, nullptr, true));
     RB_CHECK(launch_emit_pairs(d, p, s));
     if (p.n_proxies > 0)
         RB_CHECK(launch_compound_pairs(d, p, s, w.scan_status, w.scan_stride));
@@ -554,11 +554,10 @@ mi_rb_status enqueue_step(World &w, int last_stage) {
                                 w.scan_stride));
     if (ev) RB_CHECK(hipEventRecord(w.ev[4], s));
     if (last_stage < MI_RB_STAGE_CONSTRAINTS) return MI_RB_OK;
-    RB_CHECK(launch_exclusive_scan(d.has_contact, d.contact_off, p.max_pairs,
-                                   (uint32_t *)(d.counters + RB_CNT_CONTACT_TOTAL),
-                                   w.scan_status + RB_SCAN_CONTACTS * w.scan_stride, s,
-                                   d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW,
-                                   nullptr, nullptr, true));
+    RB_CHECK(launch_compact_flags(d.has_contact, d.contact_pair, p.max_pairs,
+                                  (uint32_t *)(d.counters + RB_CNT_CONTACT_TOTAL),
+                                  w.scan_status + RB_SCAN_CONTACTS * w.scan_stride, s,
+                                  d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW, true));
     RB_CHECK(launch_constraints(d, p, s));
     if (p.warm_start == MI_RB_WARM_LEARNED) RB_CHECK(launch_mlp_warm(d, p, s));
     if (ev) RB_CHECK(hipEventRecord(w.ev[5], s));

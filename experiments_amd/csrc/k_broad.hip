@@ -34,6 +34,13 @@ namespace {
 
 constexpr uint32_t KEY_NONE = 0xffffffffu;
 
+// LDS written by lanes of this wave, then read by others of it
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ void grid_pos(float4 mn, float4 mx, float inv_cell, const int *dims,
                                          int gp[3]) {
     float cx = (mn.x + mx.x) * 0.5f, cy = (mn.y + mx.y) * 0.5f, cz = (mn.z + mx.z) * 0.5f;
@@ -520,22 +527,24 @@ __global__ __launch_bounds__(256) void k_hg_hash(const float4 *__restrict__ mn,
 }
 
 // Cell starts of the sorted keys, the occupancy bit of every occupied cell,
-// a flag per occupied level, and the AABBs in sorted order (so that the pair
-// search reads a cell member's key and box at one index).  occ[] and the
-// level flags after it are cleared before this kernel.
+// a flag per occupied level, and the AABBs in sorted order, two float4 each
+// with the key and the index in their w (so that a cell member is one 32-byte
+// read).  occ[] and the level flags after it are cleared before this kernel.
 __global__ __launch_bounds__(256) void k_hg_cells(const uint2 *__restrict__ kv, int n,
                                                   const float4 *__restrict__ aabb_min,
                                                   const float4 *__restrict__ aabb_max, HGridP g,
                                                   uint32_t *__restrict__ cell_start,
                                                   uint32_t *__restrict__ occ,
                                                   uint32_t *__restrict__ level_used,
-                                                  float4 *__restrict__ smn,
-                                                  float4 *__restrict__ smx) {
+                                                  float4 *__restrict__ boxes) {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     uint2 e = kv[s];
-    smn[s] = aabb_min[e.y];
-    smx[s] = aabb_max[e.y];
+    float4 mn = aabb_min[e.y], mx = aabb_max[e.y];
+    mn.w = __uint_as_float(e.x);
+    mx.w = __uint_as_float(e.y);
+    boxes[2 * (size_t)s] = mn;
+    boxes[2 * (size_t)s + 1] = mx;
     if (e.x == KEY_NONE) return;
     if (s == 0 || kv[s - 1].x != e.x) {
         cell_start[e.x] = (uint32_t)s;
@@ -544,97 +553,255 @@ __global__ __launch_bounds__(256) void k_hg_cells(const uint2 *__restrict__ kv, 
     }
 }
 
-// HG_LANES lanes per sorted entry, lane q taking stencil cells q, q +
-// HG_LANES, ...  A pair (x, y), x > y, belongs to body x.  WRITE = 0: count
-// every found pair for its body; WRITE = 1: store y in the body's range of
-// the scanned counts (slot order within a range is that of the atomics;
-// k_pairs_group orders it).  The entry visits the 27 cells around it on its
-// own level and on every coarser level that holds bodies, and walks only the
-// occupied ones.  With lane_hits the count pass also records each lane's
-// pair count and its first HG_KEEP partners, and the write pass stores
-// those without walking again (only a lane that found more walks again).
-constexpr int HG_LANES = RB_HG_LANES;
-constexpr int HG_KEEP = RB_HG_KEEP;
-template <int WRITE>
-__global__ __launch_bounds__(256) void k_hg_pairs(int n, const uint2 *__restrict__ kv,
-                                                  const uint32_t *__restrict__ cell_start,
-                                                  const uint32_t *__restrict__ occ,
-                                                  const uint32_t *__restrict__ level_used,
-                                                  const float4 *__restrict__ smn,
-                                                  const float4 *__restrict__ smx, HGridP g,
-                                                  uint32_t *__restrict__ counts,
-                                                  const uint32_t *__restrict__ offsets,
-                                                  uint32_t *__restrict__ cursor, int max_pairs,
-                                                  uint32_t *__restrict__ ys,
-                                                  uint32_t *__restrict__ lane_hits) {
-    constexpr int C = (27 + HG_LANES - 1) / HG_LANES;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int t = gid / HG_LANES, lane = gid % HG_LANES;
-    if (t >= n) return;
-    uint2 e = kv[t];
-    if (e.x == KEY_NONE) return;
-    const int x = (int)e.y;
-    uint32_t *rec = lane_hits ? lane_hits + (size_t)gid * (1 + HG_KEEP) : nullptr;
-    if (WRITE && rec) {
-        const uint32_t found = rec[0];
-        if (found <= (uint32_t)HG_KEEP) {
-            for (uint32_t h = 0; h < found; h++) {
-                const int y = (int)rec[1 + h];
-                const uint32_t hi = (uint32_t)(x > y ? x : y), lo = (uint32_t)(x > y ? y : x);
-                const uint32_t pos = offsets[hi] + atomicAdd(&cursor[hi], 1u);
-                if (pos < (uint32_t)max_pairs) ys[pos] = lo;
-            }
-            return;
-        }
+// The pair search: a wave per HG_OWN sorted entries.
+//
+// An entry looks for the members after it on its own level (the rest of its
+// cell and the 13 cells after it in (z, y, x) order, so that each pair is met
+// from one side) and for all members of the 27 cells around it on each coarser
+// level.  The three cells of a stencil row are one key range, so a row is one
+// walk over the sorted boxes; at the grid's edge the wrapped cell is a walk of
+// its own.
+//
+// 1. Lane (entry, level) reads the occupancy bits of its rows and lists those
+//    that hold a member within reach.  2. The lanes look the listed rows'
+//    starts up.  3. Each lane walks one row at a time and takes the next one
+//    of the list when it is through.
+//
+// What bounds it is the latency of dependent reads of single members.  With
+// eight lanes an entry that each walked the occupied ones of their own four
+// cells, level after level, 64 lanes waited for the longest walk of each step:
+// 509 us at 1,048,576 bodies on four levels; listed rows keep the lanes on
+// members: 199, and 166 with two members a read.  (The write pass read 24
+// words an entry again, 87 us; it now streams the pairs that this pass left:
+// 40.)
+constexpr int HG_OWN = RB_HG_OWN, HG_REC = RB_HG_REC;
+constexpr int HG_WAVES = 4;
+// rows of an entry on the lowest of four levels: 5 of its own, 9 of each other
+constexpr int HG_ROWS = HG_OWN * 32;
+struct HGLDS {
+    float4 mn[HG_OWN], mx[HG_OWN];
+    uint32_t first[HG_ROWS];  // first cell's key and, from bit 30, the cells after it
+    uint32_t start[HG_ROWS];
+    uint8_t own[HG_ROWS];
+};
+
+// hits(m, c, y): the lanes of m hold a pair of bodies c and y
+template <class Hits>
+__device__ __forceinline__ void hg_search(int n, const uint32_t *__restrict__ cell_start,
+                                          const uint32_t *__restrict__ occ,
+                                          const uint32_t *__restrict__ level_used,
+                                          const float4 *__restrict__ boxes, const HGridP &g,
+                                          int t0, HGLDS &S, Hits hits) {
+    const int lane = threadIdx.x & 63;
+    const int own = lane & (HG_OWN - 1), sub = lane / HG_OWN;
+    const int t = t0 + own;
+    const uint32_t xmask = (uint32_t)g.dims[0] - 1u;
+    float4 mn0 = mk4(0, 0, 0, 0), mx0 = mn0;
+    uint32_t key = KEY_NONE, next = KEY_NONE;
+    if (t < n) {
+        mn0 = boxes[2 * (size_t)t];
+        mx0 = boxes[2 * (size_t)t + 1];
+        key = __float_as_uint(mn0.w);
+        if (t + 1 < n) next = __float_as_uint(boxes[2 * (size_t)t + 2].w);
     }
-    uint32_t found = 0, keep[HG_KEEP] = {};
-    const int lx = (int)(e.x >> g.cell_bits);
-    const float4 mn0 = smn[t], mx0 = smx[t];
-    for (int l = lx; l < g.levels; l++) {
-        if (l != lx && !level_used[l]) continue;
-        int gp[3];
+    if (sub == 0) {
+        S.mn[own] = mn0;
+        S.mx[own] = mx0;
+    }
+    const int lx = (int)(key >> g.cell_bits), l = lx + sub;
+    // per row the cells that hold members within reach (bit dx + 1), three
+    // bits a row
+    uint32_t rows = 0u;
+    int gp[3] = {0, 0, 0};
+    if (key != KEY_NONE && l < g.levels && (sub == 0 || level_used[l])) {
         const float inv_l = g.inv_cell0 * exp2f(-(float)l);
         hg_cell(mn0, mx0, inv_l, g.dims, gp);
-        const uint32_t reach = reachable_cells(mn0, mx0, inv_l);
-        const uint32_t lk = (uint32_t)l << g.cell_bits;
-        uint32_t nk[C], u0[C];
+        const float c = 1.0f / inv_l, h = 0.5f * c;
+        // (reachable_cells's rule, an axis at a time and with room for the
+        // rounding of far coordinates: a pair is looked for from one side only)
+        uint32_t ok[3];
 #pragma unroll
-        for (int k = 0; k < C; k++) {
-            const int q = lane + k * HG_LANES;
-            nk[k] = 0;
-            u0[k] = (uint32_t)n;
-            if (q < 27 && ((reach >> q) & 1u)) {
-                const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
-                nk[k] = lk | pos_hash(gp[0] + dx, gp[1] + dy, gp[2] + dz, g.dims);
-                if ((occ[nk[k] >> 5] >> (nk[k] & 31u)) & 1u) u0[k] = cell_start[nk[k]];
+        for (int k = 0; k < 3; k++) {
+            const float lo = k == 0 ? mn0.x : k == 1 ? mn0.y : mn0.z;
+            const float hi = k == 0 ? mx0.x : k == 1 ? mx0.y : mx0.z;
+            const float ctr = (lo + hi) * 0.5f, eps = 1e-4f * c + 1e-6f * fabsf(ctr);
+            const float f = floorf(ctr * inv_l);
+            ok[k] = 0u;
+#pragma unroll
+            for (int d = -1; d <= 1; d++) {
+                const float c0 = (f + (float)d) * c - h - eps;
+                const float c1 = (f + (float)(d + 1)) * c + h + eps;
+                if (!(hi < c0) && !(lo > c1)) ok[k] |= 1u << (d + 1);
             }
         }
+        const uint32_t lk = (uint32_t)l << g.cell_bits, gx = (uint32_t)gp[0];
+        uint32_t wl[9], wr[9];
 #pragma unroll
-        for (int k = 0; k < C; k++)
-            for (uint32_t u = u0[k]; u < (uint32_t)n; u++) {
-                uint2 f = kv[u];
-                if (f.x != nk[k]) break;
-                int y = (int)f.y;
-                if (l == lx && y >= x) continue;
-                if (!aabb_overlap(mn0, mx0, smn[u], smx[u])) continue;
-                const uint32_t hi = (uint32_t)(x > y ? x : y), lo = (uint32_t)(x > y ? y : x);
-                if (!WRITE) {
-                    atomicAdd(&counts[hi], 1u);
+        for (int r = 0; r < 9; r++) {
+            const uint32_t b = lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
+            const bool in = ((ok[1] >> (r % 3)) & 1u) && ((ok[2] >> (r / 3)) & 1u) &&
+                            (sub > 0 || r >= 4);
+            wl[r] = in ? occ[(b | ((gx - 1u) & xmask)) >> 5] : 0u;
+            wr[r] = in ? occ[(b | ((gx + 1u) & xmask)) >> 5] : 0u;
+        }
 #pragma unroll
-                    for (int h = 0; h < HG_KEEP; h++)
-                        if (found == (uint32_t)h) keep[h] = (uint32_t)y;
-                    found++;
-                } else {
-                    uint32_t pos = offsets[hi] + atomicAdd(&cursor[hi], 1u);
-                    if (pos < (uint32_t)max_pairs) ys[pos] = lo;
+        for (int r = 0; r < 9; r++) {
+            // (rows of cells start at a multiple of four, so their cell 0 and 1
+            // lie in one word, as do their last two)
+            const uint32_t xl = (gx - 1u) & xmask, xr = (gx + 1u) & xmask;
+            const uint32_t b = lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
+            const uint32_t wc = ((b | gx) >> 5) == ((b | xl) >> 5) ? wl[r] : wr[r];
+            uint32_t m = ((wl[r] >> ((b | xl) & 31u)) & 1u) |
+                         ((wc >> ((b | gx) & 31u)) & 1u) << 1 |
+                         ((wr[r] >> ((b | xr) & 31u)) & 1u) << 2;
+            m &= ok[0];
+            if (sub == 0 && r == 4) m = (m & 4u) | (next == key ? 2u : 0u);
+            rows |= m << (3 * r);
+        }
+    }
+    // the wrapped cell of every row waits for the second round
+    const uint32_t wrapped = gp[0] == 0 ? 0111111111u : (uint32_t)gp[0] == xmask ? 0444444444u : 0u;
+    uint32_t rest = rows & wrapped;
+    rows &= ~wrapped;
+    const uint32_t lk = (uint32_t)l << g.cell_bits;
+    for (int round = 0; round < 2; round++) {
+        uint32_t total = 0;
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            const uint32_t m = (rows >> (3 * r)) & 7u;
+            const uint64_t has = __ballot(m != 0u);
+            if (m) {
+                const uint32_t p = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, total));
+                const uint32_t b = lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
+                const uint32_t lo = (uint32_t)__builtin_ctz(m), hi = 31u - (uint32_t)__builtin_clz(m);
+                const uint32_t x = ((uint32_t)gp[0] + lo - 1u) & xmask;
+                S.first[p] = b | x | (hi - lo) << 30;
+                // (the own row starts after the entry itself)
+                S.start[p] = sub == 0 && r == 4 && round == 0 ? (uint32_t)t + 1u : 0u;
+                S.own[p] = (uint8_t)own;
+            }
+            total += (uint32_t)__popcll(has);
+        }
+        if (total) {
+            wave_fence();
+            for (uint32_t p = lane; p < total; p += 64)
+                if (S.start[p] == 0u) S.start[p] = cell_start[S.first[p] & 0x3fffffffu];
+            wave_fence();
+            uint32_t at = 64u, u = 0u, last = 0u;
+            int y = 0;
+            float4 a = mn0, b = mx0;
+            bool walk = (uint32_t)lane < total;
+            auto take = [&](uint32_t p) {
+                const uint32_t f = S.first[p];
+                const int o = (int)S.own[p];
+                a = S.mn[o];
+                b = S.mx[o];
+                u = S.start[p];
+                last = (f & 0x3fffffffu) + (f >> 30);
+                y = __float_as_int(b.w);
+            };
+            if (walk) take((uint32_t)lane);
+            while (__ballot(walk)) {
+                bool hit[2] = {false, false}, end = false;
+                int c[2] = {0, 0};
+                if (walk) {
+                    const uint32_t v = u + 1u < (uint32_t)n ? u + 1u : u;
+                    const float4 p0 = boxes[2 * (size_t)u], q0 = boxes[2 * (size_t)u + 1];
+                    const float4 p1 = boxes[2 * (size_t)v], q1 = boxes[2 * (size_t)v + 1];
+                    const bool in0 = __float_as_uint(p0.w) <= last;
+                    const bool in1 = in0 && v != u && __float_as_uint(p1.w) <= last;
+                    hit[0] = in0 && aabb_overlap(a, b, p0, q0);
+                    hit[1] = in1 && aabb_overlap(a, b, p1, q1);
+                    c[0] = __float_as_int(q0.w);
+                    c[1] = __float_as_int(q1.w);
+                    u += 2u;
+                    end = !in1 || u >= (uint32_t)n;
+                }
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const uint64_t m = __ballot(hit[k]);
+                    if (m) hits(m, c[k], y);
+                }
+                const uint64_t done = __ballot(end);
+                if (done) {
+                    if (end) {
+                        const uint32_t p = __builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(done >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)done, at));
+                        walk = p < total;
+                        if (walk) take(p);
+                    }
+                    at += (uint32_t)__popcll(done);
                 }
             }
+        }
+        rows = rest;
+        if (__ballot(rest != 0u) == 0ull) break;
+        wave_fence();
     }
-    if (!WRITE && rec) {
-        rec[0] = found;
-#pragma unroll
-        for (int h = 0; h < HG_KEEP; h++) rec[1 + h] = keep[h];
+}
+// A pair (x, y), x > y, belongs to body x.  The count pass keeps its wave's
+// pairs in LDS, counts them and leaves them in the wave's part of rec (HG_REC
+// pairs; rec_n[wave] their number, or more when they did not fit) for the
+// write pass, which searches again only where they did not fit (slot order
+// within a body's range is that of the atomics; k_pairs_group orders it).
+__global__ __launch_bounds__(64 * HG_WAVES) void k_hg_count(
+    int n, const uint32_t *__restrict__ cell_start, const uint32_t *__restrict__ occ,
+    const uint32_t *__restrict__ level_used, const float4 *__restrict__ boxes, HGridP g,
+    uint32_t *__restrict__ counts, uint2 *__restrict__ rec, uint32_t *__restrict__ rec_n) {
+    __shared__ HGLDS S[HG_WAVES];
+    __shared__ uint2 s_rec[HG_WAVES][HG_REC];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int wave = (int)blockIdx.x * HG_WAVES + w;
+    if ((int64_t)wave * HG_OWN >= n) return;
+    uint32_t found = 0;
+    hg_search(n, cell_start, occ, level_used, boxes, g, wave * HG_OWN, S[w],
+              [&](uint64_t m, int c, int y) {
+                  if ((m >> lane) & 1ull) {
+                      const uint32_t p = __builtin_amdgcn_mbcnt_hi(
+                          (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, found));
+                      const uint32_t hi = (uint32_t)(c > y ? c : y), lo = (uint32_t)(c > y ? y : c);
+                      if (p < (uint32_t)HG_REC) s_rec[w][p] = make_uint2(hi, lo);
+                      else atomicAdd(&counts[hi], 1u);
+                  }
+                  found += (uint32_t)__popcll(m);
+              });
+    wave_fence();
+    const uint32_t kept = found < (uint32_t)HG_REC ? found : (uint32_t)HG_REC;
+    for (uint32_t p = lane; p < kept; p += 64) {
+        const uint2 e = s_rec[w][p];
+        atomicAdd(&counts[e.x], 1u);
+        rec[(size_t)wave * HG_REC + p] = e;
     }
+    if (lane == 0) rec_n[wave] = found;
+}
+__global__ __launch_bounds__(64 * HG_WAVES) void k_hg_write(
+    int n, const uint32_t *__restrict__ cell_start, const uint32_t *__restrict__ occ,
+    const uint32_t *__restrict__ level_used, const float4 *__restrict__ boxes, HGridP g,
+    const uint32_t *__restrict__ offsets, uint32_t *__restrict__ cursor, int max_pairs,
+    uint32_t *__restrict__ ys, const uint2 *__restrict__ rec,
+    const uint32_t *__restrict__ rec_n) {
+    __shared__ HGLDS S[HG_WAVES];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int wave = (int)blockIdx.x * HG_WAVES + w;
+    if ((int64_t)wave * HG_OWN >= n) return;
+    auto put = [&](uint32_t hi, uint32_t lo) {
+        const uint32_t pos = offsets[hi] + atomicAdd(&cursor[hi], 1u);
+        if (pos < (uint32_t)max_pairs) ys[pos] = lo;
+    };
+    const uint32_t found = rec_n[wave];
+    if (found <= (uint32_t)HG_REC) {
+        for (uint32_t p = lane; p < found; p += 64) {
+            const uint2 e = rec[(size_t)wave * HG_REC + p];
+            put(e.x, e.y);
+        }
+        return;
+    }
+    hg_search(n, cell_start, occ, level_used, boxes, g, wave * HG_OWN, S[w],
+              [&](uint64_t m, int c, int y) {
+                  if ((m >> lane) & 1ull)
+                      put((uint32_t)(c > y ? c : y), (uint32_t)(c > y ? y : c));
+              });
 }
 
 // The pair range of body x: [offsets[x], offsets[x] + counts[x]) clipped to
@@ -1151,19 +1318,19 @@ static void launch_pairs_group(int n, uint32_t *counts, uint32_t *offsets, uint3
 // per body, scan, write, then each body's pairs ordered by y.
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *smn, float4 *smx,
+                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,
-                              uint32_t *scan_status, hipStream_t s, hipEvent_t *ev,
-                              uint32_t *lane_hits) {
+                              uint32_t *scan_status, hipStream_t s, hipEvent_t *ev, uint2 *rec,
+                              uint32_t *rec_n) {
     HGridP g;
     g.inv_cell0 = inv_cell0;
     g.dims[0] = dims[0]; g.dims[1] = dims[1]; g.dims[2] = dims[2];
     g.cell_bits = cell_bits;
     g.levels = levels;
     const int blocks = n > 0 ? (n + 255) / 256 : 1;
-    const int hg_blocks = (int)(((int64_t)n * HG_LANES + 255) / 256);
+    const int hg_blocks = (n + HG_WAVES * HG_OWN - 1) / (HG_WAVES * HG_OWN);
     uint32_t *big_n = big + (n > 0 ? n : 0);
     if (ev) hipEventRecord(ev[0], s);
     RB_LAUNCH(k_hg_hash, dim3(blocks), dim3(256), 0, s, mn, mx, n, g, kv, counts, cursor,
@@ -1179,17 +1346,15 @@ hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float i
         e = launch_fill_u32(occ, 0u, occ_words + 4, s);
         if (e != hipSuccess) return e;
         RB_LAUNCH(k_hg_cells, dim3(blocks), dim3(256), 0, s, kv, n, mn, mx, g, cell_start,
-                           occ, level_used, smn, smx);
-        RB_LAUNCH(k_hg_pairs<0>, dim3(hg_blocks), dim3(256), 0, s, n, kv, cell_start, occ,
-                           level_used, smn, smx, g, counts, (const uint32_t *)nullptr, cursor,
-                           max_pairs, ys, lane_hits);
+                           occ, level_used, boxes);
+        RB_LAUNCH(k_hg_count, dim3(hg_blocks), dim3(64 * HG_WAVES), 0, s, n, cell_start, occ,
+                  level_used, boxes, g, counts, rec, rec_n);
     }
     e = launch_exclusive_scan(counts, offsets, n, total, scan_status, s, nullptr, overflow);
     if (e != hipSuccess) return e;
     if (n > 0)
-        RB_LAUNCH(k_hg_pairs<1>, dim3(hg_blocks), dim3(256), 0, s, n, kv, cell_start, occ,
-                           level_used, smn, smx, g, counts, offsets, cursor, max_pairs, ys,
-                           lane_hits);
+        RB_LAUNCH(k_hg_write, dim3(hg_blocks), dim3(64 * HG_WAVES), 0, s, n, cell_start, occ,
+                  level_used, boxes, g, offsets, cursor, max_pairs, ys, rec, rec_n);
     if (ev) hipEventRecord(ev[3], s);
     launch_pairs_group(n, counts, offsets, total, max_pairs, ys, pairs, num_pairs, overflow, big,
                        big_n, blocks, s);

@@ -370,19 +370,19 @@ hipError_t launch_mlp_warm(const DeviceWorld &d, const StepParams &p, hipStream_
 hipError_t launch_mlp_targets(const DeviceWorld &d, int capacity, float *x_out, float *t_out,
                               hipStream_t s);
 
-// the stand-alone grid API.  lane_hits (may be null): RB_HG_LANES x (1 +
-// RB_HG_KEEP) words per body, where the count pass leaves each lane's pairs
-// for the write pass
-#define RB_HG_LANES 8
-#define RB_HG_KEEP 2
+// the stand-alone grid API.  boxes: two per AABB.  rec, rec_n: where the count
+// pass leaves the pairs of each RB_HG_OWN sorted AABBs for the write pass,
+// RB_HG_REC pairs and one count
+#define RB_HG_OWN 16
+#define RB_HG_REC 192
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *smn, float4 *smx,
+                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,
-                              uint32_t *scan_status, hipStream_t s, hipEvent_t *ev,
-                              uint32_t *lane_hits);
+                              uint32_t *scan_status, hipStream_t s, hipEvent_t *ev, uint2 *rec,
+                              uint32_t *rec_n);
 // the sweep-and-prune API.  rec, rec_n: where the count pass leaves the pairs
 // of each 32 sorted AABBs for the write pass, RB_SAP_REC pairs and one count
 #define RB_SAP_REC 512

@@ -1747,16 +1747,17 @@ struct Grid {
     uint32_t *cursor = nullptr, *big = nullptr;
     uint32_t *cell_start = nullptr, *counts = nullptr, *offsets = nullptr, *total = nullptr;
     uint32_t *occ = nullptr;             // occupancy bit per cell, then one flag per level
-    float4 *smn = nullptr, *smx = nullptr;  // AABBs in sorted order
+    float4 *boxes = nullptr;             // AABBs in sorted order, with their keys and indices
     int *overflow = nullptr;
     SortWork sw{};
     uint32_t *scan_status = nullptr;
-    uint32_t *lane_hits = nullptr;       // per body and search lane: pair count, first partners
+    uint2 *rec = nullptr;                // pairs of the count pass for the write pass
+    uint32_t *rec_n = nullptr;
     int cell_bits = 0;
     hipEvent_t ev[5] = {};
     void release() {
         void *ps[] = {kv, ys, cursor, big, cell_start, counts, offsets, total, overflow, sw.tmp,
-                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, smn, smx, lane_hits};
+                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, boxes, rec, rec_n};
         for (void *p : ps) if (p) hipFree(p);
         for (auto &e : ev) if (e) hipEventDestroy(e);
     }
@@ -1777,18 +1778,20 @@ extern "C" mi_rb_status mi_rb_grid_create(const mi_rb_grid_desc *desc, int max_a
     if (g->cell_bits > 28) { delete g; return MI_RB_INVALID_ARG; }
     size_t ncells = (size_t)1 << (g->cell_bits + 2);
     int n = max_aabbs, P = desc->max_pairs;
+    const size_t rec_units = ((size_t)n + RB_HG_OWN - 1) / RB_HG_OWN;
     bool ok = dalloc(&g->kv, n) == hipSuccess && dalloc(&g->ys, P) == hipSuccess &&
               dalloc(&g->cursor, n) == hipSuccess && dalloc(&g->big, (size_t)n + 2) == hipSuccess &&
               dalloc(&g->cell_start, ncells) == hipSuccess &&
-              dalloc(&g->occ, ncells / 32 + 4) == hipSuccess && dalloc(&g->smn, n) == hipSuccess &&
-              dalloc(&g->smx, n) == hipSuccess && dalloc(&g->counts, n) == hipSuccess &&
+              dalloc(&g->occ, ncells / 32 + 4) == hipSuccess &&
+              dalloc(&g->boxes, 2 * (size_t)n) == hipSuccess && dalloc(&g->counts, n) == hipSuccess &&
               dalloc(&g->offsets, n) == hipSuccess && dalloc(&g->total, 4) == hipSuccess &&
               dalloc(&g->overflow, 4) == hipSuccess && dalloc(&g->sw.tmp, n) == hipSuccess &&
               dalloc(&g->sw.hist, 8 * 256) == hipSuccess &&
               dalloc(&g->sw.status, sort_status_words(n, 8)) == hipSuccess &&
               dalloc(&g->sw.tile_ctr, 16) == hipSuccess &&
               dalloc(&g->scan_status, rb_scan_status_words(n)) == hipSuccess &&
-              dalloc(&g->lane_hits, (size_t)n * RB_HG_LANES * (1 + RB_HG_KEEP)) == hipSuccess;
+              dalloc(&g->rec, rec_units * RB_HG_REC) == hipSuccess &&
+              dalloc(&g->rec_n, rec_units) == hipSuccess;
     if (!ok) { g->release(); delete g; return MI_RB_DEVICE; }
     g->sw.max_n = n;
     g->sw.max_tiles = rb_sort_tiles(n);
@@ -1823,11 +1826,11 @@ extern "C" mi_rb_status mi_rb_grid_find_pairs(void *grid, const void *d_aabb_min
     RB_CHECK(launch_hgrid_pairs(static_cast<const float4 *>(d_aabb_min),
                                 static_cast<const float4 *>(d_aabb_max), n,
                                 1.0f / g->desc.cell_size, g->desc.dims, g->cell_bits,
-                                g->desc.levels, g->kv, g->cell_start, g->occ, g->smn, g->smx,
+                                g->desc.levels, g->kv, g->cell_start, g->occ, g->boxes,
                                 g->counts, g->offsets, g->cursor, g->big, g->total, g->ys,
                                 g->desc.max_pairs,
                                 static_cast<int2 *>(d_pairs), static_cast<int *>(d_num_pairs),
-                                g->overflow, g->sw, g->scan_status, s, g->ev, g->lane_hits));
+                                g->overflow, g->sw, g->scan_status, s, g->ev, g->rec, g->rec_n));
     return MI_RB_OK;
 }
 

@@ -207,7 +207,8 @@ constexpr int SG_FACES = 16;
 constexpr int SG_POLY = 2 * SG_VERTS;
 constexpr int SG_GROUPS = NP_BLOCK / SG;
 static_assert(SG_POLY <= SG, "one lane per polygon vertex");
-__device__ __forceinline__ bool small_hull(const HullInfo &h) {
+template <class Hull>
+__device__ __forceinline__ bool small_hull(const Hull &h) {
     return h.num_vertices <= SG_VERTS && h.num_edges <= SG_EDGES && h.num_faces <= SG_FACES;
 }
 // LDS written by lanes of this wave, then read by others of it
@@ -254,7 +255,8 @@ static_assert(RB_MAX_HULL_VERTS <= RB_MAX_POLY, "a face's side planes fit the po
 // by an overlap bound first
 constexpr int FACE_PLAIN_MAX = 32;
 
-__device__ __forceinline__ bool hull_limits_ok(const HullInfo &hA, const HullInfo &hB) {
+template <class Hull>
+__device__ __forceinline__ bool hull_limits_ok(const Hull &hA, const Hull &hB) {
     return hA.num_vertices <= RB_MAX_HULL_VERTS && hB.num_vertices <= RB_MAX_HULL_VERTS &&
            hA.num_edges <= RB_MAX_HULL_EDGES && hB.num_edges <= RB_MAX_HULL_EDGES &&
            hA.num_faces <= 2 * NP_BLOCK && hB.num_faces <= 2 * NP_BLOCK;
@@ -355,55 +357,120 @@ __global__ __launch_bounds__(256) void k_narrow_special(
     }
 }
 
-// Pass 0, QL lanes per pair: the face of A that B's centre lies furthest
-// outside of, and the face of B that A's centre lies furthest outside of.
-// Both axes are built and projected with pass 1's arithmetic, so an axis
-// that separates here separates in pass 1 too, and pass 1 (which projects
-// every face axis, or leaves out only axes that cannot separate) would give
-// the pair no contact: it gets none here.  The other pairs (and every pair
-// that is not hull-hull within the limits) are flagged for pass 1 (pairs of
-// two small hulls in cand for its SG-lane kernel, the others in has_contact
-// for its wave-per-pair kernel), which takes them in pair order from the
-// compacted flags and sets cand and has_contact itself (pass 2 for its
-// candidates).  Most broadphase pairs are apart, so pass 1 runs on a
-// fraction of them.  With QL > 1
-// the lanes of a pair split its faces and vertices.
-// lanes per pair of pass 0 (4 timed faster than 1 and 8 on the 65,537-hull
-// scene: fewer cache lines per load than 1, less repeated work than 8)
+// Pass 0, four lanes per pair: the face of A that B's centre lies furthest
+// outside of, and the face of B that A's centre lies furthest outside of.  A
+// pair that one of these two axes separates by more than the rounding of pass
+// 1 (which projects every face axis, or leaves out only axes that cannot
+// separate) would get no contact from pass 1: it gets none here.  The other
+// pairs (and every pair that is not hull-hull within the limits) are flagged
+// for pass 1 (pairs of two small hulls in cand for its SG-lane kernel, the
+// others in has_contact for its wave-per-pair kernel), which takes them in
+// pair order from the compacted flags and sets cand and has_contact itself
+// (pass 2 for its candidates).  Most broadphase pairs are apart, so pass 1
+// runs on a fraction of them.
+//
+// The lanes of a pair split its faces and vertices (4 timed faster than 1 and
+// 8 on the 65,537-hull scene: fewer cache lines per load than 1, less repeated
+// work than 8).  The kernel is bound by its instructions, most of which were
+// pass 1's rotations (two quaternion products each, a dozen a pair), taken so
+// that the separation was pass 1's to the bit.  The margin needs no bits: the
+// pair is worked on in the hulls' own frames, with one relative rotation
+// matrix (3.4M pairs of small hulls 258 -> 185 us, 635k pairs of 32-vertex
+// hulls 97 -> 76).
 constexpr int QUICK_LANES = 4;
-template <int QL>
-__device__ __forceinline__ void group_argmax(float &d, int &idx) {
-#pragma unroll
-    for (int o = 1; o < QL; o <<= 1) {
-        const float od = __shfl_xor(d, o, 64);
-        const int oi = __shfl_xor(idx, o, 64);
-        if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
-    }
+template <int PERM>
+__device__ __forceinline__ float quad_f(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), PERM, 0xf, 0xf, true));
 }
-// project() with the group's own hull (vector loads), its vertices split
-// over the QL lanes of the group (every lane of the group must call it)
-template <int QL>
-__device__ __forceinline__ void project_group(const float4 *__restrict__ v, int nv, int sub,
-                                              float4 pos, float4 orn, float4 dir, float &mn,
-                                              float &mx) {
-    const float4 ld = qt_inv_rotate(orn, dir);
-    const float off = dot3(pos, dir);
-    float lo = FLT_MAX, hi = -FLT_MAX;
-    for (int i = sub; i < nv; i += QL) {
-        const float4 q = v[i];
-        const float dp = (q.x * ld.x + q.y * ld.y) + q.z * ld.z;
-        lo = fminf(lo, dp);
-        hi = fmaxf(hi, dp);
-    }
-#pragma unroll
-    for (int o = 1; o < QL; o <<= 1) {
-        lo = fminf(lo, __shfl_xor(lo, o, 64));
-        hi = fmaxf(hi, __shfl_xor(hi, o, 64));
-    }
-    mn = lo + off;
-    mx = hi + off;
+// lane ^ 1 and lane ^ 2 of the quad; quad_from: every lane gets lane K's value
+constexpr int QUAD_X1 = 0xb1, QUAD_X2 = 0x4e;
+template <int K>
+__device__ __forceinline__ int quad_from(int x) {
+    return __builtin_amdgcn_mov_dpp(x, K * 0x55, 0xf, 0xf, true);
 }
-template <int QL>
+template <int K>
+__device__ __forceinline__ float quad_from(float x) {
+    return quad_f<K * 0x55>(x);
+}
+template <int K>
+__device__ __forceinline__ float4 quad_from(float4 v) {
+    return mk4(quad_from<K>(v.x), quad_from<K>(v.y), quad_from<K>(v.z), quad_from<K>(v.w));
+}
+__device__ __forceinline__ float quad_max(float x) {
+    x = fmaxf(x, quad_f<QUAD_X1>(x));
+    return fmaxf(x, quad_f<QUAD_X2>(x));
+}
+__device__ __forceinline__ float quad_min(float x) {
+    x = fminf(x, quad_f<QUAD_X1>(x));
+    return fminf(x, quad_f<QUAD_X2>(x));
+}
+__device__ __forceinline__ void quad_argmax(float &d, int &idx) {
+    float od = quad_f<QUAD_X1>(d);
+    int oi = __builtin_amdgcn_mov_dpp(idx, QUAD_X1, 0xf, 0xf, true);
+    if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
+    od = quad_f<QUAD_X2>(d);
+    oi = __builtin_amdgcn_mov_dpp(idx, QUAD_X2, 0xf, 0xf, true);
+    if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
+}
+struct V3 { float x, y, z; };
+__device__ __forceinline__ float fdot(V3 a, float x, float y, float z) {
+    return fmaf(a.x, x, fmaf(a.y, y, a.z * z));
+}
+__device__ __forceinline__ float norm1(float x, float y, float z) {
+    return fabsf(x) + fabsf(y) + fabsf(z);
+}
+// The pose of hull A seen from hull B: x_B = m x_A + tb, x_A = m^T x_B + ta.
+// near: an upper bound of the rounding by which a gap along a unit axis in
+// these frames and one from pass 1's projections differ, without the hulls'
+// part, near_l times a bound of their vertices' norms; the bound holds for
+// unit quaternions (ok).
+struct RelPose {
+    V3 m[3], ta, tb;
+    float near;
+    bool ok;
+    __device__ __forceinline__ V3 to_b(float x, float y, float z) const {  // m v
+        return {fdot(m[0], x, y, z), fdot(m[1], x, y, z), fdot(m[2], x, y, z)};
+    }
+    __device__ __forceinline__ V3 to_a(float x, float y, float z) const {  // m^T v
+        return {fmaf(m[0].x, x, fmaf(m[1].x, y, m[2].x * z)),
+                fmaf(m[0].y, x, fmaf(m[1].y, y, m[2].y * z)),
+                fmaf(m[0].z, x, fmaf(m[1].z, y, m[2].z * z))};
+    }
+};
+constexpr float NEAR_L = 1e-4f;
+__device__ __forceinline__ RelPose rel_pose(float4 pA, float4 a, float4 pB, float4 b) {
+    RelPose r;
+    // conj(b) a
+    const float qx = fmaf(b.w, a.x, fmaf(-b.x, a.w, fmaf(-b.y, a.z, b.z * a.y)));
+    const float qy = fmaf(b.w, a.y, fmaf(-b.y, a.w, fmaf(-b.z, a.x, b.x * a.z)));
+    const float qz = fmaf(b.w, a.z, fmaf(-b.z, a.w, fmaf(-b.x, a.y, b.y * a.x)));
+    const float qw = fmaf(b.w, a.w, fmaf(b.x, a.x, fmaf(b.y, a.y, b.z * a.z)));
+    const float x2 = qx + qx, y2 = qy + qy, z2 = qz + qz;
+    const float xx = qx * x2, yy = qy * y2, zz = qz * z2;
+    const float wx = qw * x2, wy = qw * y2, wz = qw * z2;
+    r.m[0] = {1.f - (yy + zz), fmaf(qx, y2, -wz), fmaf(qx, z2, wy)};
+    r.m[1] = {fmaf(qx, y2, wz), 1.f - (xx + zz), fmaf(qy, z2, -wx)};
+    r.m[2] = {fmaf(qx, z2, -wy), fmaf(qy, z2, wx), 1.f - (xx + yy)};
+    // conj(a) (pB - pA) a
+    const float dx = pB.x - pA.x, dy = pB.y - pA.y, dz = pB.z - pA.z;
+    const float cx = 2.f * fmaf(a.z, dy, -a.y * dz), cy = 2.f * fmaf(a.x, dz, -a.z * dx),
+                cz = 2.f * fmaf(a.y, dx, -a.x * dy);
+    r.ta = {fmaf(a.w, cx, dx) - fmaf(a.y, cz, -a.z * cy),
+            fmaf(a.w, cy, dy) - fmaf(a.z, cx, -a.x * cz),
+            fmaf(a.w, cz, dz) - fmaf(a.x, cy, -a.y * cx)};
+    const V3 t = r.to_b(r.ta.x, r.ta.y, r.ta.z);
+    r.tb = {-t.x, -t.y, -t.z};
+    r.near = 4e-6f * (norm1(pA.x, pA.y, pA.z) + norm1(pB.x, pB.y, pB.z)) +
+             NEAR_L * norm1(dx, dy, dz);
+    const float na = fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, a.w * a.w)));
+    const float nb = fmaf(b.x, b.x, fmaf(b.y, b.y, fmaf(b.z, b.z, b.w * b.w)));
+    r.ok = fabsf(na - 1.f) < 1e-5f && fabsf(nb - 1.f) < 1e-5f;
+    return r;
+}
+struct QuickHull {
+    int face_offset, num_faces, vertex_offset, num_vertices, num_edges;
+    float4 center;
+};
 __global__ __launch_bounds__(256) void k_narrow_quick(
     int max_pairs, const int *__restrict__ num_pairs_ptr, const int2 *__restrict__ pairs,
     const float4 *__restrict__ pos, const float4 *__restrict__ quat,
@@ -411,6 +478,7 @@ __global__ __launch_bounds__(256) void k_narrow_quick(
     const HullInfo *__restrict__ hulls, const float4 *__restrict__ verts,
     const float4 *__restrict__ planes, uint32_t *__restrict__ has_contact,
     uint32_t *__restrict__ cand) {
+    constexpr int QL = QUICK_LANES;
     int npairs = *num_pairs_ptr;
     if (npairs > max_pairs) npairs = max_pairs;
     const int sub = threadIdx.x & (QL - 1);
@@ -419,54 +487,80 @@ __global__ __launch_bounds__(256) void k_narrow_quick(
     if (p >= npairs) return;
     const int2 pr = pairs[p];
     bool sep = false, small = false;
-    if (inv_mass[pr.x] != 0.f || inv_mass[pr.y] != 0.f) {
-        const HullInfo hA = hulls[shape[pr.x]];
-        const HullInfo hB = hulls[shape[pr.y]];
+    // the pair's records, a part a lane (a load costs by its lanes, also where
+    // they read the same): masses and shapes, both poses, then the three
+    // 16-byte parts of each hull that are used here
+    const int body = sub & 1 ? pr.y : pr.x;
+    const int ms = sub < 2 ? __float_as_int(inv_mass[body]) : shape[body];
+    const float4 pose = (sub & 2 ? quat : pos)[body];
+    const float mA = __int_as_float(quad_from<0>(ms)), mB = __int_as_float(quad_from<1>(ms));
+    if (mA != 0.f || mB != 0.f) {
+        const int part = sub < 2 ? sub : 2;
+        QuickHull hA, hB;
+        auto hull = [&](int s, QuickHull &h) {
+            static_assert(offsetof(HullInfo, num_edges) == 20 && offsetof(HullInfo, center) == 32);
+            const int4 v = ((const int4 *)(hulls + s))[part];
+            h.face_offset = quad_from<0>(v.x);
+            h.num_faces = quad_from<0>(v.y);
+            h.vertex_offset = quad_from<0>(v.z);
+            h.num_vertices = quad_from<0>(v.w);
+            h.num_edges = quad_from<1>(v.y);
+            h.center = mk4(__int_as_float(quad_from<2>(v.x)), __int_as_float(quad_from<2>(v.y)),
+                           __int_as_float(quad_from<2>(v.z)), 0.f);
+        };
+        hull(quad_from<2>(ms), hA);
+        hull(quad_from<3>(ms), hB);
         if (hA.num_vertices > 0 && hB.num_vertices > 0 && hull_limits_ok(hA, hB)) {
             small = small_hull(hA) && small_hull(hB);
-            float4 pA = pos[pr.x], pB = pos[pr.y];
-            const float4 oA = quat[pr.x], oB = quat[pr.y];
-            pA.w = 0.f;
-            pB.w = 0.f;
-            const float4 cA = xform(hA.center, pA, oA), cB = xform(hB.center, pB, oB);
-            const float4 dc = sub4(cA, cB);
+            const RelPose r = rel_pose(quad_from<0>(pose), quad_from<2>(pose),
+                                       quad_from<1>(pose), quad_from<3>(pose));
             const float4 *pa = planes + hA.face_offset, *pb = planes + hB.face_offset;
-            // the faces: largest signed distance of the other centre (local
-            // frame); any choice keeps the result exact
-            const float4 lB = qt_inv_rotate(oA, sub4(cB, pA));
-            const float4 lA = qt_inv_rotate(oB, sub4(cA, pB));
+            // the faces: largest signed distance of the other centre (any
+            // choice keeps the result exact)
+            const V3 b0 = r.to_a(hB.center.x, hB.center.y, hB.center.z);
+            const V3 a0 = r.to_b(hA.center.x, hA.center.y, hA.center.z);
+            const V3 lB = {b0.x + r.ta.x, b0.y + r.ta.y, b0.z + r.ta.z};
+            const V3 lA = {a0.x + r.tb.x, a0.y + r.tb.y, a0.z + r.tb.z};
             float sa = -FLT_MAX, sb = -FLT_MAX;
             int fa = 0x7fffffff, fb = 0x7fffffff;
             for (int f = sub; f < hA.num_faces; f += QL) {
                 const float4 pl = pa[f];
-                const float d = dot3(pl, lB) + pl.w;
+                const float d = fdot(lB, pl.x, pl.y, pl.z) + pl.w;
                 if (d > sa) { sa = d; fa = f; }
             }
             for (int f = sub; f < hB.num_faces; f += QL) {
                 const float4 pl = pb[f];
-                const float d = dot3(pl, lA) + pl.w;
+                const float d = fdot(lA, pl.x, pl.y, pl.z) + pl.w;
                 if (d > sb) { sb = d; fb = f; }
             }
-            group_argmax<QL>(sa, fa);
-            group_argmax<QL>(sb, fb);
+            quad_argmax(sa, fa);
+            quad_argmax(sb, fb);
             if (fa >= hA.num_faces) fa = 0;  // NaN distances: any face will do
             if (fb >= hB.num_faces) fb = 0;
+            // both axes in both frames (a hull without faces gives none: a
+            // zero axis has no gap)
+            const float4 z = mk4(0.f, 0.f, 0.f, 0.f);
+            const float4 wa = hA.num_faces > 0 ? pa[fa] : z, wb = hB.num_faces > 0 ? pb[fb] : z;
+            const V3 wab = r.to_b(wa.x, wa.y, wa.z), wba = r.to_a(wb.x, wb.y, wb.z);
             const float4 *vA = verts + hA.vertex_offset, *vB = verts + hB.vertex_offset;
-            float mn0, mx0, mn1, mx1;
-            if (hA.num_faces > 0) {
-                float4 w = qt_rotate(oA, pa[fa]);
-                if (dot3(dc, w) < 0) w = scl4(w, -1.f);
-                project_group<QL>(vA, hA.num_vertices, sub, pA, oA, w, mn0, mx0);
-                project_group<QL>(vB, hB.num_vertices, sub, pB, oB, w, mn1, mx1);
-                sep = mx0 < mn1 || mx1 < mn0;
+            float maxA = -FLT_MAX, minB = FLT_MAX, maxB = -FLT_MAX, minA = FLT_MAX, len = 0.f;
+            for (int i = sub; i < hA.num_vertices; i += QL) {
+                const float4 v = vA[i];
+                maxA = fmaxf(maxA, fdot({v.x, v.y, v.z}, wa.x, wa.y, wa.z));
+                minA = fminf(minA, fdot(wba, v.x, v.y, v.z));
+                len = fmaxf(len, norm1(v.x, v.y, v.z));
             }
-            if (!sep && hB.num_faces > 0) {
-                float4 w = qt_rotate(oB, pb[fb]);
-                if (dot3(dc, w) < 0) w = scl4(w, -1.f);
-                project_group<QL>(vB, hB.num_vertices, sub, pB, oB, w, mn0, mx0);
-                project_group<QL>(vA, hA.num_vertices, sub, pA, oA, w, mn1, mx1);
-                sep = mx0 < mn1 || mx1 < mn0;
+            for (int i = sub; i < hB.num_vertices; i += QL) {
+                const float4 v = vB[i];
+                minB = fminf(minB, fdot(wab, v.x, v.y, v.z));
+                maxB = fmaxf(maxB, fdot({v.x, v.y, v.z}, wb.x, wb.y, wb.z));
+                len = fmaxf(len, norm1(v.x, v.y, v.z));
             }
+            const float lim = r.near + 2.f * NEAR_L * quad_max(len);
+            const float gapA = (quad_min(minB) + fdot(r.ta, wa.x, wa.y, wa.z)) - quad_max(maxA);
+            const float gapB = (quad_min(minA) + fdot(r.tb, wb.x, wb.y, wb.z)) - quad_max(maxB);
+            sep = r.ok && (gapA > lim * norm1(wa.x, wa.y, wa.z) ||
+                           gapB > lim * norm1(wb.x, wb.y, wb.z));
         }
     }
     // listed pairs: has_contact flags the wave-per-pair face pass, cand the
@@ -1902,7 +1996,7 @@ hipError_t launch_narrowphase(const DeviceWorld &d, const StepParams &p, hipStre
     uint32_t *work = (uint32_t *)d.cand_kv, *work_small = work + p.max_pairs;
     uint32_t *n_work = (uint32_t *)(d.counters + RB_CNT_FACE_WORK);
     uint32_t *n_small = (uint32_t *)(d.counters + RB_CNT_FACE_SMALL);
-    RB_LAUNCH(k_narrow_quick<QUICK_LANES>,
+    RB_LAUNCH(k_narrow_quick,
               dim3(((long long)p.max_pairs * QUICK_LANES + 255) / 256), dim3(256), 0, s,
               p.max_pairs, d.counters + RB_CNT_PAIRS, d.pairs, d.pos, d.quat, d.inv_mass, d.shape,
               d.hulls, d.verts, d.planes, d.has_contact, d.narrow_cand);

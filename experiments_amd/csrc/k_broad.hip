@@ -163,153 +163,271 @@ __global__ __launch_bounds__(256) void k_setup(
 }
 
 // First sorted index and occupancy bit of every occupied cell, and the AABBs
-// in sorted order (the pair search then reads a cell member's key and box at
-// one index).  occ[] was cleared by k_setup.
+// in sorted order with their keys and indices (the pair search reads a cell
+// member in one 32-byte piece).  occ[] was cleared by k_setup.
 __global__ void k_cell_start(const uint2 *__restrict__ kv, int n,
                              const float4 *__restrict__ aabb_min,
                              const float4 *__restrict__ aabb_max, uint32_t *__restrict__ cell_start,
-                             uint32_t *__restrict__ occ, float4 *__restrict__ smn,
-                             float4 *__restrict__ smx) {
+                             uint32_t *__restrict__ occ, float4 *__restrict__ boxes) {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     uint2 e = kv[s];
+    float4 mn = aabb_min[e.y], mx = aabb_max[e.y];
+    mn.w = __uint_as_float(e.x);
+    mx.w = __uint_as_float(e.y);
+    boxes[2 * (size_t)s] = mn;
+    boxes[2 * (size_t)s + 1] = mx;
     if (e.x == KEY_NONE) return;
-    smn[s] = aabb_min[e.y];
-    smx[s] = aabb_max[e.y];
     if (s == 0 || kv[s - 1].x != e.x) {
         cell_start[e.x] = (uint32_t)s;
         atomicOr(&occ[e.x >> 5], 1u << (e.x & 31u));
     }
 }
 
-constexpr int FP_BLOCK = 256;
-
-// LANES lanes per sorted entry; lane q walks the stencil cells
-// [q*C, q*C + C), C = ceil(27 / LANES), cells numbered z, then y, then x
-// from outermost to innermost, so a body's cells are searched in parallel
-// (32 lanes for few dense bodies, 1 for many).  The overlaps are numbered in
-// the order a serial search visits them (cells in stencil order, members in
-// sorted order, then the scene's large bodies in index order): a count pass,
-// a prefix over the lanes, and a store pass that keeps the first K in LDS.
-// The kept indices are distinct (a body sits in one cell), so the list is
-// ordered by rank.
-template <int LANES>
-__global__ __launch_bounds__(FP_BLOCK) void k_find_pairs(
-    int n, const uint2 *__restrict__ kv, const uint32_t *__restrict__ cell_start,
-    const uint32_t *__restrict__ occ, const float4 *__restrict__ smn,
-    const float4 *__restrict__ smx, const float4 *__restrict__ aabb_min,
-    const float4 *__restrict__ aabb_max, const int *__restrict__ large_list,
-    const int *__restrict__ large_first,
-    const int *__restrict__ large_num, GridP g, int K, int *__restrict__ body_slots,
-    uint32_t *__restrict__ pair_count, int *overflow) {
-    constexpr int ENTRIES = FP_BLOCK / LANES;
-    constexpr int C = (27 + LANES - 1) / LANES;
-    extern __shared__ int s_lists[];
-    const int lane = threadIdx.x & (LANES - 1);
-    const int slot = threadIdx.x / LANES;
-    const int seg = slot & (64 / LANES - 1);  // which LANES-lane segment of the wave
-    const int t = blockIdx.x * ENTRIES + slot;
-    // every exit below is uniform over the entry's lanes
-    if (t >= n) return;
-    const uint2 e = kv[t];
-    if (e.x == KEY_NONE) return;  // large body: k_large_count / k_large_write
-    const int i = (int)e.y;
-    int *dst = body_slots + (size_t)i * K;
-    // the list: in LDS for the lanes' rank sort (odd stride: the lists start
-    // in distinct banks); one lane keeps it in its own slots of body_slots,
-    // so its workgroups need no LDS (260 B per lane limited them to two per
-    // CU) and sort it there
-    int *lst = LANES == 1 ? dst : s_lists + slot * (K | 1);
-    const int sc = (int)(e.x >> g.cell_bits);
-    const float4 mn0 = smn[t], mx0 = smx[t];
-    int gp[3];
-    grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
-    const uint32_t sk = (uint32_t)sc << g.cell_bits;
-    uint32_t c = 0;
-    if constexpr (LANES == 1) {
-        // one lane: the occupancy bits of the 27 cells fetched together,
-        // then the occupied cells walked in order
-        uint32_t bits = 0;
-        const uint32_t reach = reachable_cells(mn0, mx0, g.inv_cell);
-#pragma unroll
-        for (int q = 0; q < 27; q++) {
-            const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
-            const uint32_t nkq = pos_hash(gp[0] + dx, gp[1] + dy, gp[2] + dz, g.dims) | sk;
-            bits |= ((occ[nkq >> 5] >> (nkq & 31u)) & 1u) << q;
+// Stencil rows: the three cells of a row along x are one key range (z and y
+// the outer strides of the key), so a wave that looks for the neighbours of
+// OWN sorted boxes lists the rows that hold members and its lanes walk one
+// listed row at a time, two members a read, taking the next one off the list
+// when they are through.  (A lane per entry or a lane per few cells, which
+// walked its own cells, left 64 lanes to wait for the longest of their chains
+// of dependent reads.)
+template <int OWN, int ROWS>
+struct RowsLDS {
+    float4 mn[OWN], mx[OWN];  // the wave's boxes, key and index in their w
+    uint32_t first[ROWS];     // a row's first key
+    uint32_t start[ROWS];     // its first member, 0: cell_start of the key
+    uint8_t own[ROWS];        // the box and, from bit 6, the cells after the first
+};
+// boxes: the AABBs in sorted order, two float4 each with the key and the index
+// in their w.  hits(m, c, o): the lanes of m hold a member, body c, that
+// overlaps the wave's box o; LOWER: only members of lower index than the box's.
+template <bool LOWER, int OWN, int ROWS, class Hits>
+__device__ __forceinline__ void walk_rows(int n, uint32_t total,
+                                          const uint32_t *__restrict__ cell_start,
+                                          const float4 *__restrict__ boxes,
+                                          RowsLDS<OWN, ROWS> &S, Hits hits) {
+    const uint32_t lane = threadIdx.x & 63;
+    wave_fence();
+    for (uint32_t p = lane; p < total; p += 64)
+        if (S.start[p] == 0u) S.start[p] = cell_start[S.first[p]];
+    wave_fence();
+    uint32_t at = 64u, u = 0u, last = 0u;
+    int o = 0, y = 0;
+    float4 a = mk4(0.f, 0.f, 0.f, 0.f), b = a;
+    bool walk = lane < total;
+    auto take = [&](uint32_t p) {
+        const uint32_t w = S.own[p];
+        o = (int)(w & 63u);
+        a = S.mn[o];
+        b = S.mx[o];
+        u = S.start[p];
+        last = S.first[p] + (w >> 6);
+        y = __float_as_int(b.w);
+    };
+    if (walk) take(lane);
+    while (__ballot(walk)) {
+        bool hit[2] = {false, false}, end = false;
+        int c[2] = {0, 0};
+        if (walk) {
+            const uint32_t v = u + 1u < (uint32_t)n ? u + 1u : u;
+            const float4 p0 = boxes[2 * (size_t)u], q0 = boxes[2 * (size_t)u + 1];
+            const float4 p1 = boxes[2 * (size_t)v], q1 = boxes[2 * (size_t)v + 1];
+            const bool in0 = __float_as_uint(p0.w) <= last;
+            const bool in1 = in0 && v != u && __float_as_uint(p1.w) <= last;
+            c[0] = __float_as_int(q0.w);
+            c[1] = __float_as_int(q1.w);
+            hit[0] = in0 && (!LOWER || c[0] < y) && aabb_overlap(a, b, p0, q0);
+            hit[1] = in1 && (!LOWER || c[1] < y) && aabb_overlap(a, b, p1, q1);
+            u += 2u;
+            end = !in1 || u >= (uint32_t)n;
         }
-        bits &= reach;
-        while (bits) {
-            const int q = __builtin_ctz(bits);
-            bits &= bits - 1u;
-            const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
-            const uint32_t nkq = pos_hash(gp[0] + dx, gp[1] + dy, gp[2] + dz, g.dims) | sk;
-            for (uint32_t u = cell_start[nkq]; u < (uint32_t)n; u++) {
-                const uint2 f = kv[u];
-                if (f.x != nkq) break;
-                if ((int)f.y < i && aabb_overlap(mn0, mx0, smn[u], smx[u])) {
-                    if (c < (uint32_t)K) lst[c] = (int)f.y;
-                    c++;
-                }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint64_t m = __ballot(hit[k]);
+            if (m) hits(m, c[k], o);
+        }
+        const uint64_t done = __ballot(end);
+        if (done) {
+            if (end) {
+                const uint32_t p = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(done >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)done, at));
+                walk = p < total;
+                if (walk) take(p);
             }
-        }
-    } else {
-        uint32_t nk[C], u0[C];
-        const uint32_t reach = reachable_cells(mn0, mx0, g.inv_cell);
-#pragma unroll
-        for (int k = 0; k < C; k++) {
-            const int q = lane * C + k;
-            nk[k] = 0;
-            u0[k] = (uint32_t)n;
-            if (q < 27 && ((reach >> q) & 1u)) {
-                const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
-                nk[k] = pos_hash(gp[0] + dx, gp[1] + dy, gp[2] + dz, g.dims) | sk;
-                if ((occ[nk[k] >> 5] >> (nk[k] & 31u)) & 1u) u0[k] = cell_start[nk[k]];
-            }
-        }
-        // one walk: a lane's first HITS overlaps stay in registers, so the
-        // members are walked again only by a lane that found more
-        constexpr int HITS = 4;
-        int hit[HITS] = {0, 0, 0, 0};
-        uint32_t cnt = 0;
-#pragma unroll
-        for (int k = 0; k < C; k++)
-            for (uint32_t u = u0[k]; u < (uint32_t)n; u++) {
-                const uint2 f = kv[u];
-                if (f.x != nk[k]) break;
-                if ((int)f.y < i && aabb_overlap(mn0, mx0, smn[u], smx[u])) {
-#pragma unroll
-                    for (int h = 0; h < HITS; h++)
-                        if (cnt == (uint32_t)h) hit[h] = (int)f.y;
-                    cnt++;
-                }
-            }
-        uint32_t incl = cnt;
-#pragma unroll
-        for (int o = 1; o < LANES; o <<= 1) {
-            uint32_t v = __shfl_up(incl, o, LANES);
-            if (lane >= o) incl += v;
-        }
-        c = __shfl(incl, LANES - 1, LANES);
-        uint32_t v = incl - cnt;
-        if (cnt <= (uint32_t)HITS) {
-#pragma unroll
-            for (int h = 0; h < HITS; h++)
-                if ((uint32_t)h < cnt && v + h < (uint32_t)K) lst[v + h] = hit[h];
-        } else {
-#pragma unroll
-            for (int k = 0; k < C; k++)
-                for (uint32_t u = u0[k]; u < (uint32_t)n && v < (uint32_t)K; u++) {
-                    const uint2 f = kv[u];
-                    if (f.x != nk[k]) break;
-                    if ((int)f.y < i && aabb_overlap(mn0, mx0, smn[u], smx[u])) lst[v++] = (int)f.y;
-                }
+            at += (uint32_t)__popcll(done);
         }
     }
+    wave_fence();
+}
+// Occupied cells among x - 1, x, x + 1 (bits 0 to 2) of the row at key b, from
+// the occupancy words of the outer two.  (Rows of two or more cells start at
+// even keys: at the grid's edge x still lies in the word of one of them.)
+__device__ __forceinline__ uint32_t row_bits(uint32_t wl, uint32_t wr, uint32_t b, uint32_t xl,
+                                             uint32_t x, uint32_t xr) {
+    const uint32_t wc = ((b | x) >> 5) == ((b | xl) >> 5) ? wl : wr;
+    return ((wl >> ((b | xl) & 31u)) & 1u) | ((wc >> ((b | x) & 31u)) & 1u) << 1 |
+           ((wr >> ((b | xr) & 31u)) & 1u) << 2;
+}
+// List a row's cells m (not wrapped: adjacent keys) of the wave's box `own`
+// behind the total rows before; every lane of the wave calls it.
+template <int OWN, int ROWS>
+__device__ __forceinline__ void list_row(RowsLDS<OWN, ROWS> &S, uint32_t &total, uint32_t m,
+                                         uint32_t b, uint32_t x, uint32_t xmask, int own,
+                                         uint32_t start) {
+    const uint64_t has = __ballot(m != 0u);
+    if (m) {
+        const uint32_t p = __builtin_amdgcn_mbcnt_hi(
+            (uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, total));
+        const uint32_t lo = (uint32_t)__builtin_ctz(m), hi = 31u - (uint32_t)__builtin_clz(m);
+        S.first[p] = b | ((x + lo - 1u) & xmask);
+        S.start[p] = start;
+        S.own[p] = (uint8_t)((uint32_t)own | (hi - lo) << 6);
+    }
+    total += (uint32_t)__popcll(has);
+}
+
+// The pair search: a wave per OWN sorted entries, 64 / OWN lanes an entry (16
+// entries where their waves fill the chip, below FP_FEW bodies 4: 64 us against
+// 95 at 65,537 hulls, 23.4 against 13.7 at 4,096 cubes).  The lanes list the
+// entry's stencil rows that hold members within reach, the wave walks them
+// (walk_rows), and an entry's overlaps with bodies of lower index go to its
+// list, the scene's large bodies after them, which is then ordered by rank.  An
+// entry with more than K overlaps keeps the first K that a serial search meets
+// (cells in stencil order, z then y then x, members in sorted order).  Bound by
+// the latency of the member reads.  (A lane per entry, walking the occupied
+// cells in turn: 276 us at 3.4M pairs of 4,096 scenes, now 183; 32 lanes an
+// entry, a cell each: 106 us at 65,537 hulls, now 64.)
+constexpr int FP_WAVES = 4;
+constexpr int FP_FEW = 1 << 14;
+constexpr int FP_LIST = RB_MAX_BODY_PAIRS;  // K is no larger
+template <int OWN>
+struct FindLDS {
+    RowsLDS<OWN, OWN * 9> rows;
+    uint32_t count[OWN];
+    int list[OWN][FP_LIST | 1];
+};
+
+// One wave: the first K overlaps of entry (mn0, mx0), index i, in the order of
+// a serial search, a stencil cell a lane.
+__device__ __forceinline__ void first_overlaps(int n, const uint32_t *__restrict__ cell_start,
+                                               const uint32_t *__restrict__ occ,
+                                               const float4 *__restrict__ boxes, const GridP &g,
+                                               float4 mn0, float4 mx0, int *__restrict__ lst,
+                                               int K) {
+    const int q = threadIdx.x & 63, i = __float_as_int(mx0.w);
+    const uint32_t key = __float_as_uint(mn0.w), sk = key >> g.cell_bits << g.cell_bits;
+    int gp[3];
+    grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
+    uint32_t nk = 0, u0 = (uint32_t)n, at = 0;
+    if (q < 27 && ((reachable_cells(mn0, mx0, g.inv_cell) >> q) & 1u)) {
+        nk = pos_hash(gp[0] + q % 3 - 1, gp[1] + (q / 3) % 3 - 1, gp[2] + q / 9 - 1, g.dims) | sk;
+        if ((occ[nk >> 5] >> (nk & 31u)) & 1u) u0 = cell_start[nk];
+    }
+    for (int pass = 0; pass < 2; pass++) {
+        uint32_t c = at;
+        for (uint32_t u = u0; u < (uint32_t)n; u++) {
+            const float4 p = boxes[2 * (size_t)u], m = boxes[2 * (size_t)u + 1];
+            if (__float_as_uint(p.w) != nk) break;
+            if (__float_as_int(m.w) < i && aabb_overlap(mn0, mx0, p, m)) {
+                if (pass && c < (uint32_t)K) lst[c] = __float_as_int(m.w);
+                c++;
+            }
+        }
+        if (pass) break;
+        uint32_t incl = c;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(incl, o, 64);
+            if (q >= o) incl += v;
+        }
+        at = incl - c;
+    }
+}
+
+template <int OWN>
+__global__ __launch_bounds__(64 * FP_WAVES) void k_find_pairs(
+    int n, const uint32_t *__restrict__ cell_start, const uint32_t *__restrict__ occ,
+    const float4 *__restrict__ boxes, const float4 *__restrict__ aabb_min,
+    const float4 *__restrict__ aabb_max, const int *__restrict__ large_list,
+    const int *__restrict__ large_first, const int *__restrict__ large_num, GridP g, int K,
+    int *__restrict__ body_slots, uint32_t *__restrict__ pair_count, int *overflow) {
+    constexpr int LANES = 64 / OWN;
+    __shared__ FindLDS<OWN> s_find[FP_WAVES];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    FindLDS<OWN> &S = s_find[w];
+    const int t0 = ((int)blockIdx.x * FP_WAVES + w) * OWN;
+    if (t0 >= n) return;
+    const int own = lane / LANES, sub = lane & (LANES - 1);
+    const int t = t0 + own;
+    float4 mn0 = mk4(0.f, 0.f, 0.f, 0.f), mx0 = mn0;
+    uint32_t key = KEY_NONE;  // (large bodies: k_large_count / k_large_write)
+    if (t < n) {
+        mn0 = boxes[2 * (size_t)t];
+        mx0 = boxes[2 * (size_t)t + 1];
+        key = __float_as_uint(mn0.w);
+    }
+    if (sub == 0) {
+        S.rows.mn[own] = mn0;
+        S.rows.mx[own] = mx0;
+        S.count[own] = 0u;
+    }
+    const int i = __float_as_int(mx0.w);
+    // the entry's rows sub, sub + LANES, ..: their cells that hold members
+    // within reach (bit dx + 1)
+    constexpr int R = (9 + LANES - 1) / LANES;
+    const uint32_t xmask = (uint32_t)g.dims[0] - 1u;
+    uint32_t bits[R], base[R], wrap0 = 0u, wrap2 = 0u;
+    int gp[3] = {0, 0, 0};
+    grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
+    const uint32_t x = (uint32_t)gp[0], xl = (x - 1u) & xmask, xr = (x + 1u) & xmask;
+    {
+        const uint32_t reach = key != KEY_NONE ? reachable_cells(mn0, mx0, g.inv_cell) : 0u;
+        const uint32_t sk = key >> g.cell_bits << g.cell_bits;
+        uint32_t wl[R], wr[R];
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int r = sub + k * LANES;
+            bits[k] = r < 9 ? (reach >> (3 * r)) & 7u : 0u;
+            base[k] = sk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
+            wl[k] = bits[k] ? occ[(base[k] | xl) >> 5] : 0u;
+            wr[k] = bits[k] ? occ[(base[k] | xr) >> 5] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < R; k++) bits[k] &= row_bits(wl[k], wr[k], base[k], xl, x, xr);
+    }
+    // round 0: the rows; rounds 1 and 2: their cells wrapped round the grid's
+    // edge (x - 1 of cell 0, x + 1 of the last)
+    for (int round = 0; round < 3; round++) {
+        uint32_t total = 0;
+        bool more = false;
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const uint32_t edge = (x == 0u ? 1u : 0u) | (x == xmask ? 4u : 0u);
+            const uint32_t m = bits[k] & (round == 0 ? ~edge : round == 1 ? edge & 1u : edge & 4u);
+            more |= (bits[k] & edge) != 0u;
+            list_row(S.rows, total, m, base[k], x, xmask, own, 0u);
+        }
+        if (total)
+            walk_rows<true>(n, total, cell_start, boxes, S.rows, [&](uint64_t m, int c, int o) {
+                if ((m >> lane) & 1ull) {
+                    const uint32_t p = atomicAdd(&S.count[o], 1u);
+                    if (p < (uint32_t)K) S.list[o][p] = c;
+                }
+            });
+        if (__ballot(more) == 0ull) break;
+    }
+    wave_fence();
+    uint32_t c = S.count[own];
+    for (uint64_t over = __ballot(sub == 0 && c > (uint32_t)K); over; over &= over - 1ull) {
+        const int o = __builtin_ctzll(over) / LANES;
+        first_overlaps(n, cell_start, occ, boxes, g, S.rows.mn[o], S.rows.mx[o], S.list[o], K);
+    }
+    int *dst = body_slots + (size_t)i * K, *lst = S.list[own];
     if (large_num) {
-        const int l0 = large_first[sc], nl = large_num[sc];
+        const int sc = key != KEY_NONE ? (int)(key >> g.cell_bits) : -1;
+        const int l0 = sc >= 0 ? large_first[sc] : 0, nl = sc >= 0 ? large_num[sc] : 0;
         const uint64_t segmask = LANES == 64 ? ~0ull : ((1ull << LANES) - 1ull);
         for (int q0 = 0; q0 < nl; q0 += LANES) {
-            const int q = q0 + lane;
+            const int q = q0 + sub;
             bool hit = false, stop = false;
             int L = 0;
             if (q < nl) {
@@ -317,41 +435,29 @@ __global__ __launch_bounds__(FP_BLOCK) void k_find_pairs(
                 stop = L >= i;  // list sorted by index
                 hit = !stop && aabb_overlap(mn0, mx0, aabb_min[L], aabb_max[L]);
             }
-            const uint64_t hm = (__ballot(hit) >> (LANES * seg)) & segmask;
-            const uint64_t sm = (__ballot(stop) >> (LANES * seg)) & segmask;
+            const uint64_t hm = (__ballot(hit) >> (LANES * own)) & segmask;
+            const uint64_t sm = (__ballot(stop) >> (LANES * own)) & segmask;
             if (hit) {
-                uint32_t w = c + (uint32_t)__popcll(hm & ((1ull << lane) - 1ull));
-                if (w < (uint32_t)K) lst[w] = L;
+                const uint32_t p = c + (uint32_t)__popcll(hm & ((1ull << sub) - 1ull));
+                if (p < (uint32_t)K) lst[p] = L;
             }
             c += (uint32_t)__popcll(hm);
             if (sm) break;
         }
     }
     if (c > (uint32_t)K) {
-        if (lane == 0) atomicOr(overflow, (int)MI_RB_OVERFLOW_BODY_PAIRS);
+        if (sub == 0) atomicOr(overflow, (int)MI_RB_OVERFLOW_BODY_PAIRS);
         c = (uint32_t)K;
     }
-    if constexpr (LANES == 1) {
-        // insertion sort in place (distinct indices, a few per body)
-        for (uint32_t k = 1; k < c; k++) {
-            const int x = dst[k];
-            int m = (int)k - 1;
-            while (m >= 0 && dst[m] > x) {
-                dst[m + 1] = dst[m];
-                m--;
-            }
-            dst[m + 1] = x;
-        }
-    } else {
-        wave_sync();  // the list's LDS stores come before the other lanes' loads
-        for (uint32_t w = lane; w < c; w += LANES) {
-            const int j = lst[w];
-            uint32_t r = 0;
-            for (uint32_t k = 0; k < c; k++) r += lst[k] < j ? 1u : 0u;
-            dst[r] = j;
-        }
+    wave_fence();
+    // ordered by rank (a large body's entry has none)
+    for (uint32_t p = sub; p < c; p += LANES) {
+        const int j = lst[p];
+        uint32_t r = 0;
+        for (uint32_t k = 0; k < c; k++) r += lst[k] < j ? 1u : 0u;
+        dst[r] = j;
     }
-    if (lane == 0) pair_count[i] = c;
+    if (sub == 0 && key != KEY_NONE) pair_count[i] = c;
 }
 
 // Overflow list: pairs (x, j) of each large body x with every body j < x of
@@ -578,14 +684,10 @@ constexpr int HG_OWN = RB_HG_OWN, HG_REC = RB_HG_REC;
 constexpr int HG_WAVES = 4;
 // rows of an entry on the lowest of four levels: 5 of its own, 9 of each other
 constexpr int HG_ROWS = HG_OWN * 32;
-struct HGLDS {
-    float4 mn[HG_OWN], mx[HG_OWN];
-    uint32_t first[HG_ROWS];  // first cell's key and, from bit 30, the cells after it
-    uint32_t start[HG_ROWS];
-    uint8_t own[HG_ROWS];
-};
+using HGLDS = RowsLDS<HG_OWN, HG_ROWS>;
 
 // hits(m, c, y): the lanes of m hold a pair of bodies c and y
+// (as walk_rows calls it)
 template <class Hits>
 __device__ __forceinline__ void hg_search(int n, const uint32_t *__restrict__ cell_start,
                                           const uint32_t *__restrict__ occ,
@@ -646,14 +748,8 @@ __device__ __forceinline__ void hg_search(int n, const uint32_t *__restrict__ ce
         }
 #pragma unroll
         for (int r = 0; r < 9; r++) {
-            // (rows of cells start at a multiple of four, so their cell 0 and 1
-            // lie in one word, as do their last two)
-            const uint32_t xl = (gx - 1u) & xmask, xr = (gx + 1u) & xmask;
             const uint32_t b = lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
-            const uint32_t wc = ((b | gx) >> 5) == ((b | xl) >> 5) ? wl[r] : wr[r];
-            uint32_t m = ((wl[r] >> ((b | xl) & 31u)) & 1u) |
-                         ((wc >> ((b | gx) & 31u)) & 1u) << 1 |
-                         ((wr[r] >> ((b | xr) & 31u)) & 1u) << 2;
+            uint32_t m = row_bits(wl[r], wr[r], b, (gx - 1u) & xmask, gx, (gx + 1u) & xmask);
             m &= ok[0];
             if (sub == 0 && r == 4) m = (m & 4u) | (next == key ? 2u : 0u);
             rows |= m << (3 * r);
@@ -667,77 +763,18 @@ __device__ __forceinline__ void hg_search(int n, const uint32_t *__restrict__ ce
     for (int round = 0; round < 2; round++) {
         uint32_t total = 0;
 #pragma unroll
-        for (int r = 0; r < 9; r++) {
-            const uint32_t m = (rows >> (3 * r)) & 7u;
-            const uint64_t has = __ballot(m != 0u);
-            if (m) {
-                const uint32_t p = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(has >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)has, total));
-                const uint32_t b = lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims);
-                const uint32_t lo = (uint32_t)__builtin_ctz(m), hi = 31u - (uint32_t)__builtin_clz(m);
-                const uint32_t x = ((uint32_t)gp[0] + lo - 1u) & xmask;
-                S.first[p] = b | x | (hi - lo) << 30;
-                // (the own row starts after the entry itself)
-                S.start[p] = sub == 0 && r == 4 && round == 0 ? (uint32_t)t + 1u : 0u;
-                S.own[p] = (uint8_t)own;
-            }
-            total += (uint32_t)__popcll(has);
-        }
-        if (total) {
-            wave_fence();
-            for (uint32_t p = lane; p < total; p += 64)
-                if (S.start[p] == 0u) S.start[p] = cell_start[S.first[p] & 0x3fffffffu];
-            wave_fence();
-            uint32_t at = 64u, u = 0u, last = 0u;
-            int y = 0;
-            float4 a = mn0, b = mx0;
-            bool walk = (uint32_t)lane < total;
-            auto take = [&](uint32_t p) {
-                const uint32_t f = S.first[p];
-                const int o = (int)S.own[p];
-                a = S.mn[o];
-                b = S.mx[o];
-                u = S.start[p];
-                last = (f & 0x3fffffffu) + (f >> 30);
-                y = __float_as_int(b.w);
-            };
-            if (walk) take((uint32_t)lane);
-            while (__ballot(walk)) {
-                bool hit[2] = {false, false}, end = false;
-                int c[2] = {0, 0};
-                if (walk) {
-                    const uint32_t v = u + 1u < (uint32_t)n ? u + 1u : u;
-                    const float4 p0 = boxes[2 * (size_t)u], q0 = boxes[2 * (size_t)u + 1];
-                    const float4 p1 = boxes[2 * (size_t)v], q1 = boxes[2 * (size_t)v + 1];
-                    const bool in0 = __float_as_uint(p0.w) <= last;
-                    const bool in1 = in0 && v != u && __float_as_uint(p1.w) <= last;
-                    hit[0] = in0 && aabb_overlap(a, b, p0, q0);
-                    hit[1] = in1 && aabb_overlap(a, b, p1, q1);
-                    c[0] = __float_as_int(q0.w);
-                    c[1] = __float_as_int(q1.w);
-                    u += 2u;
-                    end = !in1 || u >= (uint32_t)n;
-                }
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const uint64_t m = __ballot(hit[k]);
-                    if (m) hits(m, c[k], y);
-                }
-                const uint64_t done = __ballot(end);
-                if (done) {
-                    if (end) {
-                        const uint32_t p = __builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(done >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)done, at));
-                        walk = p < total;
-                        if (walk) take(p);
-                    }
-                    at += (uint32_t)__popcll(done);
-                }
-            }
-        }
+        for (int r = 0; r < 9; r++)
+            // (the own row starts after the entry itself)
+            list_row(S, total, (rows >> (3 * r)) & 7u,
+                     lk | pos_hash(0, gp[1] + r % 3 - 1, gp[2] + r / 3 - 1, g.dims),
+                     (uint32_t)gp[0], xmask, own,
+                     sub == 0 && r == 4 && round == 0 ? (uint32_t)t + 1u : 0u);
+        if (total)
+            walk_rows<false>(n, total, cell_start, boxes, S, [&](uint64_t m, int c, int o) {
+                hits(m, c, __float_as_int(S.mx[o].w));
+            });
         rows = rest;
         if (__ballot(rest != 0u) == 0ull) break;
-        wave_fence();
     }
 }
 // A pair (x, y), x > y, belongs to body x.  The count pass keeps its wave's
@@ -1246,7 +1283,7 @@ hipError_t launch_cell_start(const DeviceWorld &d, const StepParams &p, hipStrea
     const int n = p.n_bodies;
     if (n == 0) return hipSuccess;
     RB_LAUNCH(k_cell_start, dim3((n + 255) / 256), dim3(256), 0, s, d.kv, n, d.aabb_min,
-                       d.aabb_max, d.cell_start, d.occ, d.smn, d.smx);
+                       d.aabb_max, d.cell_start, d.occ, d.boxes);
     return rb_launch_status();
 }
 
@@ -1254,17 +1291,15 @@ hipError_t launch_find_pairs(const DeviceWorld &d, const StepParams &p, hipStrea
     int n = p.n_bodies;
     if (n == 0) return hipSuccess;
     int K = p.max_pairs_per_body;
-    // 32 lanes per body while the bodies alone do not fill the chip, else
-    // one lane per body (its cells walked in turn)
-    const int lanes = n < (1 << 18) ? 32 : 1;
-    const int entries = FP_BLOCK / lanes;
-    size_t lds = lanes == 1 ? 0 : sizeof(int) * (size_t)entries * (K | 1);
-    auto kern = lanes == 32 ? k_find_pairs<32> : k_find_pairs<1>;
-    RB_LAUNCH(kern, dim3((n + entries - 1) / entries), dim3(FP_BLOCK), lds, s, n,
-                       d.kv, d.cell_start, d.occ, d.smn, d.smx, d.aabb_min, d.aabb_max,
-                       d.large_list,
-                       p.n_large ? d.large_first : nullptr, p.n_large ? d.large_num : nullptr,
-                       grid_of(p), K, d.body_slots, d.pair_count, d.counters + RB_CNT_OVERFLOW);
+    auto find = [&](auto kern, int own) {
+        const int entries = FP_WAVES * own;
+        RB_LAUNCH(kern, dim3((n + entries - 1) / entries), dim3(64 * FP_WAVES), 0, s, n,
+                  d.cell_start, d.occ, d.boxes, d.aabb_min, d.aabb_max, d.large_list,
+                  p.n_large ? d.large_first : nullptr, p.n_large ? d.large_num : nullptr,
+                  grid_of(p), K, d.body_slots, d.pair_count, d.counters + RB_CNT_OVERFLOW);
+    };
+    if (n < FP_FEW) find(k_find_pairs<4>, 4);
+    else find(k_find_pairs<16>, 16);
     if (p.n_large > 0) {
         dim3 g(p.n_large, p.large_chunks);
         RB_LAUNCH(k_large_count, g, dim3(256), 0, s, d.large_list, d.scene,

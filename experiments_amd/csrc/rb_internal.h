@@ -62,6 +62,7 @@ struct Contact4 {
 static_assert(sizeof(Contact4) == 96, "Contact4 layout");
 
 // Limits of the wave-per-pair narrowphase.
+#define RB_MAX_BODY_PAIRS 64  // most pairs listed per body
 #define RB_MAX_HULL_VERTS 64
 #define RB_MAX_HULL_FACES 64
 #define RB_MAX_FACE_VERTS 64
@@ -146,7 +147,7 @@ struct DeviceWorld {
     uint32_t *cell_start;
     uint32_t *occ;               // occupancy bit per cell key, cleared by k_setup
     int occ_words;
-    float4 *smn, *smx;           // AABBs in sorted key order
+    float4 *boxes;               // AABBs in sorted key order, two float4 each: key, index in w
     int *body_slots;             // max_pairs_per_body per body
     int *large_slots;
     uint32_t *pair_count, *pair_off;

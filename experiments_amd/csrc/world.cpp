@@ -362,8 +362,7 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.cell_start, ncells));
     d.occ_words = (int)(ncells / 32 + 1);
     RB_CHECK(w.alloc(&d.occ, (size_t)d.occ_words));
-    RB_CHECK(w.alloc(&d.smn, n));
-    RB_CHECK(w.alloc(&d.smx, n));
+    RB_CHECK(w.alloc(&d.boxes, 2 * (size_t)n));
     RB_CHECK(w.alloc(&d.body_slots, (size_t)n * K));
     RB_CHECK(w.alloc(&d.pair_count, n));
     RB_CHECK(w.alloc(&d.pair_off, n));
@@ -623,7 +622,7 @@ extern "C" void mi_rb_config_reference(mi_rb_config *c) {
 extern "C" mi_rb_status mi_rb_create(const mi_rb_config *cfg, void **out_world) {
     if (!cfg || !out_world) return MI_RB_INVALID_ARG;
     if (cfg->max_bodies <= 0 || cfg->max_pairs <= 0 || cfg->max_contacts <= 0 ||
-        cfg->max_pairs_per_body <= 0 || cfg->max_pairs_per_body > 64 || cfg->dt <= 0.f ||
+        cfg->max_pairs_per_body <= 0 || cfg->max_pairs_per_body > RB_MAX_BODY_PAIRS || cfg->dt <= 0.f ||
         cfg->solver_iterations < 0 || cfg->solver_iterations > RB_MAX_SWEEPS || cfg->sat_mode < 0 ||
         cfg->sat_mode > 1 || cfg->reduction_mode < 0 || cfg->reduction_mode > 1)
         return MI_RB_INVALID_ARG;

@@ -1,0 +1,67 @@
+"""The step's pair search: dense clusters whose bodies have from none to over a
+hundred overlaps, with room for 1 to 64 a body, in grids of 4 to 64 cells an
+axis (wrapped), alone (4 entries a wave) and among so many bodies that 16
+entries share a wave.  A body's pairs are the first ones of a serial search:
+stencil cells in z, y, x order, members in sorted order, large bodies last."""
+import numpy as np
+import pytest
+
+from experiments_amd import _lib as L
+from experiments_amd import scenes
+from oracle.step import Snapshot, oracle_broadphase
+
+pytestmark = pytest.mark.gpu
+
+
+def expected(s, mn, mx, skv, pairs, room):
+    """The oracle's pairs, each body's cut to the first `room` found."""
+    dims, inv = s.params["dims"], np.float32(s.params["inv_cell"])
+    place = np.empty(len(skv), np.int64)
+    place[skv[:, 1]] = np.arange(len(skv))
+    cell = np.floor((mn[:, :3] + mx[:, :3]) * np.float32(0.5) * inv).astype(np.int64)
+    kept, over = [], False
+    lists = np.split(pairs, np.nonzero(np.diff(pairs[:, 0]))[0] + 1)
+    for p in lists:
+        if len(p) > room:
+            over = True
+            i, j = p[0, 0], p[:, 1]
+            d = (cell[j] - cell[i] + 1) % np.array(dims)
+            large = np.asarray(s.is_large)[j] != 0
+            assert d[~large].max() <= 2
+            d[large] = 3
+            order = np.lexsort((place[j], d[:, 0], d[:, 1], d[:, 2]))
+            p = p[np.sort(order[:room])]
+        kept.append(p)
+    return np.concatenate(kept), over
+
+
+@pytest.mark.parametrize("room,dims,others", [
+    (room, dims, 0) for room in (1, 20, 63, 64) for dims in ((4, 4, 4), (8, 4, 16), (64, 64, 64))
+] + [(20, (64, 64, 64), 131072), (64, (64, 64, 64), 131072)])
+def test_first_pairs(room, dims, others):
+    rng = np.random.default_rng(room)
+    sc = scenes.Scene("cluster", iterations=1)
+    sc.shapes = [scenes.cube_points(0.5), scenes.box_points(400.0, 1.0, 400.0)]
+    at = np.concatenate([rng.uniform(-1.6, 1.6, (260, 3)), rng.uniform(-4.0, 4.0, (77, 3))])
+    if others:
+        g = np.arange(others)
+        far = np.stack([g % 64, g // 64 % 64, g // 4096], 1) * 2.2 + [8.0, 0.0, 8.0]
+        at = np.concatenate([at, far])
+    q = rng.normal(size=(len(at), 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    if not others:
+        sc.add(0.0, (0.0, -3.0, 0.0), (0.0, 0.0, 0.0, 1.0), 1)
+    for a, b in zip(at, q):
+        sc.add(1.0, tuple(a), tuple(b), 0)
+    w = scenes.build_world(sc, max_pairs_per_body=room, max_pairs=1 << 20, max_contacts=1 << 14,
+                           grid_dims=dims)
+    s = Snapshot(w)
+    w.step_partial(L.STAGE_PAIRS)
+    mn, mx, skv, pairs = oracle_broadphase(s)
+    per_body = np.bincount(pairs[:, 0])
+    assert per_body.max() > 100
+    ref, over = expected(s, mn, mx, skv, pairs, room)
+    assert np.array_equal(w.pairs(), ref)
+    assert over
+    assert bool(w.stats()["overflow_flags"] & L.OVERFLOW_BODY_PAIRS) == over
+    w.close()

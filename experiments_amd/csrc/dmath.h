@@ -39,9 +39,12 @@ __device__ __forceinline__ float4 qt_mul(float4 a, float4 b) {
     return mk4(c.x + tx, c.y + ty, c.z + tz, a.w * b.w - dot3(a, b));
 }
 __device__ __forceinline__ float4 qt_inv(float4 q) { return mk4(-q.x, -q.y, -q.z, q.w); }
+// qt_mul(qt_mul(q, (v, 0)), qt_inv(q)), without the terms that the zero makes
+// zero (8 of 49 operations)
 __device__ __forceinline__ float4 qt_rotate(float4 q, float4 v) {
-    float4 vc = mk4(v.x, v.y, v.z, 0.f);
-    return qt_mul(qt_mul(q, vc), qt_inv(q));
+    float4 c = cross3(q, v);
+    float4 t = mk4(c.x + q.w * v.x, c.y + q.w * v.y, c.z + q.w * v.z, -dot3(q, v));
+    return qt_mul(t, qt_inv(q));
 }
 __device__ __forceinline__ float4 qt_inv_rotate(float4 q, float4 v) {
     return qt_rotate(qt_inv(q), v);

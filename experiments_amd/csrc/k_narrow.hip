@@ -28,30 +28,67 @@ using namespace rb;
 
 namespace {
 
-// lexicographic (value, index) reductions over the wave
+// A 16-lane row's reductions read the other lane's value through DPP: lane ^ 1
+// and lane ^ 2 of the quad, then the mirrored lane of 8 and of 16 (whose quads
+// hold their results already), which takes no LDS; across rows by shuffles.
+// (With the shorter rotation 65,537 32-vertex hulls' clip pass 422 -> 406 us,
+// their face pass 136 -> 131.)
+constexpr int DPP_X1 = 0xb1, DPP_X2 = 0x4e, DPP_MIRROR8 = 0x141, DPP_MIRROR16 = 0x140;
+template <int CTRL>
+__device__ __forceinline__ int dpp(int x) {
+    return __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __int_as_float(dpp<CTRL>(__float_as_int(x)));
+}
+// by value, component by component (an array or an address would be memory)
+__device__ __forceinline__ float4 pick4(bool c, float4 a, float4 b) {
+    return mk4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
+}
+// lexicographic (value, index) minimum and maximum
+__device__ __forceinline__ void take_min(float &d, int &idx, float od, int oi) {
+    if (od < d || (od == d && oi < idx)) { d = od; idx = oi; }
+}
+__device__ __forceinline__ void take_max(float &d, int &idx, float od, int oi) {
+    if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
+}
+__device__ __forceinline__ void row_argmin(float &d, int &idx) {
+    take_min(d, idx, dpp<DPP_X1>(d), dpp<DPP_X1>(idx));
+    take_min(d, idx, dpp<DPP_X2>(d), dpp<DPP_X2>(idx));
+    take_min(d, idx, dpp<DPP_MIRROR8>(d), dpp<DPP_MIRROR8>(idx));
+    take_min(d, idx, dpp<DPP_MIRROR16>(d), dpp<DPP_MIRROR16>(idx));
+}
+__device__ __forceinline__ void row_argmax(float &d, int &idx) {
+    take_max(d, idx, dpp<DPP_X1>(d), dpp<DPP_X1>(idx));
+    take_max(d, idx, dpp<DPP_X2>(d), dpp<DPP_X2>(idx));
+    take_max(d, idx, dpp<DPP_MIRROR8>(d), dpp<DPP_MIRROR8>(idx));
+    take_max(d, idx, dpp<DPP_MIRROR16>(d), dpp<DPP_MIRROR16>(idx));
+}
+__device__ __forceinline__ int row8_max_i32(int v) {
+    v = max(v, dpp<DPP_X1>(v));
+    v = max(v, dpp<DPP_X2>(v));
+    return max(v, dpp<DPP_MIRROR8>(v));
+}
+__device__ __forceinline__ int row_max_i32(int v) {
+    v = row8_max_i32(v);
+    return max(v, dpp<DPP_MIRROR16>(v));
+}
+// the same over the wave
 __device__ __forceinline__ void wave_argmin(float &d, int &idx) {
+    row_argmin(d, idx);
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        float od = __shfl_xor(d, o, 64);
-        int oi = __shfl_xor(idx, o, 64);
-        if (od < d || (od == d && oi < idx)) { d = od; idx = oi; }
-    }
+    for (int o = 16; o <= 32; o <<= 1) take_min(d, idx, __shfl_xor(d, o, 64), __shfl_xor(idx, o, 64));
 }
 __device__ __forceinline__ void wave_argmax(float &d, int &idx) {
+    row_argmax(d, idx);
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        float od = __shfl_xor(d, o, 64);
-        int oi = __shfl_xor(idx, o, 64);
-        if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
-    }
+    for (int o = 16; o <= 32; o <<= 1) take_max(d, idx, __shfl_xor(d, o, 64), __shfl_xor(idx, o, 64));
 }
 __device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        int ov = __shfl_xor(v, o, 64);
-        v = ov > v ? ov : v;
-    }
-    return v;
+    v = row_max_i32(v);
+    v = max(v, __shfl_xor(v, 16, 64));
+    return max(v, __shfl_xor(v, 32, 64));
 }
 
 // Hull vertices are read through the scalar data cache: every lane needs
@@ -188,12 +225,17 @@ constexpr int NP_BLOCK = 64;
 // the low 6 bits (ties and the dropped bits go to the higher lane); a NaN
 // projection ranks below every number and a lane without a vertex below all
 __device__ __forceinline__ int probe_key(float v, int lane, bool valid) {
-    int f = __float_as_int(v);
-    f = f >= 0 ? f : (f ^ 0x7fffffff);
-    if (!(v >= -FLT_MAX)) f = INT_MIN + 64;
-    if (f < INT_MIN + 64) f = INT_MIN + 64;
-    if (!valid) f = INT_MIN;
-    return (f & ~63) | lane;
+    int f = __float_as_int(fmaxf(v, -FLT_MAX));
+    f ^= (f >> 31) & 0x7fffffff;
+    return ((valid ? f : INT_MIN) & ~63) | lane;
+}
+// probe k's direction is n + t (a e1 + b e2); the projection of a vertex on it
+// from its projections on the three
+__device__ __forceinline__ float probe_dot(int k, float dn, float d1, float d2) {
+    const float t = k <= 4 ? 0.35f : 0.8f * 0.70710678f;
+    if (k == 0) return dn;
+    if (k <= 4) return k & 1 ? fmaf(k & 2 ? -t : t, d1, dn) : fmaf(k & 2 ? -t : t, d2, dn);
+    return fmaf(k & 1 ? t : -t, d1, fmaf(k & 2 ? t : -t, d2, dn));
 }
 // probe directions of the clip pass's second edge-axis bound: dc, four at
 // 0.35 and four at 0.8 (rotated by 45 degrees) around it
@@ -221,30 +263,7 @@ __device__ __forceinline__ void group_sync() {
 __device__ __forceinline__ uint32_t group_ballot(bool x, int gbase) {
     return (uint32_t)((__ballot(x) >> gbase) & ((1ull << SG) - 1ull));
 }
-__device__ __forceinline__ void group_argmin(float &d, int &idx) {
-#pragma unroll
-    for (int o = SG / 2; o >= 1; o >>= 1) {
-        float od = __shfl_xor(d, o, 64);
-        int oi = __shfl_xor(idx, o, 64);
-        if (od < d || (od == d && oi < idx)) { d = od; idx = oi; }
-    }
-}
-__device__ __forceinline__ void group_argmax(float &d, int &idx) {
-#pragma unroll
-    for (int o = SG / 2; o >= 1; o >>= 1) {
-        float od = __shfl_xor(d, o, 64);
-        int oi = __shfl_xor(idx, o, 64);
-        if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
-    }
-}
-__device__ __forceinline__ int group_max_i32(int v) {
-#pragma unroll
-    for (int o = SG / 2; o >= 1; o >>= 1) {
-        int ov = __shfl_xor(v, o, 64);
-        v = ov > v ? ov : v;
-    }
-    return v;
-}
+static_assert(SG == 16, "a group is a DPP row");
 // log2 of the lanes per axis for a batch of cnt <= SG axes
 __device__ __forceinline__ int group_lanes_log2(int cnt) {
     return cnt > 8 ? 0 : cnt > 4 ? 1 : cnt > 2 ? 2 : cnt > 1 ? 3 : 4;
@@ -378,39 +397,26 @@ __global__ __launch_bounds__(256) void k_narrow_special(
 // matrix (3.4M pairs of small hulls 258 -> 185 us, 635k pairs of 32-vertex
 // hulls 97 -> 76).
 constexpr int QUICK_LANES = 4;
-template <int PERM>
-__device__ __forceinline__ float quad_f(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), PERM, 0xf, 0xf, true));
-}
-// lane ^ 1 and lane ^ 2 of the quad; quad_from: every lane gets lane K's value
-constexpr int QUAD_X1 = 0xb1, QUAD_X2 = 0x4e;
-template <int K>
-__device__ __forceinline__ int quad_from(int x) {
-    return __builtin_amdgcn_mov_dpp(x, K * 0x55, 0xf, 0xf, true);
-}
-template <int K>
-__device__ __forceinline__ float quad_from(float x) {
-    return quad_f<K * 0x55>(x);
+// every lane of the quad gets lane K's value
+template <int K, class T>
+__device__ __forceinline__ T quad_from(T x) {
+    return dpp<K * 0x55>(x);
 }
 template <int K>
 __device__ __forceinline__ float4 quad_from(float4 v) {
     return mk4(quad_from<K>(v.x), quad_from<K>(v.y), quad_from<K>(v.z), quad_from<K>(v.w));
 }
 __device__ __forceinline__ float quad_max(float x) {
-    x = fmaxf(x, quad_f<QUAD_X1>(x));
-    return fmaxf(x, quad_f<QUAD_X2>(x));
+    x = fmaxf(x, dpp<DPP_X1>(x));
+    return fmaxf(x, dpp<DPP_X2>(x));
 }
 __device__ __forceinline__ float quad_min(float x) {
-    x = fminf(x, quad_f<QUAD_X1>(x));
-    return fminf(x, quad_f<QUAD_X2>(x));
+    x = fminf(x, dpp<DPP_X1>(x));
+    return fminf(x, dpp<DPP_X2>(x));
 }
 __device__ __forceinline__ void quad_argmax(float &d, int &idx) {
-    float od = quad_f<QUAD_X1>(d);
-    int oi = __builtin_amdgcn_mov_dpp(idx, QUAD_X1, 0xf, 0xf, true);
-    if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
-    od = quad_f<QUAD_X2>(d);
-    oi = __builtin_amdgcn_mov_dpp(idx, QUAD_X2, 0xf, 0xf, true);
-    if (od > d || (od == d && oi < idx)) { d = od; idx = oi; }
+    take_max(d, idx, dpp<DPP_X1>(d), dpp<DPP_X1>(idx));
+    take_max(d, idx, dpp<DPP_X2>(d), dpp<DPP_X2>(idx));
 }
 struct V3 { float x, y, z; };
 __device__ __forceinline__ float fdot(V3 a, float x, float y, float z) {
@@ -768,6 +774,14 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face(
     }
 }
 
+// centre A - centre B of a group's pair: the row's lower 8 lanes rotate A's
+// centre, the upper 8 B's
+__device__ __forceinline__ float4 row_centre_diff(bool hi8, float4 center, float4 p, float4 o) {
+    const float4 c = xform(center, p, o);
+    const float4 d = mk4(dpp<DPP_MIRROR16>(c.x), dpp<DPP_MIRROR16>(c.y), dpp<DPP_MIRROR16>(c.z), 0.f);
+    return sub4(pick4(hi8, d, c), pick4(hi8, c, d));
+}
+
 // Pass 1 for pairs of two small hulls (listed by pass 0 after the others):
 // SG lanes per pair, four pairs per wave.  The face axes (at most 32) are
 // those of the wave kernel's plain path, built and projected with the same
@@ -801,7 +815,9 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
         if (gl < nvA) sVA[grp][gl] = verts[hA.vertex_offset + gl];
         if (gl < nvB) sVB[grp][gl] = verts[hB.vertex_offset + gl];
         group_sync();
-        const float4 dc = sub4(xform(hA.center, pA, oA), xform(hB.center, pB, oB));
+        const bool hi8 = gl >= SG_VERTS;
+        const float4 dc = row_centre_diff(hi8, pick4(hi8, hB.center, hA.center),
+                                          pick4(hi8, pB, pA), pick4(hi8, oB, oA));
         const int nfA = hA.num_faces, nf = nfA + hB.num_faces;
         bool sep_found = false;
         float best = FLT_MAX;
@@ -831,7 +847,7 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
             if (gl == 0) { has_contact[p] = 0; cand[p] = 0; }
             continue;
         }
-        group_argmin(best, best_ax);
+        row_argmin(best, best_ax);
         if (gl == 0) {
             cand[p] = 1;
             face_best[p] = make_int4(__float_as_int(best), best_ax, hA.num_edges * hB.num_edges, 1);
@@ -952,20 +968,18 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip(
             const float4 wA4 = lane < hA.num_vertices
                                    ? add4(qt_rotate(oA, verts[hA.vertex_offset + lane]), dAB)
                                    : mk4(0.f, 0.f, 0.f, 0.f);
+            const float bn = dot3(wB4, n), b1 = dot3(wB4, e1), b2 = dot3(wB4, e2);
+            const float an = -dot3(wA4, n), a1 = -dot3(wA4, e1), a2 = -dot3(wA4, e2);
 #pragma unroll
             for (int k = 0; k < NPROBE; k++) {
-                const float t = k == 0 ? 0.f : (k <= 4 ? 0.35f : 0.8f * 0.70710678f);
-                const float a = k <= 4 ? ((k & 1) ? 1.f : 0.f) * ((k & 2) ? -1.f : 1.f) : ((k & 1) ? 1.f : -1.f);
-                const float b = k <= 4 ? ((k & 1) ? 0.f : 1.f) * ((k & 2) ? -1.f : 1.f) : ((k & 2) ? 1.f : -1.f);
-                const float4 u = add4(n, add4(scl4(e1, t * a), scl4(e2, t * b)));
                 // Any vertex gives a valid bound, so the furthest one is
                 // found on one ordered integer key per lane (the projection's
                 // ordered bits with the lane in the low 6 bits); a NaN
                 // projection counts as none and lanes without a vertex lose.
-                const int ib =
-                    wave_max_i32(probe_key(dot3(wB4, u), lane, lane < hB.num_vertices)) & 63;
-                const int ia =
-                    wave_max_i32(probe_key(-dot3(wA4, u), lane, lane < hA.num_vertices)) & 63;
+                const int ib = wave_max_i32(probe_key(probe_dot(k, bn, b1, b2), lane,
+                                                      lane < hB.num_vertices)) & 63;
+                const int ia = wave_max_i32(probe_key(probe_dot(k, an, a1, a2), lane,
+                                                      lane < hA.num_vertices)) & 63;
                 if (lane == ib) sProbe[k] = wB4;
                 if (lane == ia) sProbe[NPROBE + k] = wA4;
             }
@@ -1365,6 +1379,15 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip(
 // arithmetic and the same tie rules, so the manifold is identical; the lanes
 // of a group take the same branches, reductions stay inside the group, and
 // LDS is the group's own.
+//
+// Bound by its instructions (the vector units are busy throughout, at four
+// waves a SIMD), most of them rotations that the reference's operation order
+// fixes.  A hull's points fill at most 8 lanes of a group, so both hulls'
+// centres, vertices and faces' corners are rotated together, a hull a half, and
+// so are the probes' maxima taken; the edges of both are one list (553k
+// contacts: 677 -> 614 us, with the shorter rotation and the reductions
+// through DPP; the face pass of small hulls 280 -> 223).  Listing the edge rows
+// that the first bound drops whole, as pass 2 does, gained nothing here (616).
 
 struct SmallClipLDS {
     float4 ea[SG_EDGES], eb[SG_EDGES];
@@ -1410,10 +1433,16 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
         pB.w = 0.f;
         const int nvA = hA.num_vertices, nvB = hB.num_vertices;
         group_sync();  // the previous candidate's reads of S are done
-        if (gl < hA.num_edges) S.ea[gl] = qt_rotate(oA, edges[hA.edge_offset + gl]);
-        if (gl + SG < hA.num_edges) S.ea[gl + SG] = qt_rotate(oA, edges[hA.edge_offset + gl + SG]);
-        if (gl < hB.num_edges) S.eb[gl] = qt_rotate(oB, edges[hB.edge_offset + gl]);
-        if (gl + SG < hB.num_edges) S.eb[gl + SG] = qt_rotate(oB, edges[hB.edge_offset + gl + SG]);
+        // both hulls' edges, one list over the lanes
+        constexpr int ER = (2 * SG_EDGES + SG - 1) / SG;
+        const int neA = hA.num_edges, neAB = neA + hB.num_edges;
+        float4 ev[ER];
+#pragma unroll
+        for (int k = 0; k < ER; k++) {
+            const int e = gl + k * SG;
+            ev[k] = mk4(0.f, 0.f, 0.f, 0.f);
+            if (e < neAB) ev[k] = edges[e < neA ? hA.edge_offset + e : hB.edge_offset + e - neA];
+        }
         if (gl < nvA) S.va[gl] = verts[hA.vertex_offset + gl];
         if (gl < nvB) S.vb[gl] = verts[hB.vertex_offset + gl];
         // the faces' planes and (first index, count) records are read after
@@ -1423,9 +1452,23 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
         if (gl < hB.num_faces) S.pb[gl] = planes[hB.face_offset + gl];
         const int2 fiA_l = gl < hA.num_faces ? face_index[hA.face_offset + gl] : make_int2(0, 0);
         const int2 fiB_l = gl < hB.num_faces ? face_index[hB.face_offset + gl] : make_int2(0, 0);
+#pragma unroll
+        for (int k = 0; k < ER; k++) {
+            const int e = gl + k * SG;
+            if (e < neAB) {
+                const float4 r = qt_rotate(pick4(e < neA, oA, oB), ev[k]);
+                if (e < neA) S.ea[e] = r;
+                else S.eb[e - neA] = r;
+            }
+        }
         group_sync();
 
-        const float4 dc = sub4(xform(hA.center, pA, oA), xform(hB.center, pB, oB));
+        // what is rotated for a point of each hull, the row's lower 8 lanes do
+        // for A and the upper 8 for B (a hull has at most 8 vertices)
+        const bool hi8 = gl >= SG_VERTS;
+        const int g8 = gl & (SG_VERTS - 1);
+        const float4 oH = pick4(hi8, oB, oA), pH = pick4(hi8, pB, pA);
+        const float4 dc = row_centre_diff(hi8, pick4(hi8, hB.center, hA.center), pH, oH);
         float best = FLT_MAX;
         int best_ax = 0x7fffffff;
         const int nf = hA.num_faces + hB.num_faces;
@@ -1442,19 +1485,19 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
                                                                  : mk4(0.f, 1.f, 0.f, 0.f)));
             float4 e2 = cross3(n, e1);
             const float4 dAB = sub4(pA, pB);
-            const float4 wB4 = gl < nvB ? qt_rotate(oB, S.vb[gl]) : mk4(0.f, 0.f, 0.f, 0.f);
-            const float4 wA4 = gl < nvA ? add4(qt_rotate(oA, S.va[gl]), dAB) : mk4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int k = 0; k < NPROBE; k++) {
-                const float t = k == 0 ? 0.f : (k <= 4 ? 0.35f : 0.8f * 0.70710678f);
-                const float a2 = k <= 4 ? ((k & 1) ? 1.f : 0.f) * ((k & 2) ? -1.f : 1.f) : ((k & 1) ? 1.f : -1.f);
-                const float b2 = k <= 4 ? ((k & 1) ? 0.f : 1.f) * ((k & 2) ? -1.f : 1.f) : ((k & 2) ? 1.f : -1.f);
-                const float4 u = add4(n, add4(scl4(e1, t * a2), scl4(e2, t * b2)));
-                const int ib = group_max_i32(probe_key(dot3(wB4, u), gl, gl < nvB)) & (SG - 1);
-                const int ia = group_max_i32(probe_key(-dot3(wA4, u), gl, gl < nvA)) & (SG - 1);
-                if (gl == ib) S.pts[k] = wB4;
-                if (gl == ia) S.pts[NPROBE + k] = wA4;
+            const bool has = g8 < (hi8 ? nvB : nvA);
+            float4 wv = mk4(0.f, 0.f, 0.f, 0.f);
+            if (has) {
+                wv = qt_rotate(oH, hi8 ? S.vb[g8] : S.va[g8]);
+                if (!hi8) wv = add4(wv, dAB);
             }
+            const float sg = hi8 ? 1.f : -1.f;
+            const float dn = sg * dot3(wv, n), d1 = sg * dot3(wv, e1), d2 = sg * dot3(wv, e2);
+            float4 *probes = S.pts + (hi8 ? 0 : NPROBE);
+#pragma unroll
+            for (int k = 0; k < NPROBE; k++)
+                if ((row8_max_i32(probe_key(probe_dot(k, dn, d1, d2), gl, has)) & 63) == gl)
+                    probes[k] = wv;
             group_sync();
         }
         const int nEB = hB.num_edges;
@@ -1561,25 +1604,23 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
             const int slot = gl >> lg, part = gl & ((1 << lg) - 1);
             project_axis(S.pq[slot < pn ? slot : 0], lg, part, slot < pn);
         }
-        group_argmin(best, best_ax);
+        row_argmin(best, best_ax);
         if (face_d < best || (face_d == best && fb0.y < best_ax)) { best = face_d; best_ax = fb0.y; }
         if (best_ax == 0x7fffffff || (edge_reject && best < 0.f)) {
             if (gl == 0) has_contact[p] = 0;
             continue;
         }
         float4 sep;
-        if (best_ax < hA.num_faces) {
-            sep = qt_rotate(oA, S.pa[best_ax]);
-            if (dot3(dc, sep) < 0) sep = scl4(sep, -1.f);
-        } else if (best_ax < nf) {
-            sep = qt_rotate(oB, S.pb[best_ax - hA.num_faces]);
-            if (dot3(dc, sep) < 0) sep = scl4(sep, -1.f);
+        if (best_ax < nf) {
+            const bool onA = best_ax < hA.num_faces;
+            sep = qt_rotate(pick4(onA, oA, oB),
+                            onA ? S.pa[best_ax] : S.pb[best_ax - hA.num_faces]);
         } else {
             const int k = best_ax - nf;
             const int f0 = k / nEB, f1 = k - f0 * nEB;
             sep = normalize3(cross3(S.ea[f0], S.eb[f1]));
-            if (dot3(dc, sep) < 0) sep = scl4(sep, -1.f);
         }
+        if (dot3(dc, sep) < 0) sep = scl4(sep, -1.f);
         if (dot3(neg4(dc), sep) > 0.0f) sep = neg4(sep);
 
         // ---- clipping: incident face of B, reference face of A ----
@@ -1590,7 +1631,7 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
             const float d = dot3(qt_rotate(oB, mk4(pl.x, pl.y, pl.z, 0.f)), sep);
             if (d > dB) { dB = d; fB = gl; }
         }
-        group_argmax(dB, fB);
+        row_argmax(dB, fB);
         float dA = FLT_MAX;
         int fA = 0x7fffffff;
         if (gl < hA.num_faces) {
@@ -1598,7 +1639,7 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
             const float d = dot3(qt_rotate(oA, mk4(pl.x, pl.y, pl.z, 0.f)), sep);
             if (d < dA) { dA = d; fA = gl; }
         }
-        group_argmin(dA, fA);
+        row_argmin(dA, fA);
         if (fB == 0x7fffffff || fA == 0x7fffffff) {
             if (gl == 0) has_contact[p] = 0;
             continue;
@@ -1606,19 +1647,23 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
         // fB, fA < SG_FACES: the group's lanes fB, fA hold those faces' records
         const int2 fiB = make_int2(__shfl(fiB_l.x, gbase + fB, 64), __shfl(fiB_l.y, gbase + fB, 64));
         int nin = fiB.y < SG_VERTS ? fiB.y : SG_VERTS;
-        if (gl < nin) S.poly[0][gl] = xform(S.vb[indices[fiB.x + gl]], pB, oB);
         const int2 fiA = make_int2(__shfl(fiA_l.x, gbase + fA, 64), __shfl(fiA_l.y, gbase + fA, 64));
         const float4 plA = S.pa[fA];
         const float4 wpn = qt_rotate(oA, mk4(plA.x, plA.y, plA.z, 0.f));
         float4 *sSide = S.pts;
         const int nside = fiA.y < SG_VERTS ? fiA.y : SG_VERTS;
-        if (gl < nside) {
-            const float4 va = S.va[indices[fiA.x + gl]];
-            const float4 vb = S.va[indices[fiA.x + (gl + 1) % fiA.y]];
-            const float4 we = qt_rotate(oA, sub4(va, vb));
-            const float4 pn4 = neg4(cross3(we, wpn));
-            const float4 wa = xform(va, pA, oA);
-            sSide[gl] = mk4(pn4.x, pn4.y, pn4.z, -dot3(wa, pn4));
+        // the reference face's corners and side planes, the incident polygon
+        if (g8 < (hi8 ? nin : nside)) {
+            const float4 v = hi8 ? S.vb[indices[fiB.x + g8]] : S.va[indices[fiA.x + g8]];
+            const float4 wv = xform(v, pH, oH);
+            if (hi8) {
+                S.poly[0][g8] = wv;
+            } else {
+                const float4 vb = S.va[indices[fiA.x + (g8 + 1) % fiA.y]];
+                const float4 we = qt_rotate(oA, sub4(v, vb));
+                const float4 pn4 = neg4(cross3(we, wpn));
+                sSide[g8] = mk4(pn4.x, pn4.y, pn4.z, -dot3(wv, pn4));
+            }
         }
         int cur = 0;
         bool poly_over = fiB.y > SG_VERTS || fiA.y > SG_VERTS;
@@ -1714,10 +1759,10 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
                 for (int k = 0; k < 4; k++) {
                     int ik = f[k] < FLT_MAX ? gl : 0x7fffffff;
                     float fk = f[k];
-                    group_argmin(fk, ik);
+                    row_argmin(fk, ik);
                     if (ik != 0x7fffffff) idx[k] = ik;
                 }
-                group_argmin(dw, iw);
+                row_argmin(dw, iw);
                 if (idx[0] != iw && idx[1] != iw && idx[2] != iw && idx[3] != iw) idx[0] = iw;
                 nr = 4;
             }
@@ -1738,7 +1783,7 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
                 for (int k = 0; k < 4; k++)
                     key[k] = (int)((__float_as_uint(f[k]) & 0xffffff00u) | (0xffu & (uint32_t)gl));
             }
-            for (int k = 0; k < 4; k++) idx[k] = group_max_i32(key[k]) & 0xff;
+            for (int k = 0; k < 4; k++) idx[k] = row_max_i32(key[k]) & 0xff;
             nr = 4;
         }
         if (gl == 0) {

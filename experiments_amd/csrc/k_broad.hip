@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
 #include <utility>
 
 #include "dmath.h"
@@ -541,43 +542,48 @@ __global__ __launch_bounds__(256) void k_large_write(
     }
 }
 
+// Lists into the pair array: EMIT_LANES lanes a body, whose list of a few
+// partners they read and write as one run; then, for the overflow-list bodies,
+// whose lists can hold a whole scene's worth, as many workgroups a body as its
+// scene's size can use, up to 32.  (3.4M pairs of 4,096 scenes: a thread a body
+// 88 us and 32 workgroups for each scene's ground 29 more, now 31; 16 for
+// each ground, mostly idle, 52.)
+constexpr int EMIT_LANES = 8;
 __global__ __launch_bounds__(256) void k_emit_pairs(
-    int n, const uint32_t *__restrict__ pair_count, const uint32_t *__restrict__ pair_off,
-    const int *__restrict__ body_slots, int K, const int *__restrict__ is_large,
-    const int *__restrict__ large_index, const int *__restrict__ large_off,
-    const int *__restrict__ large_slots, int max_pairs, int2 *__restrict__ pairs,
-    const uint32_t *total, int *num_pairs, int *overflow) {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x == 0) {
-        uint32_t tt = *total;
-        if (tt > (uint32_t)max_pairs) {
-            atomicOr(overflow, (int)MI_RB_OVERFLOW_PAIRS);
-            tt = (uint32_t)max_pairs;
+    int n, int body_blocks, int large_blocks, const uint32_t *__restrict__ pair_count,
+    const uint32_t *__restrict__ pair_off, const int *__restrict__ body_slots, int K,
+    const int *__restrict__ is_large, const int *__restrict__ large_list,
+    const int *__restrict__ large_off, const int *__restrict__ large_slots, int max_pairs,
+    int2 *__restrict__ pairs, const uint32_t *total, int *num_pairs, int *overflow) {
+    const int b = (int)blockIdx.x;
+    int x;
+    uint32_t k0, step;
+    const int *src;
+    if (b < body_blocks) {
+        if (b == 0 && threadIdx.x == 0) {
+            uint32_t tt = *total;
+            if (tt > (uint32_t)max_pairs) {
+                atomicOr(overflow, (int)MI_RB_OVERFLOW_PAIRS);
+                tt = (uint32_t)max_pairs;
+            }
+            *num_pairs = (int)tt;
         }
-        *num_pairs = (int)tt;
+        x = b * (256 / EMIT_LANES) + (int)threadIdx.x / EMIT_LANES;
+        if (x >= n) return;
+        if (is_large && is_large[x]) return;
+        k0 = threadIdx.x % EMIT_LANES;
+        step = EMIT_LANES;
+        src = body_slots + (size_t)x * K;
+    } else {
+        const int q = (b - body_blocks) / large_blocks;
+        x = large_list[q];
+        k0 = (uint32_t)((b - body_blocks) % large_blocks) * blockDim.x + threadIdx.x;
+        step = (uint32_t)large_blocks * blockDim.x;
+        src = large_slots + large_off[q];
     }
-    if (x >= n) return;
-    if (is_large && is_large[x]) return;  // long lists: k_emit_large
-    uint32_t c = pair_count[x], off = pair_off[x];
-    const int *src = body_slots + (size_t)x * K;
-    for (uint32_t k = 0; k < c; k++) {
-        uint32_t o = off + k;
-        if (o < (uint32_t)max_pairs) pairs[o] = make_int2(x, src[k]);
-    }
-}
-
-// Pair lists of the overflow-list bodies can hold a whole scene's worth of
-// partners: spread each one over a grid row of workgroups instead of one thread.
-__global__ __launch_bounds__(256) void k_emit_large(
-    const int *__restrict__ large_list, const uint32_t *__restrict__ pair_count,
-    const uint32_t *__restrict__ pair_off, const int *__restrict__ large_off,
-    const int *__restrict__ large_slots, int max_pairs, int2 *__restrict__ pairs) {
-    const int q = blockIdx.x;
-    const int x = large_list[q];
     const uint32_t c = pair_count[x], off = pair_off[x];
-    const int *src = large_slots + large_off[q];
-    for (uint32_t k = blockIdx.y * blockDim.x + threadIdx.x; k < c; k += gridDim.y * blockDim.x) {
-        uint32_t o = off + k;
+    for (uint32_t k = k0; k < c; k += step) {
+        const uint32_t o = off + k;
         if (o < (uint32_t)max_pairs) pairs[o] = make_int2(x, src[k]);
     }
 }
@@ -613,13 +619,18 @@ __global__ __launch_bounds__(256) void k_hg_hash(const float4 *__restrict__ mn,
                                                  const float4 *__restrict__ mx, int n, HGridP g,
                                                  uint2 *__restrict__ kv, uint32_t *__restrict__ counts,
                                                  uint32_t *__restrict__ cursor,
-                                                 uint32_t *__restrict__ big_n, int *overflow) {
+                                                 uint32_t *__restrict__ big_n, int *overflow,
+                                                 float4 *__restrict__ raw) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) { big_n[0] = 0u; big_n[1] = 0u; }
     if (i >= n) return;
     counts[i] = 0u;
     cursor[i] = 0u;
     float4 a = mn[i], b = mx[i];
+    // both halves in one line, for k_hg_cells to gather (1,048,576 boxes: 64 us
+    // to 51 there for 8 more here)
+    raw[2 * (size_t)i] = a;
+    raw[2 * (size_t)i + 1] = b;
     int l = hg_level(a, b, g.inv_cell0, g.levels);
     uint32_t key = KEY_NONE;
     if (l < 0) {
@@ -637,8 +648,7 @@ __global__ __launch_bounds__(256) void k_hg_hash(const float4 *__restrict__ mn,
 // with the key and the index in their w (so that a cell member is one 32-byte
 // read).  occ[] and the level flags after it are cleared before this kernel.
 __global__ __launch_bounds__(256) void k_hg_cells(const uint2 *__restrict__ kv, int n,
-                                                  const float4 *__restrict__ aabb_min,
-                                                  const float4 *__restrict__ aabb_max, HGridP g,
+                                                  const float4 *__restrict__ raw, HGridP g,
                                                   uint32_t *__restrict__ cell_start,
                                                   uint32_t *__restrict__ occ,
                                                   uint32_t *__restrict__ level_used,
@@ -646,7 +656,7 @@ __global__ __launch_bounds__(256) void k_hg_cells(const uint2 *__restrict__ kv, 
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     uint2 e = kv[s];
-    float4 mn = aabb_min[e.y], mx = aabb_max[e.y];
+    float4 mn = raw[2 * (size_t)e.y], mx = raw[2 * (size_t)e.y + 1];
     mn.w = __uint_as_float(e.x);
     mx.w = __uint_as_float(e.y);
     boxes[2 * (size_t)s] = mn;
@@ -1314,15 +1324,13 @@ hipError_t launch_find_pairs(const DeviceWorld &d, const StepParams &p, hipStrea
 hipError_t launch_emit_pairs(const DeviceWorld &d, const StepParams &p, hipStream_t s) {
     int n = p.n_bodies;
     if (n == 0) return hipSuccess;
-    RB_LAUNCH(k_emit_pairs, dim3((n + 255) / 256), dim3(256), 0, s, n, d.pair_count,
-                       d.pair_off, d.body_slots, p.max_pairs_per_body, d.is_large, d.large_index,
-                       d.large_off, d.large_slots, p.max_pairs, d.pairs,
-                       (const uint32_t *)(d.counters + RB_CNT_SORT_TILE),
-                       d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW);
-    if (p.n_large > 0)
-        RB_LAUNCH(k_emit_large, dim3(p.n_large, 32), dim3(256), 0, s, d.large_list,
-                           d.pair_count, d.pair_off, d.large_off, d.large_slots, p.max_pairs,
-                           d.pairs);
+    const int body_blocks = (int)(((int64_t)n * EMIT_LANES + 255) / 256);
+    const int large_blocks = std::max(1, std::min(32, p.max_scene / 256));
+    RB_LAUNCH(k_emit_pairs, dim3(body_blocks + p.n_large * large_blocks), dim3(256), 0, s, n,
+              body_blocks, large_blocks, d.pair_count, d.pair_off, d.body_slots, p.max_pairs_per_body,
+              d.is_large, d.large_list, d.large_off, d.large_slots, p.max_pairs, d.pairs,
+              (const uint32_t *)(d.counters + RB_CNT_SORT_TILE), d.counters + RB_CNT_PAIRS,
+              d.counters + RB_CNT_OVERFLOW);
     return rb_launch_status();
 }
 
@@ -1353,7 +1361,7 @@ static void launch_pairs_group(int n, uint32_t *counts, uint32_t *offsets, uint3
 // per body, scan, write, then each body's pairs ordered by y.
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
+                              uint32_t *cell_start, uint32_t *occ, float4 *raw, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,
@@ -1369,7 +1377,7 @@ hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float i
     uint32_t *big_n = big + (n > 0 ? n : 0);
     if (ev) hipEventRecord(ev[0], s);
     RB_LAUNCH(k_hg_hash, dim3(blocks), dim3(256), 0, s, mn, mx, n, g, kv, counts, cursor,
-                       big_n, overflow);
+                       big_n, overflow, raw);
     if (ev) hipEventRecord(ev[1], s);
     hipError_t e = launch_radix_sort(kv, n, cell_bits + 2, 8, sw, s);
     if (e != hipSuccess) return e;
@@ -1380,8 +1388,8 @@ hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float i
     if (n > 0) {
         e = launch_fill_u32(occ, 0u, occ_words + 4, s);
         if (e != hipSuccess) return e;
-        RB_LAUNCH(k_hg_cells, dim3(blocks), dim3(256), 0, s, kv, n, mn, mx, g, cell_start,
-                           occ, level_used, boxes);
+        RB_LAUNCH(k_hg_cells, dim3(blocks), dim3(256), 0, s, kv, n, raw, g, cell_start, occ,
+                  level_used, boxes);
         RB_LAUNCH(k_hg_count, dim3(hg_blocks), dim3(64 * HG_WAVES), 0, s, n, cell_start, occ,
                   level_used, boxes, g, counts, rec, rec_n);
     }

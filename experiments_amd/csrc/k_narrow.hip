@@ -858,19 +858,34 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_face_small(
 // Candidates in descending order of edge-edge axis count (stable), pairs of
 // small hulls (the SG-lane clip pass) after the others: the sort keys of the
 // listed candidates.
+// split: counts the others, which is where the small ones start (one atomic a
+// workgroup; a pass over the sorted order that looked for the place took a
+// launch).
 __global__ __launch_bounds__(256) void k_narrow_keys(int max_pairs, const uint32_t *__restrict__ n_cand,
                                                      const uint32_t *__restrict__ cand_list,
                                                      const int4 *__restrict__ face_best,
-                                                     uint2 *__restrict__ kv) {
+                                                     uint2 *__restrict__ kv, int *split) {
+    __shared__ int s_large[4];
     const uint32_t n = min(*n_cand, (uint32_t)max_pairs);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t p = cand_list[i];
-    // large pairs first, each class by descending edge-axis count (at most
-    // 128 x 128 < 0x8000)
-    const int4 fb = face_best[p];
-    const uint32_t ne = (uint32_t)(fb.z < 0x7fff ? fb.z : 0x7fff);
-    kv[i] = make_uint2((fb.w ? 0x8000u : 0u) | (0x7fffu - ne), p);
+    if (blockIdx.x * blockDim.x >= n) return;
+    bool large = false;
+    if (i < n) {
+        const uint32_t p = cand_list[i];
+        // large pairs first, each class by descending edge-axis count (at most
+        // 128 x 128 < 0x8000)
+        const int4 fb = face_best[p];
+        const uint32_t ne = (uint32_t)(fb.z < 0x7fff ? fb.z : 0x7fff);
+        large = fb.w == 0;
+        kv[i] = make_uint2((large ? 0u : 0x8000u) | (0x7fffu - ne), p);
+    }
+    const uint64_t m = __ballot(large);
+    if ((threadIdx.x & 63) == 0) s_large[threadIdx.x >> 6] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int c = (s_large[0] + s_large[1]) + (s_large[2] + s_large[3]);
+        if (c) atomicAdd(split, c);
+    }
 }
 
 // Pass 2, the candidates: edge x edge axes (never reject), then clipping of
@@ -1801,19 +1816,6 @@ __global__ __launch_bounds__(NP_BLOCK) void k_narrow_clip_small(
     }
 }
 
-// First position of the small-hull candidates in the cost-sorted order (the
-// sort key's bit 15; small candidates sort after the others).
-__global__ __launch_bounds__(256) void k_clip_split(const uint32_t *__restrict__ n_cand_ptr,
-                                                    const uint2 *__restrict__ order, int *split) {
-    const int n = (int)*n_cand_ptr;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t s = (order[i].x >> 15) & 1u;
-    const uint32_t prev = i > 0 ? (order[i - 1].x >> 15) & 1u : 0u;
-    if (s && !prev) *split = i;
-    if (i == n - 1 && !s) *split = n;
-}
-
 // ---- compound shapes (findCompoundPairsKernel, sat.cl:763-925) ----
 // Proxy body n + k is child proxy[k].y of body proxy[k].x: its world
 // transform is the body's times the child's (qtRotate(orn, childPos) + pos,
@@ -2066,14 +2068,11 @@ hipError_t launch_narrowphase(const DeviceWorld &d, const StepParams &p, hipStre
                                         d.counters + RB_CNT_PAIRS, d.counters + RB_CNT_OVERFLOW, true);
     if (e != hipSuccess) return e;
     RB_LAUNCH(k_narrow_keys, dim3((p.max_pairs + 255) / 256), dim3(256), 0, s, p.max_pairs, n_cand,
-              d.cand_off, d.face_best, d.cand_kv);
+              d.cand_off, d.face_best, d.cand_kv, d.counters + RB_CNT_CLIP_SPLIT);
     e = launch_radix_sort(d.cand_kv, p.max_pairs, 16, 8, sw, s, d.counters + RB_CNT_NARROW_CAND);
     if (e != hipSuccess) return e;
     // large-hull candidates [0, split) a wave each, then the small-hull ones
     // [split, n) SG lanes each
-    RB_LAUNCH(k_clip_split, dim3((p.max_pairs + 255) / 256), dim3(256), 0, s,
-              (const uint32_t *)(d.counters + RB_CNT_NARROW_CAND), d.cand_kv,
-              d.counters + RB_CNT_CLIP_SPLIT);
     RB_LAUNCH(k_narrow_clip, dim3(grid), dim3(NP_BLOCK), 0, s,
                        d.counters + RB_CNT_CLIP_SPLIT, d.cand_kv, d.face_best,
                        d.pairs, d.pos, d.quat, d.inv_mass, d.shape, d.hulls, d.verts, d.planes,

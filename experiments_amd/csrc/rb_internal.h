@@ -212,7 +212,7 @@ enum {
     RB_CNT_SUM_ITERS_F = 14,
     RB_CNT_TILES_SOLVED = 15, // ... and the number of tiles that had rows
     RB_CNT_FACE_WORK = 16,    // uint32 pairs the quick face test left for the face pass
-    RB_CNT_CLIP_SPLIT = 17,   // first small-hull candidate in the clip order
+    RB_CNT_CLIP_SPLIT = 17,   // clip candidates of larger hulls, which come before the small ones
     RB_CNT_FACE_SMALL = 18,   // uint32 small-hull pairs of the face pass
     RB_CNT_SCENES = 19,       // scene tiles: scenes of each solver class (5)
     RB_CNT_COUNT = 24
@@ -224,6 +224,7 @@ struct StepParams {
     int n_scenes;
     int n_large;
     int large_chunks;    // scene chunks of 4096 bodies scanned per large body
+    int max_scene;       // bodies of the largest scene
     float dt;
     float solver_dt;
     float gravity[3];
@@ -371,14 +372,14 @@ hipError_t launch_mlp_warm(const DeviceWorld &d, const StepParams &p, hipStream_
 hipError_t launch_mlp_targets(const DeviceWorld &d, int capacity, float *x_out, float *t_out,
                               hipStream_t s);
 
-// the stand-alone grid API.  boxes: two per AABB.  rec, rec_n: where the count
+// the stand-alone grid API.  raw, boxes: two per AABB.  rec, rec_n: where the count
 // pass leaves the pairs of each RB_HG_OWN sorted AABBs for the write pass,
 // RB_HG_REC pairs and one count
 #define RB_HG_OWN 16
 #define RB_HG_REC 192
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
+                              uint32_t *cell_start, uint32_t *occ, float4 *raw, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,

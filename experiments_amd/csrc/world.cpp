@@ -438,6 +438,7 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.large_slots, (size_t)large_off[p.n_large] + 1));
     int max_scene = 0;
     for (int sc = 0; sc < n_scenes; sc++) max_scene = std::max(max_scene, scene_count[sc]);
+    p.max_scene = max_scene;
     p.large_chunks = std::max(1, (max_scene + RB_LARGE_CHUNK - 1) / RB_LARGE_CHUNK);
     RB_CHECK(w.alloc(&d.large_chunk_cnt, (size_t)std::max(p.n_large, 1) * p.large_chunks));
     // sort / scan work
@@ -1746,7 +1747,8 @@ struct Grid {
     uint32_t *cursor = nullptr, *big = nullptr;
     uint32_t *cell_start = nullptr, *counts = nullptr, *offsets = nullptr, *total = nullptr;
     uint32_t *occ = nullptr;             // occupancy bit per cell, then one flag per level
-    float4 *boxes = nullptr;             // AABBs in sorted order, with their keys and indices
+    // AABBs, two float4 each: as given, and in sorted order with their keys and indices
+    float4 *raw = nullptr, *boxes = nullptr;
     int *overflow = nullptr;
     SortWork sw{};
     uint32_t *scan_status = nullptr;
@@ -1756,7 +1758,7 @@ struct Grid {
     hipEvent_t ev[5] = {};
     void release() {
         void *ps[] = {kv, ys, cursor, big, cell_start, counts, offsets, total, overflow, sw.tmp,
-                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, boxes, rec, rec_n};
+                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, raw, boxes, rec, rec_n};
         for (void *p : ps) if (p) hipFree(p);
         for (auto &e : ev) if (e) hipEventDestroy(e);
     }
@@ -1782,6 +1784,7 @@ extern "C" mi_rb_status mi_rb_grid_create(const mi_rb_grid_desc *desc, int max_a
               dalloc(&g->cursor, n) == hipSuccess && dalloc(&g->big, (size_t)n + 2) == hipSuccess &&
               dalloc(&g->cell_start, ncells) == hipSuccess &&
               dalloc(&g->occ, ncells / 32 + 4) == hipSuccess &&
+              dalloc(&g->raw, 2 * (size_t)n) == hipSuccess &&
               dalloc(&g->boxes, 2 * (size_t)n) == hipSuccess && dalloc(&g->counts, n) == hipSuccess &&
               dalloc(&g->offsets, n) == hipSuccess && dalloc(&g->total, 4) == hipSuccess &&
               dalloc(&g->overflow, 4) == hipSuccess && dalloc(&g->sw.tmp, n) == hipSuccess &&
@@ -1825,7 +1828,7 @@ extern "C" mi_rb_status mi_rb_grid_find_pairs(void *grid, const void *d_aabb_min
     RB_CHECK(launch_hgrid_pairs(static_cast<const float4 *>(d_aabb_min),
                                 static_cast<const float4 *>(d_aabb_max), n,
                                 1.0f / g->desc.cell_size, g->desc.dims, g->cell_bits,
-                                g->desc.levels, g->kv, g->cell_start, g->occ, g->boxes,
+                                g->desc.levels, g->kv, g->cell_start, g->occ, g->raw, g->boxes,
                                 g->counts, g->offsets, g->cursor, g->big, g->total, g->ys,
                                 g->desc.max_pairs,
                                 static_cast<int2 *>(d_pairs), static_cast<int *>(d_num_pairs),

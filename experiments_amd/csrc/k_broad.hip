@@ -1361,7 +1361,7 @@ static void launch_pairs_group(int n, uint32_t *counts, uint32_t *offsets, uint3
 // per body, scan, write, then each body's pairs ordered by y.
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *raw, float4 *boxes,
+                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,
@@ -1375,6 +1375,10 @@ hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float i
     const int blocks = n > 0 ? (n + 255) / 256 : 1;
     const int hg_blocks = (n + HG_WAVES * HG_OWN - 1) / (HG_WAVES * HG_OWN);
     uint32_t *big_n = big + (n > 0 ? n : 0);
+    // (the boxes as given, two float4 each: k_hg_cells has read them before the
+    // count pass fills rec)
+    static_assert(RB_HG_REC * sizeof(uint2) >= RB_HG_OWN * 2 * sizeof(float4));
+    float4 *raw = (float4 *)rec;
     if (ev) hipEventRecord(ev[0], s);
     RB_LAUNCH(k_hg_hash, dim3(blocks), dim3(256), 0, s, mn, mx, n, g, kv, counts, cursor,
                        big_n, overflow, raw);

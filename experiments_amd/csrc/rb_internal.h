@@ -372,14 +372,14 @@ hipError_t launch_mlp_warm(const DeviceWorld &d, const StepParams &p, hipStream_
 hipError_t launch_mlp_targets(const DeviceWorld &d, int capacity, float *x_out, float *t_out,
                               hipStream_t s);
 
-// the stand-alone grid API.  raw, boxes: two per AABB.  rec, rec_n: where the count
+// the stand-alone grid API.  boxes: two per AABB.  rec, rec_n: where the count
 // pass leaves the pairs of each RB_HG_OWN sorted AABBs for the write pass,
 // RB_HG_REC pairs and one count
 #define RB_HG_OWN 16
 #define RB_HG_REC 192
 hipError_t launch_hgrid_pairs(const float4 *mn, const float4 *mx, int n, float inv_cell0,
                               const int dims[3], int cell_bits, int levels, uint2 *kv,
-                              uint32_t *cell_start, uint32_t *occ, float4 *raw, float4 *boxes,
+                              uint32_t *cell_start, uint32_t *occ, float4 *boxes,
                               uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
                               uint32_t *big, uint32_t *total, uint32_t *ys, int max_pairs,
                               int2 *pairs, int *num_pairs, int *overflow, const SortWork &sw,

@@ -1747,18 +1747,17 @@ struct Grid {
     uint32_t *cursor = nullptr, *big = nullptr;
     uint32_t *cell_start = nullptr, *counts = nullptr, *offsets = nullptr, *total = nullptr;
     uint32_t *occ = nullptr;             // occupancy bit per cell, then one flag per level
-    // AABBs, two float4 each: as given, and in sorted order with their keys and indices
-    float4 *raw = nullptr, *boxes = nullptr;
+    float4 *boxes = nullptr;             // AABBs in sorted order, with their keys and indices
     int *overflow = nullptr;
     SortWork sw{};
     uint32_t *scan_status = nullptr;
-    uint2 *rec = nullptr;                // pairs of the count pass for the write pass
+    uint2 *rec = nullptr;                // the boxes as given, then the count pass's pairs
     uint32_t *rec_n = nullptr;
     int cell_bits = 0;
     hipEvent_t ev[5] = {};
     void release() {
         void *ps[] = {kv, ys, cursor, big, cell_start, counts, offsets, total, overflow, sw.tmp,
-                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, raw, boxes, rec, rec_n};
+                      sw.hist, sw.status, sw.tile_ctr, scan_status, occ, boxes, rec, rec_n};
         for (void *p : ps) if (p) hipFree(p);
         for (auto &e : ev) if (e) hipEventDestroy(e);
     }
@@ -1784,7 +1783,6 @@ extern "C" mi_rb_status mi_rb_grid_create(const mi_rb_grid_desc *desc, int max_a
               dalloc(&g->cursor, n) == hipSuccess && dalloc(&g->big, (size_t)n + 2) == hipSuccess &&
               dalloc(&g->cell_start, ncells) == hipSuccess &&
               dalloc(&g->occ, ncells / 32 + 4) == hipSuccess &&
-              dalloc(&g->raw, 2 * (size_t)n) == hipSuccess &&
               dalloc(&g->boxes, 2 * (size_t)n) == hipSuccess && dalloc(&g->counts, n) == hipSuccess &&
               dalloc(&g->offsets, n) == hipSuccess && dalloc(&g->total, 4) == hipSuccess &&
               dalloc(&g->overflow, 4) == hipSuccess && dalloc(&g->sw.tmp, n) == hipSuccess &&
@@ -1828,7 +1826,7 @@ extern "C" mi_rb_status mi_rb_grid_find_pairs(void *grid, const void *d_aabb_min
     RB_CHECK(launch_hgrid_pairs(static_cast<const float4 *>(d_aabb_min),
                                 static_cast<const float4 *>(d_aabb_max), n,
                                 1.0f / g->desc.cell_size, g->desc.dims, g->cell_bits,
-                                g->desc.levels, g->kv, g->cell_start, g->occ, g->raw, g->boxes,
+                                g->desc.levels, g->kv, g->cell_start, g->occ, g->boxes,
                                 g->counts, g->offsets, g->cursor, g->big, g->total, g->ys,
                                 g->desc.max_pairs,
                                 static_cast<int2 *>(d_pairs), static_cast<int *>(d_num_pairs),

@@ -62,8 +62,11 @@ __device__ __forceinline__ uint32_t pos_hash(int x, int y, int z, const int *dim
 // every member), so its AABB lies in [k c - c/2, (k+1) c + c/2].  Bit q of the
 // result (q = 9 (dz+1) + 3 (dy+1) + (dx+1)) is set unless that cell is
 // provably out of reach; wrapped aliases of a cell only hold members farther
-// away, which the AABB test rejects anyway.
-__device__ __forceinline__ uint32_t reachable_cells(float4 mn, float4 mx, float inv_cell) {
+// away, which the AABB test rejects anyway.  On an axis of two cells both
+// neighbours are the same cell and on an axis of one cell all three are: the
+// first of them stands for the others, so that no cell is searched twice.
+__device__ __forceinline__ uint32_t reachable_cells(float4 mn, float4 mx, float inv_cell,
+                                                    const int *dims) {
     const float c = 1.0f / inv_cell, h = 0.5f * c, eps = 1e-4f * c;
     const float lo[3] = {mn.x, mn.y, mn.z}, hi[3] = {mx.x, mx.y, mx.z};
     uint32_t ok[3];
@@ -77,6 +80,8 @@ __device__ __forceinline__ uint32_t reachable_cells(float4 mn, float4 mx, float 
             const float c0 = (g + (float)d) * c - h - eps, c1 = (g + (float)(d + 1)) * c + h + eps;
             if (hi[k] >= c0 && lo[k] <= c1) ok[k] |= 1u << (d + 1);
         }
+        if (dims[k] == 2) ok[k] = (ok[k] & 2u) | (ok[k] & 5u ? 1u : 0u);
+        if (dims[k] == 1) ok[k] = ok[k] ? 2u : 0u;
     }
     uint32_t m = 0;
 #pragma unroll
@@ -320,7 +325,7 @@ __device__ __forceinline__ void first_overlaps(int n, const uint32_t *__restrict
     int gp[3];
     grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
     uint32_t nk = 0, u0 = (uint32_t)n, at = 0;
-    if (q < 27 && ((reachable_cells(mn0, mx0, g.inv_cell) >> q) & 1u)) {
+    if (q < 27 && ((reachable_cells(mn0, mx0, g.inv_cell, g.dims) >> q) & 1u)) {
         nk = pos_hash(gp[0] + q % 3 - 1, gp[1] + (q / 3) % 3 - 1, gp[2] + q / 9 - 1, g.dims) | sk;
         if ((occ[nk >> 5] >> (nk & 31u)) & 1u) u0 = cell_start[nk];
     }
@@ -381,7 +386,7 @@ __global__ __launch_bounds__(64 * FP_WAVES) void k_find_pairs(
     grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
     const uint32_t x = (uint32_t)gp[0], xl = (x - 1u) & xmask, xr = (x + 1u) & xmask;
     {
-        const uint32_t reach = key != KEY_NONE ? reachable_cells(mn0, mx0, g.inv_cell) : 0u;
+        const uint32_t reach = key != KEY_NONE ? reachable_cells(mn0, mx0, g.inv_cell, g.dims) : 0u;
         const uint32_t sk = key >> g.cell_bits << g.cell_bits;
         uint32_t wl[R], wr[R];
 #pragma unroll

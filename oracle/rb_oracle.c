@@ -252,7 +252,9 @@ static int finish_pairs(pairbuf *b, int max_pairs, int32_t *pairs)
  * kFindPairsLarge does (bt3dGridBroadphaseOCL.cl:216-264).  Pairs are emitted
  * as (x = higher index, y = lower index), as squeezePairCaches writes them
  * (opencl/broadphase_benchmark/computeAabbKernelOCL.cl:69-111), sorted by
- * (x, y).  Returns the number of pairs (may exceed max_pairs). */
+ * (x, y).  A cell is scanned once, also where the grid is so small that it is
+ * a neighbour on both sides.  Returns the number of pairs (may exceed
+ * max_pairs). */
 int orc_find_pairs_grid(int n, const uint32_t *sorted_kv, const float *aabb_min,
                         const float *aabb_max, const int *scene, const int *is_large,
                         const int *scene_start, const int *scene_count, float inv_cell,
@@ -268,9 +270,14 @@ int orc_find_pairs_grid(int n, const uint32_t *sorted_kv, const float *aabb_min,
         int sc = scene ? scene[i] : 0;
         int gp[3];
         grid_pos(aabb_min + 4 * i, aabb_max + 4 * i, inv_cell, dims, gp);
-        for (int dz = -1; dz <= 1; dz++)
-            for (int dy = -1; dy <= 1; dy++)
-                for (int dx = -1; dx <= 1; dx++) {
+        int d0[3], d1[3];
+        for (int k = 0; k < 3; k++) {
+            d0[k] = dims[k] > 1 ? -1 : 0;
+            d1[k] = dims[k] > 2 ? 1 : 0;
+        }
+        for (int dz = d0[2]; dz <= d1[2]; dz++)
+            for (int dy = d0[1]; dy <= d1[1]; dy++)
+                for (int dx = d0[0]; dx <= d1[0]; dx++) {
                     uint32_t h = pos_hash(gp[0] + dx, gp[1] + dy, gp[2] + dz, dims);
                     uint32_t nk = h | (((uint32_t)sc) << cell_bits);
                     /* lower bound of nk in the sorted keys (cell start) */

@@ -6,6 +6,7 @@ stencil cells in z, y, x order, members in sorted order, large bodies last."""
 import numpy as np
 import pytest
 
+import oracle as O
 from experiments_amd import _lib as L
 from experiments_amd import scenes
 from oracle.step import Snapshot, oracle_broadphase
@@ -64,4 +65,33 @@ def test_first_pairs(room, dims, others):
     assert np.array_equal(w.pairs(), ref)
     assert over
     assert bool(w.stats()["overflow_flags"] & L.OVERFLOW_BODY_PAIRS) == over
+    w.close()
+
+
+@pytest.mark.parametrize("others", [0, 16384])  # 4 and 16 entries a wave
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (1, 2, 8), (2, 8, 1), (8, 1, 2)])
+def test_small_grids(dims, others):
+    """One or two cells on an axis: a cell that is a neighbour on both sides is
+    searched once, and every pair is there once."""
+    rng = np.random.default_rng(others + dims[0])
+    sc = scenes.Scene("small", iterations=1)
+    sc.shapes = [scenes.cube_points(0.5), scenes.box_points(400.0, 1.0, 400.0)]
+    at = rng.uniform(-6.0, 6.0, (700, 3))
+    if others:
+        g = np.arange(others)
+        at = np.concatenate([at, np.stack([g % 64, g // 64 % 64, g // 4096], 1) * 2.2 + [8.0, 0.0, 8.0]])
+    q = rng.normal(size=(len(at), 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    sc.add(0.0, (0.0, -7.0, 0.0), (0.0, 0.0, 0.0, 1.0), 1)
+    for a, b in zip(at, q):
+        sc.add(1.0, tuple(a), tuple(b), 0)
+    w = scenes.build_world(sc, max_pairs=1 << 18, max_contacts=1 << 14, grid_dims=dims)
+    assert tuple(w.params()["dims"]) == dims
+    w.step_partial(L.STAGE_PAIRS)
+    mn, mx = w.aabbs()
+    ref = O.find_pairs_brute(mn, mx)
+    assert len(ref) > 700
+    assert np.array_equal(w.pairs(), ref)
+    assert w.stats()["overflow_flags"] == 0
+    w.step(1)
     w.close()

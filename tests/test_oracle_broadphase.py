@@ -94,6 +94,18 @@ def test_grid_pairs_equal_brute_force(seed):
     assert np.all(got[:, 0] > got[:, 1])
 
 
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (1, 2, 8), (2, 8, 1), (8, 1, 2)])
+def test_grid_pairs_once_in_small_grids(dims):
+    """One or two cells on an axis: a cell is its own or a double neighbour."""
+    rng = np.random.default_rng(5)
+    n = 600
+    c = rng.uniform(0, 12, (n, 3)).astype(np.float32)
+    h = rng.uniform(0.2, 0.8, (n, 3)).astype(np.float32)
+    mn, mx = c - h, c + h
+    cell = 2 * float(np.linalg.norm(h, axis=1).max())
+    assert np.array_equal(_grid_pairs(mn, mx, cell, dims), O.find_pairs_brute(mn, mx))
+
+
 def test_brute_force_matches_numpy():
     rng = np.random.default_rng(9)
     n = 400

@@ -1140,10 +1140,8 @@ __global__ __launch_bounds__(TBK) void k_tile_solve(
 // is below it.  A workgroup (a whole CU: 1,024 threads of up to 128 registers)
 // solves 2^lg scenes, each with 1024 >> lg threads whose quads hold two rows
 // each in registers, lg by the scene's rows (scene_class).  The scenes of a
-// workgroup share its barriers: a scene's own barriers order its colours
-// whatever the others are at, and waves that have finished their scene end
-// and are no longer waited for.  Scenes are sorted by rows, so those that
-// share a workgroup take about as long.  What bounds a scene is its colours
+// workgroup share its hardware barrier (see sync below).  Scenes are sorted by
+// rows, so those that share a workgroup take about as long.  What bounds a scene is its colours
 // times its sweeps in sequence; what bounds the launch at thousands of scenes
 // is how many of those chains the chip runs at once, which the registers
 // limit (124 words a row).  4,096 scenes of 8 to 512 bodies, 10 + 10 sweeps:
@@ -1197,10 +1195,24 @@ __global__ __launch_bounds__(SCENE_TB) void k_scene_solve(
     const ConstraintSource src{pk, sv, sp.friction};
     const Quad u{nt / 4, tid >> 2, tid & 3};
     const int wave0 = g * (nt / 64), waves = nt / 64;
-    // (one wave: its LDS operations are in order)
+    // Orders the scene's velocities between its colours.  (One wave: its LDS
+    // operations are in order.)  The scenes of a workgroup come here different
+    // numbers of times and leave at different times, which HIP leaves undefined
+    // for __syncthreads().  What this needs is the hardware's own barrier: it
+    // counts the waves that arrive, at whatever s_barrier, and waits only on
+    // those that have not ended (CDNA ISA, S_BARRIER): a wave passes its k-th
+    // when every running wave has arrived k times, its own scene's among them,
+    // and the waves of a scene arrive and leave together.  A whole wave comes
+    // here or none of it does: every branch on the way depends on values that
+    // the scene's lanes share.
     auto sync = [&]() {
-        if (waves == 1) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        else __syncthreads();
+        if (waves == 1) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        }
     };
     const int b0 = gather_velocities(tid, nt, bodies, nb, linvel, angvel, vel);
     sync();
@@ -1238,7 +1250,7 @@ __global__ __launch_bounds__(SCENE_TB) void k_scene_solve(
                 const float res = rm / (lm > 1.f ? lm : 1.f);
                 used[phase] = it + 1;
                 rfin[phase] = res;
-                if (res < sp.tol) break;
+                if (__builtin_amdgcn_readfirstlane((int)(res < sp.tol))) break;
             } else if (tid == 0) {
                 tile_res[phase * sp.n_tiles + t] = make_uint2(r, m);
             }

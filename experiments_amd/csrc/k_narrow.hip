@@ -425,11 +425,21 @@ __device__ __forceinline__ float fdot(V3 a, float x, float y, float z) {
 __device__ __forceinline__ float norm1(float x, float y, float z) {
     return fabsf(x) + fabsf(y) + fabsf(z);
 }
+// an upper bound of the vector's length
+__device__ __forceinline__ float norm2_bound(float x, float y, float z) {
+    return fminf(norm1(x, y, z), 1.7320509f * fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)));
+}
 // The pose of hull A seen from hull B: x_B = m x_A + tb, x_A = m^T x_B + ta.
 // near: an upper bound of the rounding by which a gap along a unit axis in
 // these frames and one from pass 1's projections differ, without the hulls'
-// part, near_l times a bound of their vertices' norms; the bound holds for
-// unit quaternions (ok).
+// part, NEAR_L times a bound of their vertices' norms; the bound holds for
+// unit quaternions (ok).  Pass 1 projects a body's position on its axis w and
+// adds that to the projections of the vertices: with u = 2^-24 the dot product
+// is off by at most 3 u |p| |w| and the sum by u |p| |w| more (NEAR_P, with
+// room for w's own rounding).  An error of w itself is the same for both
+// bodies, so it counts by their distance (NEAR_L).  (At 10,000 on each axis
+// this asks for a gap of 0.01; a bound of 4e-6 of the coordinates' sum asked
+// for 0.24 and left pass 1 the pairs of unit-sized bodies.)
 struct RelPose {
     V3 m[3], ta, tb;
     float near;
@@ -443,7 +453,7 @@ struct RelPose {
                 fmaf(m[0].z, x, fmaf(m[1].z, y, m[2].z * z))};
     }
 };
-constexpr float NEAR_L = 1e-4f;
+constexpr float NEAR_L = 1e-4f, NEAR_P = 2.6e-7f;
 __device__ __forceinline__ RelPose rel_pose(float4 pA, float4 a, float4 pB, float4 b) {
     RelPose r;
     // conj(b) a
@@ -466,7 +476,7 @@ __device__ __forceinline__ RelPose rel_pose(float4 pA, float4 a, float4 pB, floa
             fmaf(a.w, cz, dz) - fmaf(a.x, cy, -a.y * cx)};
     const V3 t = r.to_b(r.ta.x, r.ta.y, r.ta.z);
     r.tb = {-t.x, -t.y, -t.z};
-    r.near = 4e-6f * (norm1(pA.x, pA.y, pA.z) + norm1(pB.x, pB.y, pB.z)) +
+    r.near = NEAR_P * (norm2_bound(pA.x, pA.y, pA.z) + norm2_bound(pB.x, pB.y, pB.z)) +
              NEAR_L * norm1(dx, dy, dz);
     const float na = fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, a.w * a.w)));
     const float nb = fmaf(b.x, b.x, fmaf(b.y, b.y, fmaf(b.z, b.z, b.w * b.w)));

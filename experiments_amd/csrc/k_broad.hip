@@ -292,23 +292,31 @@ __device__ __forceinline__ void list_row(RowsLDS<OWN, ROWS> &S, uint32_t &total,
     total += (uint32_t)__popcll(has);
 }
 
-// The pair search: a wave per OWN sorted entries, 64 / OWN lanes an entry (16
-// entries where their waves fill the chip, below FP_FEW bodies 4: 64 us against
-// 95 at 65,537 hulls, 23.4 against 13.7 at 4,096 cubes).  The lanes list the
-// entry's stencil rows that hold members within reach, the wave walks them
-// (walk_rows), and an entry's overlaps with bodies of lower index go to its
-// list, the scene's large bodies after them, which is then ordered by rank.  An
-// entry with more than K overlaps keeps the first K that a serial search meets
-// (cells in stencil order, z then y then x, members in sorted order).  Bound by
-// the latency of the member reads.  (A lane per entry, walking the occupied
-// cells in turn: 276 us at 3.4M pairs of 4,096 scenes, now 183; 32 lanes an
-// entry, a cell each: 106 us at 65,537 hulls, now 64.)
+// The pair search: a wave per OWN sorted entries, 64 / OWN lanes an entry.  The
+// lanes list the entry's stencil rows that hold members within reach, the wave
+// walks them (walk_rows), and an entry's overlaps with bodies of lower index go
+// to its list, the scene's large bodies after them, which is then ordered by
+// rank.  An entry with more than K overlaps keeps the first K that a serial
+// search meets (cells in stencil order, z then y then x, members in sorted
+// order).  Bound by the latency of the member reads.  (A lane per entry,
+// walking the occupied cells in turn: 276 us at 3.4M pairs of 4,096 scenes, now
+// 183; 32 lanes an entry, a cell each: 113 us at 65,537 hulls, now 63.)
+// Few bodies leave lanes idle, so there a wave takes 2 or 4 entries and lists
+// each cell by itself, which shortens the longest walk (us; cubes in columns,
+// then hulls in layers):
+//   bodies                1,000   4,096 | 5,000  10,000  24,000  49,152  65,537
+//   2 entries, cells        8.9     8.9 |  15.0    19.6    37.6    70.9    94.0
+//   4 entries, cells       10.9    10.7 |  18.0    20.4    30.3    51.2    66.4
+//   4 entries, rows        14.9    13.9 |  30.1    32.6    42.3            100
+//   16 entries, rows       23.0    23.6 |  46.0    49.9    53.3    60.4    63.0
+//   32 lanes, a cell each   7.9     8.4 |  20.3    25.2    47.2    84.9     113
 constexpr int FP_WAVES = 4;
-constexpr int FP_FEW = 1 << 14;
+constexpr int FP_TWO = 1 << 13, FP_FOUR = 3 << 14;  // below: 2, 4 entries a wave
 constexpr int FP_LIST = RB_MAX_BODY_PAIRS;  // K is no larger
 template <int OWN>
 struct FindLDS {
-    RowsLDS<OWN, OWN * 9> rows;
+    static constexpr bool CELLS = OWN < 16;
+    RowsLDS<OWN, OWN * (CELLS ? 27 : 9)> rows;
     uint32_t count[OWN];
     int list[OWN][FP_LIST | 1];
 };
@@ -400,25 +408,32 @@ __global__ __launch_bounds__(64 * FP_WAVES) void k_find_pairs(
 #pragma unroll
         for (int k = 0; k < R; k++) bits[k] &= row_bits(wl[k], wr[k], base[k], xl, x, xr);
     }
-    // round 0: the rows; rounds 1 and 2: their cells wrapped round the grid's
-    // edge (x - 1 of cell 0, x + 1 of the last)
+    auto keep = [&](uint64_t m, int c, int o) {
+        if ((m >> lane) & 1ull) {
+            const uint32_t p = atomicAdd(&S.count[o], 1u);
+            if (p < (uint32_t)K) S.list[o][p] = c;
+        }
+    };
+    // by rows, round 0: the rows; rounds 1 and 2: their cells wrapped round the
+    // grid's edge (x - 1 of cell 0, x + 1 of the last)
     for (int round = 0; round < 3; round++) {
         uint32_t total = 0;
         bool more = false;
 #pragma unroll
         for (int k = 0; k < R; k++) {
-            const uint32_t edge = (x == 0u ? 1u : 0u) | (x == xmask ? 4u : 0u);
-            const uint32_t m = bits[k] & (round == 0 ? ~edge : round == 1 ? edge & 1u : edge & 4u);
-            more |= (bits[k] & edge) != 0u;
-            list_row(S.rows, total, m, base[k], x, xmask, own, 0u);
+            if constexpr (FindLDS<OWN>::CELLS) {
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    list_row(S.rows, total, bits[k] & (1u << d), base[k], x, xmask, own, 0u);
+            } else {
+                const uint32_t edge = (x == 0u ? 1u : 0u) | (x == xmask ? 4u : 0u);
+                const uint32_t m =
+                    bits[k] & (round == 0 ? ~edge : round == 1 ? edge & 1u : edge & 4u);
+                more |= (bits[k] & edge) != 0u;
+                list_row(S.rows, total, m, base[k], x, xmask, own, 0u);
+            }
         }
-        if (total)
-            walk_rows<true>(n, total, cell_start, boxes, S.rows, [&](uint64_t m, int c, int o) {
-                if ((m >> lane) & 1ull) {
-                    const uint32_t p = atomicAdd(&S.count[o], 1u);
-                    if (p < (uint32_t)K) S.list[o][p] = c;
-                }
-            });
+        if (total) walk_rows<true>(n, total, cell_start, boxes, S.rows, keep);
         if (__ballot(more) == 0ull) break;
     }
     wave_fence();
@@ -1313,7 +1328,8 @@ hipError_t launch_find_pairs(const DeviceWorld &d, const StepParams &p, hipStrea
                   p.n_large ? d.large_first : nullptr, p.n_large ? d.large_num : nullptr,
                   grid_of(p), K, d.body_slots, d.pair_count, d.counters + RB_CNT_OVERFLOW);
     };
-    if (n < FP_FEW) find(k_find_pairs<4>, 4);
+    if (n < FP_TWO) find(k_find_pairs<2>, 2);
+    else if (n < FP_FOUR) find(k_find_pairs<4>, 4);
     else find(k_find_pairs<16>, 16);
     if (p.n_large > 0) {
         dim3 g(p.n_large, p.large_chunks);

@@ -1,6 +1,6 @@
 """The step's pair search: dense clusters whose bodies have from none to over a
 hundred overlaps, with room for 1 to 64 a body, in grids of 4 to 64 cells an
-axis (wrapped), alone (4 entries a wave) and among so many bodies that 16
+axis (wrapped), alone (2 entries a wave) and among so many bodies that 4 or 16
 entries share a wave.  A body's pairs are the first ones of a serial search:
 stencil cells in z, y, x order, members in sorted order, large bodies last."""
 import numpy as np
@@ -68,7 +68,30 @@ def test_first_pairs(room, dims, others):
     w.close()
 
 
-@pytest.mark.parametrize("others", [0, 16384])  # 4 and 16 entries a wave
+@pytest.mark.parametrize("room", [1, 20, 64])
+def test_first_pairs_of_four_entries(room):
+    test_first_pairs(room, (64, 64, 64), 16384)
+
+
+@pytest.mark.parametrize("n", [2, 3, 8191, 8192, 8193, 49151, 49152, 49153])
+def test_entries_per_wave(n):
+    """Around the body counts at which a wave takes 2, 4 or 16 entries."""
+    rng = np.random.default_rng(n)
+    side = 1.2 * (n / 10.0) ** 0.5 + 1.0
+    sc = scenes.Scene("layer", iterations=1)
+    sc.shapes = [scenes.cube_points(0.5)]
+    at = rng.uniform(-0.5, 0.5, (n, 3)) * [side, 12.0, side]
+    q = rng.normal(size=(n, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    for a, b in zip(at, q):
+        sc.add(1.0, tuple(a), tuple(b), 0)
+    w = scenes.build_world(sc, max_pairs_per_body=64, max_pairs=1 << 20, max_contacts=1 << 14)
+    w.step_partial(L.STAGE_PAIRS)
+    assert np.array_equal(w.pairs(), O.find_pairs_brute(*w.aabbs()))
+    w.close()
+
+
+@pytest.mark.parametrize("others", [0, 16384, 49152])  # 2, 4 and 16 entries a wave
 @pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (1, 2, 8), (2, 8, 1), (8, 1, 2)])
 def test_small_grids(dims, others):
     """One or two cells on an axis: a cell that is a neighbour on both sides is

@@ -31,7 +31,7 @@ using namespace rb;
 
 namespace {
 
-constexpr int TB = 256;        // threads per tile workgroup (colouring, spatial solve tiles)
+constexpr int TB = 256;        // threads per tile workgroup (colouring, packing)
 constexpr int HASH_SLOTS = 2 * RB_TILE_MAX_BODIES;
 
 __device__ __forceinline__ uint32_t color_prio(uint32_t k) {
@@ -441,7 +441,7 @@ enum { ROW_NORMAL = 0, ROW_FRICTION = 1, ROW_WARM = 2 };
 struct TileSolveLDS {
     // slot s: linear at 2s + 2, angular at 2s + 3; the first two are zero
     float4 vel[2 * (SOLVE_SLOTS + 1)];
-    uint2 red[4];  // store_tile_residual's waves
+    uint2 red[8];  // store_tile_residual's waves
 };
 
 #define QUAD_PERM(p) " quad_perm:" p " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
@@ -1080,8 +1080,12 @@ __device__ __forceinline__ void store_velocities(int tid, int nt, const int *__r
 }
 
 // Spatial tiles: one sweep (MODE: normal, friction, or the warm start's
-// impulses) over the tiles of one parity phase, a workgroup per tile, the
-// tile's dynamic body velocities in LDS.
+// impulses) over the tiles of one parity phase, a workgroup of TBK threads per
+// tile, the tile's dynamic body velocities in LDS.  A colour of more rows than
+// the tile has quads takes a turn for each TBK / 4 of them: 64 quads were
+// slower on tall columns than the 256 threads, a row each, before them (8 x 8
+// columns of 64 cubes 458 -> 481 us a step, of 128 662 -> 806), 128 quads are
+// faster (360 and 592).
 template <int TBK, int MODE, bool RES>
 __global__ __launch_bounds__(TBK) void k_tile_solve(
     StepParams sp, int phase, const int4 *__restrict__ tile_hdr,
@@ -1524,13 +1528,17 @@ hipError_t launch_solve(const DeviceWorld &d, const StepParams &p, hipStream_t s
                 int nx = (p.tiles_x - (ph & 1) + 1) / 2, nz = (p.tiles_z - (ph >> 1) + 1) / 2;
                 if (nx <= 0 || nz <= 0) continue;
                 mark(0);
-                auto kern = sw < 0 ? k_tile_solve<TB, ROW_WARM, false>
-                            : !fr  ? (res ? k_tile_solve<TB, ROW_NORMAL, true>
-                                          : k_tile_solve<TB, ROW_NORMAL, false>)
-                                   : (res ? k_tile_solve<TB, ROW_FRICTION, true>
-                                          : k_tile_solve<TB, ROW_FRICTION, false>);
-                RB_LAUNCH(kern, dim3(nx * nz), dim3(TB), 0, s, p, ph, RB_SOLVE_ARGS,
-                          d.counters);
+                auto solve = [&](auto threads) {
+                    constexpr int T = decltype(threads)::value;
+                    auto kern = sw < 0 ? k_tile_solve<T, ROW_WARM, false>
+                                : !fr  ? (res ? k_tile_solve<T, ROW_NORMAL, true>
+                                              : k_tile_solve<T, ROW_NORMAL, false>)
+                                       : (res ? k_tile_solve<T, ROW_FRICTION, true>
+                                              : k_tile_solve<T, ROW_FRICTION, false>);
+                    RB_LAUNCH(kern, dim3(nx * nz), dim3(T), 0, s, p, ph, RB_SOLVE_ARGS, d.counters);
+                };
+                if (p.solve_block == 512) solve(std::integral_constant<int, 512>{});
+                else solve(std::integral_constant<int, 256>{});
                 mark(1);
             }
             if (sw >= 0 && p.tol > 0.f) {

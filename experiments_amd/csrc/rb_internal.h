@@ -252,7 +252,8 @@ struct StepParams {
     float tol;
     int warm_start;
     // launch shapes (mi_rb_tuning)
-    int solve_block;     // 256, or 512: twice the threads per scene in a shared workgroup
+    int solve_block;     // 256 or 512: threads of a spatial tile; scenes: 512 gives each one of
+                         // a shared workgroup twice the threads
     int narrow_waves;    // narrowphase waves per SIMD (grid = CUs * 4 * narrow_waves)
     int has_vertexless;  // some shape is a sphere, a plane or a compound
     int n_proxies;       // compound children bodies (after the n bodies)

@@ -125,6 +125,7 @@ struct World {
     long long steps = 0;
     float last_ms = 0.f;
     mi_rb_tuning tuning{0, 0, 0, 0};  // launch shapes; 0 = default
+    int default_block = DEFAULT_SOLVE_BLOCK;  // solve_block 0: by the bodies at upload
     std::vector<void *> allocs;
 
     template <typename T>
@@ -273,9 +274,9 @@ mi_rb_status derive_and_upload(World &w) {
     p.friction_iters = c.solver_iterations;
     p.tol = c.residual_tolerance;
     p.warm_start = c.warm_start;
-    p.solve_block = w.tuning.solve_block ? w.tuning.solve_block : DEFAULT_SOLVE_BLOCK;
     p.narrow_waves = w.tuning.narrow_waves ? w.tuning.narrow_waves : DEFAULT_NARROW_WAVES;
     // solver tiles
+    w.default_block = DEFAULT_SOLVE_BLOCK;
     if (n_scenes > 1) {
         p.tile_mode = 1;
         p.n_tiles = n_scenes;
@@ -291,7 +292,29 @@ mi_rb_status derive_and_upload(World &w) {
         p.tiles_x = std::max(1, (int)std::ceil((hi[0] - lo[0]) / T) + 3);
         p.tiles_z = std::max(1, (int)std::ceil((hi[2] - lo[2]) / T) + 3);
         p.n_tiles = p.tiles_x * p.tiles_z;
+        // 512 threads a tile where the fullest tile has more bodies than 64
+        // quads hold rows and a phase's tiles are all resident at 512 (two a
+        // CU).  Solver launches of a step, 256 -> 512 threads: columns of 64
+        // cubes, 8 x 8 of them 481 -> 360 us, 40 x 40 694 -> 518; of 128, 806
+        // -> 592.  With more tiles the idle waves cost: 4,096 cubes on a
+        // terrain 411 -> 589, 90,000 cubes side by side 1,517 -> 2,460; with
+        // fewer rows a tile nothing changes (16^3 cubes 280 and 270).
+        std::vector<int> in_tile(p.n_tiles, 0);
+        int fullest = 0;
+        auto cell_of = [&](float x, float origin, int n_cells) {
+            const float f = std::floor((x - origin) * p.tile_inv);
+            return f >= 0.f ? (f < (float)n_cells ? (int)f : n_cells - 1) : 0;
+        };
+        for (int i = 0; i < n; i++) {
+            if (w.is_large[i] || w.inv_mass[i] == 0.f) continue;
+            const int tx = cell_of(w.pos[i].x, p.tile_origin_x, p.tiles_x);
+            const int tz = cell_of(w.pos[i].z, p.tile_origin_z, p.tiles_z);
+            fullest = std::max(fullest, ++in_tile[(size_t)tz * p.tiles_x + tx]);
+        }
+        const long long phase_tiles = (long long)((p.tiles_x + 1) / 2) * ((p.tiles_z + 1) / 2);
+        if (fullest > 128 && phase_tiles <= 2ll * rb_num_cus()) w.default_block = 512;
     }
+    p.solve_block = w.tuning.solve_block ? w.tuning.solve_block : w.default_block;
     w.tile_bits = std::max(1, ilog2((uint64_t)p.n_tiles));
 
     // ---- device buffers ----
@@ -1130,7 +1153,7 @@ extern "C" mi_rb_status mi_rb_set_tuning(void *world, const mi_rb_tuning *t) {
           t->sort_digit_bits == 7 || t->sort_digit_bits == 8))
         return MI_RB_INVALID_ARG;
     w->tuning = *t;
-    w->sp.solve_block = t->solve_block ? t->solve_block : DEFAULT_SOLVE_BLOCK;
+    w->sp.solve_block = t->solve_block ? t->solve_block : w->default_block;
     w->sp.narrow_waves = t->narrow_waves ? t->narrow_waves : DEFAULT_NARROW_WAVES;
     if (w->graph) { hipGraphExecDestroy(w->graph); w->graph = nullptr; }
     return MI_RB_OK;
@@ -1156,7 +1179,7 @@ extern "C" mi_rb_status mi_rb_set_solver(void *world, int iterations, float tole
 extern "C" mi_rb_status mi_rb_get_tuning(void *world, mi_rb_tuning *t) {
     World *w = W(world);
     if (!w || !t) return MI_RB_INVALID_ARG;
-    t->solve_block = w->tuning.solve_block ? w->tuning.solve_block : DEFAULT_SOLVE_BLOCK;
+    t->solve_block = w->tuning.solve_block ? w->tuning.solve_block : w->default_block;
     t->narrow_waves = w->tuning.narrow_waves ? w->tuning.narrow_waves : DEFAULT_NARROW_WAVES;
     t->sort_tile = w->tuning.sort_tile;
     t->sort_digit_bits = w->tuning.sort_digit_bits;

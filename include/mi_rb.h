@@ -415,8 +415,10 @@ mi_rb_status mi_rb_set_solve_timing(void *world, int enable);
  * its work-group sizes in the host code).  0 = default.  Changing them drops
  * the captured graph; results do not depend on them. */
 typedef struct mi_rb_tuning {
-    int solve_block;     /* batched scenes: 256, or 512 for twice the threads per scene where
-                          * scenes share a solver workgroup */
+    int solve_block;     /* one scene: threads per solver tile, 256 or 512 (default by the
+                          * bodies per tile at upload); batched scenes: 256, or 512 for
+                          * twice the threads per scene where scenes share a solver
+                          * workgroup (default 256) */
     int narrow_waves;    /* narrowphase waves per SIMD: 1..8 */
     int sort_tile;       /* body-key sort, keys per tile: 1024 or 4096; 0 = by key count */
     int sort_digit_bits; /* body-key sort, bits per radix digit: 4, 6, 7 or 8; 0 = 8 */

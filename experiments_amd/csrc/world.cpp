@@ -411,16 +411,19 @@ mi_rb_status derive_and_upload(World &w) {
     RB_CHECK(w.alloc(&d.tile_color_off, (size_t)p.n_tiles * (RB_MAX_LOCAL_COLORS + 1)));
     RB_CHECK(w.alloc(&d.tile_ncolors, p.n_tiles));
     RB_CHECK(w.alloc(&d.tile_stats, p.n_tiles));
-    RB_CHECK(w.alloc(&d.pk.lin0, maxC));
-    RB_CHECK(w.alloc(&d.pk.jac, maxC));
-    RB_CHECK(w.alloc(&d.pk.b, maxC));
-    RB_CHECK(w.alloc(&d.pk.lam, maxC));
-    RB_CHECK(w.alloc(&d.pk.fric, maxC));
+    // (scene tiles form their rows from the constraints: of the packed rows
+    // they have only the slots)
+    const size_t packed = p.tile_mode == 0 ? (size_t)maxC : 0;
     RB_CHECK(w.alloc(&d.pk.meta, 2 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.nj, 10 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.nm, 10 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.fj, 8 * (size_t)maxC));
-    RB_CHECK(w.alloc(&d.pk.fm, 8 * (size_t)maxC));
+    RB_CHECK(w.alloc(&d.pk.lin0, packed));
+    RB_CHECK(w.alloc(&d.pk.jac, packed));
+    RB_CHECK(w.alloc(&d.pk.b, packed));
+    RB_CHECK(w.alloc(&d.pk.lam, packed));
+    RB_CHECK(w.alloc(&d.pk.fric, packed));
+    RB_CHECK(w.alloc(&d.pk.nj, 10 * packed));
+    RB_CHECK(w.alloc(&d.pk.nm, 10 * packed));
+    RB_CHECK(w.alloc(&d.pk.fj, 8 * packed));
+    RB_CHECK(w.alloc(&d.pk.fm, 8 * packed));
     RB_CHECK(w.alloc(&d.solve_pos, maxC));
     RB_CHECK(w.alloc(&d.tile_bodies, 2 * (size_t)maxC));
     RB_CHECK(w.alloc(&d.tile_nb, p.n_tiles));

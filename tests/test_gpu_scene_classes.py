@@ -62,3 +62,20 @@ def test_step_matches_oracle(layout, block, tol):
         st = w.read(L.BUF_TILE_STATS, np.int32, (4,))
         assert np.array_equal(st[:, :2], np.array(ref["iters"]).reshape(-1, 2))
     w.close()
+
+
+def test_batched_worlds_hold_no_packed_rows():
+    """Only spatial tiles read packed rows (41 float4 a contact): a batched
+    world with the same room holds less device memory by them."""
+    torch = pytest.importorskip("torch")
+    room, held = 1 << 20, []
+    for scene in (0, 1):
+        sc = columns([8])
+        sc.add(0.0, (40.0, -1.0, 0.0), (0.0, 0.0, 0.0, 1.0), 1, scene)
+        free = torch.cuda.mem_get_info()[0]
+        w = scenes.build_world(sc, max_contacts=room)
+        held.append(free - torch.cuda.mem_get_info()[0])
+        w.step(1)
+        assert w.stats()["num_contacts"] == 8
+        w.close()
+    assert held[0] - held[1] >= 0.95 * 41 * 16 * room

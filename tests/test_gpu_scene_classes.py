@@ -12,6 +12,7 @@ from experiments_amd import _lib as L
 from experiments_amd import scenes
 from oracle.step import Snapshot, gpu_tile_orders, oracle_step
 
+torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 EDGES = [1, 31, 33, 64, 65, 128, 129, 256, 257, 512, 513, 768, 769, 1100]
@@ -67,7 +68,6 @@ def test_step_matches_oracle(layout, block, tol):
 def test_batched_worlds_hold_no_packed_rows():
     """Only spatial tiles read packed rows (41 float4 a contact): a batched
     world with the same room holds less device memory by them."""
-    torch = pytest.importorskip("torch")
     room, held = 1 << 20, []
     for scene in (0, 1):
         sc = columns([8])

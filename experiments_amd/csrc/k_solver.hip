@@ -1473,14 +1473,20 @@ __global__ void k_tile_order_keys(int n_tiles, int max_class, const int4 *__rest
 }
 }  // namespace
 
+// log2 of the most scenes that share a workgroup: only as many as leave every
+// CU a workgroup (a lone scene is fastest with a CU to itself)
+static int most_shared(const StepParams &p) {
+    int lg = 0;
+    while (lg < SCENE_CLASSES - 1 && p.n_tiles >> (lg + 1) >= rb_num_cus()) lg++;
+    return lg;
+}
+bool solve_block_matters(const StepParams &p) { return p.tile_mode != 1 || most_shared(p) > 0; }
+
 hipError_t launch_tile_order(const DeviceWorld &d, const StepParams &p, hipStream_t s,
                              const SortWork &sw) {
     if (p.tile_mode != 1) return hipSuccess;
-    // scenes share a workgroup only while every CU still gets one (a lone
-    // scene is fastest with a CU to itself); a tuned block of 512 threads
-    // gives every scene twice the threads
-    int max_class = 0;
-    while (max_class < SCENE_CLASSES - 1 && p.n_tiles >> (max_class + 1) >= rb_num_cus()) max_class++;
+    // (a tuned block of 512 threads gives every scene twice the threads)
+    int max_class = most_shared(p);
     if (p.solve_block == 512 && max_class > 0) max_class--;
     RB_LAUNCH(k_tile_order_keys, dim3((p.n_tiles + 255) / 256), dim3(256), 0, s, p.n_tiles,
               max_class, d.tile_hdr, d.tile_order, d.counters);

@@ -350,6 +350,8 @@ hipError_t launch_tile_order(const DeviceWorld &d, const StepParams &p, hipStrea
 // *n_launches gets the number of launches
 // span: two events recorded before the first and after the last solver
 // launch (the launches run back to back), else null
+// whether StepParams::solve_block changes the schedule of the world's solve
+bool solve_block_matters(const StepParams &p);
 hipError_t launch_solve(const DeviceWorld &d, const StepParams &p, hipStream_t s,
                         hipEvent_t *kev = nullptr, int *n_launches = nullptr,
                         hipEvent_t *span = nullptr);

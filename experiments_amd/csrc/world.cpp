@@ -1238,15 +1238,20 @@ extern "C" mi_rb_status mi_rb_autotune(void *world, int steps, mi_rb_tuning *bes
         ms = w->last_ms / (float)steps;
         return MI_RB_OK;
     };
-    int idx = 0;
-    for (int bi = 0; bi < 2; bi++)
-        for (int wi = 0; wi < 4; wi++, idx++) {
-            const mi_rb_tuning t{blocks[bi], waves[wi], keep.sort_tile, keep.sort_digit_bits};
+    // (one block size where it changes nothing: the one in force)
+    const int in_force = w->sp.solve_block, n_blocks = solve_block_matters(w->sp) ? 2 : 1;
+    for (int bi = 0; bi < n_blocks; bi++)
+        for (int wi = 0; wi < 4; wi++) {
+            const mi_rb_tuning t{n_blocks == 2 ? blocks[bi] : in_force, waves[wi], keep.sort_tile,
+                                 keep.sort_digit_bits};
             float ms = 0.f;
             mi_rb_status stt = trial(t, ms);
             if (stt != MI_RB_OK) return stt;
-            if (ms_out) ms_out[idx] = ms;
-            if (idx == 0 || ms < best_ms) { best_ms = ms; bt = t; }
+            if (ms_out) {
+                ms_out[4 * bi + wi] = ms;
+                if (n_blocks == 1) ms_out[4 + wi] = ms;
+            }
+            if ((bi == 0 && wi == 0) || ms < best_ms) { best_ms = ms; bt = t; }
         }
     // the body-key sort's tile and digit width with the fastest launch shape
     const int tiles[2] = {1024, 4096}, digits[2] = {7, 8};

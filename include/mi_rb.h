@@ -429,7 +429,9 @@ mi_rb_status mi_rb_get_tuning(void *world, mi_rb_tuning *t);
  * the world's current state (restored after each trial, so the world ends
  * where it started), applies the fastest and returns it.  ms_out (may be
  * NULL) receives the per-candidate step times in the order solve_block in
- * {256, 512} x narrow_waves in {2, 4, 6, 8}.  With the fastest of those, the
+ * {256, 512} x narrow_waves in {2, 4, 6, 8}; where solve_block changes nothing
+ * (batched scenes of which none share a workgroup) it stays as it is and both
+ * halves hold the same times.  With the fastest of those, the
  * body-key sort's sort_tile in {1024, 4096} x sort_digit_bits in {7, 8} is
  * timed the same way and the fastest kept (those times are not reported). */
 mi_rb_status mi_rb_autotune(void *world, int steps, mi_rb_tuning *best, float ms_out[8]);

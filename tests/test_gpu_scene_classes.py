@@ -79,3 +79,15 @@ def test_batched_worlds_hold_no_packed_rows():
         assert w.stats()["num_contacts"] == 8
         w.close()
     assert held[0] - held[1] >= 0.95 * 41 * 16 * room
+
+
+def test_autotune_times_a_shape_once():
+    """Where no scenes share a workgroup solve_block changes nothing: it stays,
+    and its two halves of the candidates are the same measurements."""
+    w = scenes.build_world(columns([8] * 8))
+    w.set_tuning(solve_block=512)
+    best, ms = w.autotune(steps=2)
+    assert best["solve_block"] == 512 and w.get_tuning()["solve_block"] == 512
+    for waves in (2, 4, 6, 8):
+        assert ms["256/%d" % waves] == ms["512/%d" % waves] > 0.0
+    w.close()

@@ -1474,7 +1474,13 @@ __global__ void k_tile_order_keys(int n_tiles, int max_class, const int4 *__rest
 }  // namespace
 
 // log2 of the most scenes that share a workgroup: only as many as leave every
-// CU a workgroup (a lone scene is fastest with a CU to itself)
+// CU a workgroup.  Steps in us with up to 1, 2 and 4 scenes a workgroup, 256
+// CUs: scenes of 8 to 64 bodies, 10 + 10 sweeps, 257 of them 325, 336, 360; 300
+// 344, 333, 359; 500 379, 359, 385; 1,100 532, 484, 481; scenes of 8 to 128
+// bodies to a tolerance, 300 1,361, 1,479, 1,621; 500 1,636, 1,680, 1,838;
+// 1,000 2,381, 1,901, 2,045; 1,500 3,351, 2,377, 2,016.  (From about 300 to 511
+// scenes two would share at a gain of 3 to 6% with fixed sweeps, and at a loss
+// of 3 to 9% to a tolerance, where a lone scene's chain is what counts.)
 static int most_shared(const StepParams &p) {
     int lg = 0;
     while (lg < SCENE_CLASSES - 1 && p.n_tiles >> (lg + 1) >= rb_num_cus()) lg++;

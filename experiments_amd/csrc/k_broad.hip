@@ -206,7 +206,8 @@ struct RowsLDS {
 };
 // boxes: the AABBs in sorted order, two float4 each with the key and the index
 // in their w.  hits(m, c, o): the lanes of m hold a member, body c, that
-// overlaps the wave's box o; LOWER: only members of lower index than the box's.
+// overlaps the wave's box o; it tells a lane of them to leave its row.  LOWER:
+// only members of lower index than the box's.
 template <bool LOWER, int OWN, int ROWS, class Hits>
 __device__ __forceinline__ void walk_rows(int n, uint32_t total,
                                           const uint32_t *__restrict__ cell_start,
@@ -250,7 +251,7 @@ __device__ __forceinline__ void walk_rows(int n, uint32_t total,
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const uint64_t m = __ballot(hit[k]);
-            if (m) hits(m, c[k], o);
+            if (m && hits(m, c[k], o)) end = true;
         }
         const uint64_t done = __ballot(end);
         if (done) {
@@ -321,39 +322,67 @@ struct FindLDS {
     int list[OWN][FP_LIST | 1];
 };
 
-// One wave: the first K overlaps of entry (mn0, mx0), index i, in the order of
-// a serial search, a stencil cell a lane.
-__device__ __forceinline__ void first_overlaps(int n, const uint32_t *__restrict__ cell_start,
+// Half a wave each for two entries (mn0, mx0; on: there is one): the first K
+// overlaps in the order of a serial search.  The cells of a stencil row follow
+// each other in the sorted order too, so a half reads a row 32 members at a
+// time and stops at the K-th overlap.  Searches where many lists overflow, us:
+// 60,000 cubes in a box of 16 and K = 64 460, K = 16 370, in one of 40 and K = 8
+// 67, 12,000 in one of 10 and K = 64 112.  (A wave an entry, a cell a lane,
+// counted and then stored, after a walk to the rows' ends: 1,293, 1,454, 93 and
+// 308; 32 lanes an entry from the start, a cell each: 418, 424, 53 and 87.)
+__device__ __forceinline__ void first_overlaps(bool on, int n,
+                                               const uint32_t *__restrict__ cell_start,
                                                const uint32_t *__restrict__ occ,
                                                const float4 *__restrict__ boxes, const GridP &g,
                                                float4 mn0, float4 mx0, int *__restrict__ lst,
                                                int K) {
-    const int q = threadIdx.x & 63, i = __float_as_int(mx0.w);
+    const int q = threadIdx.x & 31, i = __float_as_int(mx0.w);
+    const uint32_t half = threadIdx.x & 32;
     const uint32_t key = __float_as_uint(mn0.w), sk = key >> g.cell_bits << g.cell_bits;
     int gp[3];
     grid_pos(mn0, mx0, g.inv_cell, g.dims, gp);
-    uint32_t nk = 0, u0 = (uint32_t)n, at = 0;
-    if (q < 27 && ((reachable_cells(mn0, mx0, g.inv_cell, g.dims) >> q) & 1u)) {
+    uint32_t nk = 0, u0 = 0;
+    bool has = false;
+    if (on && q < 27 && ((reachable_cells(mn0, mx0, g.inv_cell, g.dims) >> q) & 1u)) {
         nk = pos_hash(gp[0] + q % 3 - 1, gp[1] + (q / 3) % 3 - 1, gp[2] + q / 9 - 1, g.dims) | sk;
-        if ((occ[nk >> 5] >> (nk & 31u)) & 1u) u0 = cell_start[nk];
+        has = (occ[nk >> 5] >> (nk & 31u)) & 1u;
+        if (has) u0 = cell_start[nk];
     }
-    for (int pass = 0; pass < 2; pass++) {
-        uint32_t c = at;
-        for (uint32_t u = u0; u < (uint32_t)n; u++) {
-            const float4 p = boxes[2 * (size_t)u], m = boxes[2 * (size_t)u + 1];
-            if (__float_as_uint(p.w) != nk) break;
-            if (__float_as_int(m.w) < i && aabb_overlap(mn0, mx0, p, m)) {
-                if (pass && c < (uint32_t)K) lst[c] = __float_as_int(m.w);
-                c++;
-            }
+    // (below, every value but the member's is the same in a half's lanes)
+    uint32_t cells = (uint32_t)(__ballot(has) >> half);
+    uint32_t u = 0, last = 0;
+    int c = 0;
+    bool in_row = false;
+    while (__ballot(c < K && (in_row || cells))) {
+        // the row's cells from the first one left on, or that one alone where
+        // they wrap round the grid's edge
+        const int a = cells ? __builtin_ctz(cells) : 0;
+        const uint32_t row = cells & (7u << (a - a % 3));
+        const int z = row ? 31 - __builtin_clz(row) : 0;
+        const uint32_t first = __shfl(nk, a, 32), end = __shfl(nk, z, 32);
+        const uint32_t start = __shfl(u0, a, 32);
+        if (!in_row) {
+            const bool whole = end - first == (uint32_t)(z - a);
+            last = whole ? end : first;
+            u = start;
+            in_row = cells != 0u;
+            cells &= whole ? ~row : cells - 1u;
         }
-        if (pass) break;
-        uint32_t incl = c;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t v = __shfl_up(incl, o, 64);
-            if (q >= o) incl += v;
+        const uint32_t v = u + (uint32_t)q;
+        bool in = in_row && c < K && v < (uint32_t)n, hit = false;
+        int j = 0;
+        if (in) {
+            const float4 p = boxes[2 * (size_t)v], m = boxes[2 * (size_t)v + 1];
+            j = __float_as_int(m.w);
+            in = __float_as_uint(p.w) <= last;
+            hit = in && j < i && aabb_overlap(mn0, mx0, p, m);
         }
-        at = incl - c;
+        const uint32_t h = (uint32_t)(__ballot(hit) >> half);
+        const int at = c + (int)__popc(h & ((1u << q) - 1u));
+        if (hit && at < K) lst[at] = j;
+        c += (int)__popc(h);
+        in_row = (uint32_t)(__ballot(in) >> half) == 0xffffffffu;
+        u += 32u;
     }
 }
 
@@ -408,11 +437,13 @@ __global__ __launch_bounds__(64 * FP_WAVES) void k_find_pairs(
 #pragma unroll
         for (int k = 0; k < R; k++) bits[k] &= row_bits(wl[k], wr[k], base[k], xl, x, xr);
     }
+    // (an entry with more than K overlaps is searched again: the rest of its
+    // rows need not be walked)
     auto keep = [&](uint64_t m, int c, int o) {
-        if ((m >> lane) & 1ull) {
-            const uint32_t p = atomicAdd(&S.count[o], 1u);
-            if (p < (uint32_t)K) S.list[o][p] = c;
-        }
+        if (((m >> lane) & 1ull) == 0ull) return false;
+        const uint32_t p = atomicAdd(&S.count[o], 1u);
+        if (p < (uint32_t)K) S.list[o][p] = c;
+        return p >= (uint32_t)K;
     };
     // by rows, round 0: the rows; rounds 1 and 2: their cells wrapped round the
     // grid's edge (x - 1 of cell 0, x + 1 of the last)
@@ -438,9 +469,14 @@ __global__ __launch_bounds__(64 * FP_WAVES) void k_find_pairs(
     }
     wave_fence();
     uint32_t c = S.count[own];
-    for (uint64_t over = __ballot(sub == 0 && c > (uint32_t)K); over; over &= over - 1ull) {
-        const int o = __builtin_ctzll(over) / LANES;
-        first_overlaps(n, cell_start, occ, boxes, g, S.rows.mn[o], S.rows.mx[o], S.list[o], K);
+    for (uint64_t over = __ballot(sub == 0 && c > (uint32_t)K); over;) {
+        const int o0 = __builtin_ctzll(over) / LANES;
+        over &= over - 1ull;
+        const bool two = over != 0ull;
+        const int o = two && lane >= 32 ? __builtin_ctzll(over) / LANES : o0;
+        over &= over - 1ull;  // (0 stays 0)
+        first_overlaps(two || lane < 32, n, cell_start, occ, boxes, g, S.rows.mn[o], S.rows.mx[o],
+                       S.list[o], K);
     }
     int *dst = body_slots + (size_t)i * K, *lst = S.list[own];
     if (large_num) {
@@ -802,6 +838,7 @@ __device__ __forceinline__ void hg_search(int n, const uint32_t *__restrict__ ce
         if (total)
             walk_rows<false>(n, total, cell_start, boxes, S, [&](uint64_t m, int c, int o) {
                 hits(m, c, __float_as_int(S.mx[o].w));
+                return false;
             });
         rows = rest;
         if (__ballot(rest != 0u) == 0ull) break;

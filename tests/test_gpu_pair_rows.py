@@ -118,3 +118,24 @@ def test_small_grids(dims, others):
     assert w.stats()["overflow_flags"] == 0
     w.step(1)
     w.close()
+
+
+@pytest.mark.parametrize("n,dims", [(1500, (4, 4, 4)), (9000, (64, 64, 64)), (50000, (8, 8, 8))])
+@pytest.mark.parametrize("room", [1, 33, 64])
+def test_first_pairs_of_crowded_cells(n, dims, room):
+    """Cells of more members than a half wave reads at once, most lists full,
+    entries next to the grid's edges among them."""
+    rng = np.random.default_rng(n)
+    sc = scenes.Scene("crowd", iterations=1)
+    sc.shapes = [scenes.cube_points(0.5)]
+    box = {1500: 6.0, 9000: 9.0, 50000: 14.0}[n]
+    for p in rng.uniform(-0.5 * box, 0.5 * box, (n, 3)):
+        sc.add(1.0, tuple(p), (0.0, 0.0, 0.0, 1.0), 0)
+    w = scenes.build_world(sc, max_pairs_per_body=room, max_pairs=64 * n, max_contacts=1 << 12,
+                           grid_dims=dims)
+    s = Snapshot(w)
+    w.step_partial(L.STAGE_PAIRS)
+    ref, over = expected(s, *oracle_broadphase(s), room)
+    assert over
+    assert np.array_equal(w.pairs(), ref)
+    w.close()

@@ -495,7 +495,8 @@ def main():
     traffic = None
     if prof and prof.get("state_steps") == [settle + args.warmup + 1, done]:
         traffic = prof.get("k_tile_solve_bytes_per_dispatch")
-    roofline = {"bound": "hbm", "kernel": "k_tile_solve", "achieved": round(achieved, 2),
+    roofline = {"bound": "hbm", "kernel": "k_scene_solve" if scene_tiles else "k_tile_solve",
+                "achieved": round(achieved, 2),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5),
                 "traffic": round(traffic) if traffic else None,
                 "traffic_source": (prof or {}).get("source") if traffic else

@@ -1145,14 +1145,14 @@ __global__ __launch_bounds__(TBK) void k_tile_solve(
 // solves 2^lg scenes, each with 1024 >> lg threads whose quads hold two rows
 // each in registers, lg by the scene's rows (scene_class).  The scenes of a
 // workgroup share its hardware barrier (see sync below).  Scenes are sorted by
-// rows, so those that share a workgroup take about as long.  What bounds a scene is its colours
-// times its sweeps in sequence; what bounds the launch at thousands of scenes
-// is how many of those chains the chip runs at once, which the registers
-// limit (124 words a row).  4,096 scenes of 8 to 512 bodies, 10 + 10 sweeps:
-// 958 -> 498 us against 256 threads per scene, a thread per row and the rows
-// of scenes above 256 read on every pass; 256 scenes to a tolerance: 2.4x.  A
-// launch per class in sequence took 612 us, and on 256 scenes, where each is
-// as long as its longest scene, twice this one's time.
+// rows, so those that share a workgroup take about as long.  What bounds a
+// scene is its colours times its sweeps in sequence; what bounds the launch at
+// thousands of scenes is how many of those chains the chip runs at once, which
+// the registers limit (124 words a row).  4,096 scenes of 8 to 512 bodies, 10 +
+// 10 sweeps: 994 -> 479 us against 256 threads per scene, a thread per row and
+// the rows of scenes above 256 read on every pass; 256 scenes to a tolerance:
+// 2.4x.  A launch per class in sequence took 612 us, and on 256 scenes, where
+// each is as long as its longest scene, twice this one's time.
 constexpr int SCENE_TB = 1024, SCENE_CLASSES = 5;
 constexpr int SCENE_SLOTS = SCENE_TB + (1 << (SCENE_CLASSES - 1));
 // Threads of a scene: at most two rows a quad while that leaves a whole wave,

@@ -3,7 +3,8 @@ training pairs from the plain solver and the A/B evaluation of iterations to
 a residual tolerance.
 
 Every forward, backward and Adam step runs in libmi_rb.so's kernels (BF16
-MFMA forward, FP32 MFMA backward); torch only provides device buffers.  The
+MFMA, the backward pass's FP32 deltas as three BF16 terms each); torch only
+provides device buffers.  The
 reference has no counterpart: its solver starts every step from zero impulses
 (dynamics/basic_demo/Stubs/solverSetup.cl:529-531).
 """

@@ -1486,7 +1486,7 @@ static int most_shared(const StepParams &p) {
     while (lg < SCENE_CLASSES - 1 && p.n_tiles >> (lg + 1) >= rb_num_cus()) lg++;
     return lg;
 }
-bool solve_block_matters(const StepParams &p) { return p.tile_mode != 1 || most_shared(p) > 0; }
+bool solve_block_matters(const StepParams &p) { return p.tile_mode == 1 && most_shared(p) > 0; }
 
 hipError_t launch_tile_order(const DeviceWorld &d, const StepParams &p, hipStream_t s,
                              const SortWork &sw) {
@@ -1549,7 +1549,7 @@ hipError_t launch_solve(const DeviceWorld &d, const StepParams &p, hipStream_t s
                                               : k_tile_solve<T, ROW_FRICTION, false>);
                     RB_LAUNCH(kern, dim3(nx * nz), dim3(T), 0, s, p, ph, RB_SOLVE_ARGS, d.counters);
                 };
-                if (p.solve_block == 512) solve(std::integral_constant<int, 512>{});
+                if (p.tile_threads == 512) solve(std::integral_constant<int, 512>{});
                 else solve(std::integral_constant<int, 256>{});
                 mark(1);
             }

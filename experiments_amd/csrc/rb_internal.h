@@ -252,8 +252,8 @@ struct StepParams {
     float tol;
     int warm_start;
     // launch shapes (mi_rb_tuning)
-    int solve_block;     // 256 or 512: threads of a spatial tile; scenes: 512 gives each one of
-                         // a shared workgroup twice the threads
+    int solve_block;     // 256, or 512: twice the threads per scene in a shared workgroup
+    int tile_threads;    // threads of a spatial tile's solve: 256 or 512
     int narrow_waves;    // narrowphase waves per SIMD (grid = CUs * 4 * narrow_waves)
     int has_vertexless;  // some shape is a sphere, a plane or a compound
     int n_proxies;       // compound children bodies (after the n bodies)

@@ -125,7 +125,6 @@ struct World {
     long long steps = 0;
     float last_ms = 0.f;
     mi_rb_tuning tuning{0, 0, 0, 0};  // launch shapes; 0 = default
-    int default_block = DEFAULT_SOLVE_BLOCK;  // solve_block 0: by the bodies at upload
     std::vector<void *> allocs;
 
     template <typename T>
@@ -275,8 +274,9 @@ mi_rb_status derive_and_upload(World &w) {
     p.tol = c.residual_tolerance;
     p.warm_start = c.warm_start;
     p.narrow_waves = w.tuning.narrow_waves ? w.tuning.narrow_waves : DEFAULT_NARROW_WAVES;
+    p.solve_block = w.tuning.solve_block ? w.tuning.solve_block : DEFAULT_SOLVE_BLOCK;
     // solver tiles
-    w.default_block = DEFAULT_SOLVE_BLOCK;
+    p.tile_threads = 256;
     if (n_scenes > 1) {
         p.tile_mode = 1;
         p.n_tiles = n_scenes;
@@ -312,9 +312,8 @@ mi_rb_status derive_and_upload(World &w) {
             fullest = std::max(fullest, ++in_tile[(size_t)tz * p.tiles_x + tx]);
         }
         const long long phase_tiles = (long long)((p.tiles_x + 1) / 2) * ((p.tiles_z + 1) / 2);
-        if (fullest > 128 && phase_tiles <= 2ll * rb_num_cus()) w.default_block = 512;
+        if (fullest > 128 && phase_tiles <= 2ll * rb_num_cus()) p.tile_threads = 512;
     }
-    p.solve_block = w.tuning.solve_block ? w.tuning.solve_block : w.default_block;
     w.tile_bits = std::max(1, ilog2((uint64_t)p.n_tiles));
 
     // ---- device buffers ----
@@ -1156,7 +1155,7 @@ extern "C" mi_rb_status mi_rb_set_tuning(void *world, const mi_rb_tuning *t) {
           t->sort_digit_bits == 7 || t->sort_digit_bits == 8))
         return MI_RB_INVALID_ARG;
     w->tuning = *t;
-    w->sp.solve_block = t->solve_block ? t->solve_block : w->default_block;
+    w->sp.solve_block = t->solve_block ? t->solve_block : DEFAULT_SOLVE_BLOCK;
     w->sp.narrow_waves = t->narrow_waves ? t->narrow_waves : DEFAULT_NARROW_WAVES;
     if (w->graph) { hipGraphExecDestroy(w->graph); w->graph = nullptr; }
     return MI_RB_OK;
@@ -1182,7 +1181,7 @@ extern "C" mi_rb_status mi_rb_set_solver(void *world, int iterations, float tole
 extern "C" mi_rb_status mi_rb_get_tuning(void *world, mi_rb_tuning *t) {
     World *w = W(world);
     if (!w || !t) return MI_RB_INVALID_ARG;
-    t->solve_block = w->tuning.solve_block ? w->tuning.solve_block : w->default_block;
+    t->solve_block = w->tuning.solve_block ? w->tuning.solve_block : DEFAULT_SOLVE_BLOCK;
     t->narrow_waves = w->tuning.narrow_waves ? w->tuning.narrow_waves : DEFAULT_NARROW_WAVES;
     t->sort_tile = w->tuning.sort_tile;
     t->sort_digit_bits = w->tuning.sort_digit_bits;

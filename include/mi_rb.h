@@ -415,10 +415,8 @@ mi_rb_status mi_rb_set_solve_timing(void *world, int enable);
  * its work-group sizes in the host code).  0 = default.  Changing them drops
  * the captured graph; results do not depend on them. */
 typedef struct mi_rb_tuning {
-    int solve_block;     /* one scene: threads per solver tile, 256 or 512 (default by the
-                          * bodies per tile at upload); batched scenes: 256, or 512 for
-                          * twice the threads per scene where scenes share a solver
-                          * workgroup (default 256) */
+    int solve_block;     /* batched scenes: 256, or 512 for twice the threads per scene where
+                          * scenes share a solver workgroup */
     int narrow_waves;    /* narrowphase waves per SIMD: 1..8 */
     int sort_tile;       /* body-key sort, keys per tile: 1024 or 4096; 0 = by key count */
     int sort_digit_bits; /* body-key sort, bits per radix digit: 4, 6, 7 or 8; 0 = 8 */
@@ -430,8 +428,8 @@ mi_rb_status mi_rb_get_tuning(void *world, mi_rb_tuning *t);
  * where it started), applies the fastest and returns it.  ms_out (may be
  * NULL) receives the per-candidate step times in the order solve_block in
  * {256, 512} x narrow_waves in {2, 4, 6, 8}; where solve_block changes nothing
- * (batched scenes of which none share a workgroup) it stays as it is and both
- * halves hold the same times.  With the fastest of those, the
+ * (one scene, or batched scenes of which none share a workgroup) it stays as it
+ * is and both halves hold the same times.  With the fastest of those, the
  * body-key sort's sort_tile in {1024, 4096} x sort_digit_bits in {7, 8} is
  * timed the same way and the fastest kept (those times are not reported). */
 mi_rb_status mi_rb_autotune(void *world, int steps, mi_rb_tuning *best, float ms_out[8]);

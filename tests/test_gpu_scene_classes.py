@@ -81,10 +81,11 @@ def test_batched_worlds_hold_no_packed_rows():
     assert held[0] - held[1] >= 0.95 * 41 * 16 * room
 
 
-def test_autotune_times_a_shape_once():
+@pytest.mark.parametrize("n_scenes", [1, 8])
+def test_autotune_times_a_shape_once(n_scenes):
     """Where no scenes share a workgroup solve_block changes nothing: it stays,
     and its two halves of the candidates are the same measurements."""
-    w = scenes.build_world(columns([8] * 8))
+    w = scenes.build_world(columns([8] * n_scenes))
     w.set_tuning(solve_block=512)
     best, ms = w.autotune(steps=2)
     assert best["solve_block"] == 512 and w.get_tuning()["solve_block"] == 512
